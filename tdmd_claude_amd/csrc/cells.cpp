@@ -41,7 +41,7 @@ __global__ void assign_cells_kernel(const double* __restrict__ pos, int64_t nato
   iz = iz < 0 ? 0 : iz;
   const int c = iz * ncx * ncy + iy * ncx + ix;
   atom_cells[i] = c;
-  atomicAdd(&counts[c], 1);
+  (void)wave_add_one(counts, c);
 }
 
 __global__ void scatter_cells_kernel(const int32_t* __restrict__ atom_cells, int64_t natoms,
@@ -51,19 +51,20 @@ __global__ void scatter_cells_kernel(const int32_t* __restrict__ atom_cells, int
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= natoms) return;
   const int c = atom_cells[i];
-  const int slot = offsets[c] + atomicAdd(&cursor[c], 1);
-  cell_atoms[slot] = static_cast<int32_t>(i);
+  cell_atoms[offsets[c] + wave_add_one(cursor, c)] = static_cast<int32_t>(i);
 }
 
-// Insertion sort of each cell's segment by atom index. Cells hold tens of
-// atoms in a dense system, so one thread per cell is enough.
-__global__ void order_cells_kernel(const int32_t* __restrict__ offsets,
-                                   const int32_t* __restrict__ counts, int ncells,
-                                   int32_t* __restrict__ cell_atoms) {
+// Both counter arrays of a build, in one launch.
+__global__ void zero_cells_kernel(int32_t* __restrict__ counts, int32_t* __restrict__ cursor,
+                                  int ncells) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= ncells) return;
-  int32_t* seg = cell_atoms + offsets[c];
-  const int n = counts[c];
+  counts[c] = 0;
+  cursor[c] = 0;
+}
+
+// Insertion sort of a cell's segment by atom index, by one lane.
+__device__ __forceinline__ void sort_cell(int32_t* seg, int n) {
   for (int a = 1; a < n; ++a) {
     const int32_t v = seg[a];
     int b = a - 1;
@@ -73,6 +74,34 @@ __global__ void order_cells_kernel(const int32_t* __restrict__ offsets,
     }
     seg[b + 1] = v;
   }
+}
+
+// Each cell's atoms by increasing index. kLanes = 64: one wavefront per cell,
+// lane l takes the cell's l-th atom and counts the atoms with a smaller
+// index, its place (cells of more than 64 atoms: lane 0 sorts). One lane's
+// insertion sort of the 20-40 atoms of a solid's cell is a chain of dependent
+// loads and stores (265,000 atoms: 107 us; 7 us so), but cells of a few atoms
+// are cheaper one to a lane (1M cells of one atom: 116 us by wavefronts,
+// ~15 by lanes), hence kLanes = 1 below 8 atoms per cell in more than 32,768
+// cells (16,384 cells of 4 atoms: build 35 us by lanes, 25 by wavefronts;
+// 64,000 of one: 28 and 31).
+template <int kLanes>
+__global__ void __launch_bounds__(kBlock)
+order_cells_kernel(const int32_t* __restrict__ offsets, const int32_t* __restrict__ counts,
+                   int ncells, int32_t* __restrict__ cell_atoms) {
+  const int64_t c = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kLanes;
+  if (c >= ncells) return;
+  const int lane = threadIdx.x % kLanes;
+  int32_t* seg = cell_atoms + offsets[c];
+  const int n = counts[c];
+  if (kLanes == 1 || n > 64) {
+    if (lane == 0) sort_cell(seg, n);
+    return;
+  }
+  const int32_t v = lane < n ? seg[lane] : 0x7fffffff;
+  int pos = 0;
+  for (int m = 0; m < n; ++m) pos += __shfl(v, m, 64) < v ? 1 : 0;
+  if (lane < n) seg[pos] = v;
 }
 
 }  // namespace
@@ -102,24 +131,26 @@ int cell_build(const double* d_pos, int64_t natoms, const tdmd_box& box, double 
   char* work = static_cast<char*>(d_work);
   int32_t* cursor = reinterpret_cast<int32_t*>(work);
   void* scan_work = work + ((static_cast<size_t>(ncells) * 4 + 255) / 256) * 256;
-  int rc = tdmd_fill_u32(d_counts, 0u, static_cast<size_t>(ncells), stream);
-  if (rc) return rc;
-  rc = tdmd_fill_u32(cursor, 0u, static_cast<size_t>(ncells), stream);
-  if (rc) return rc;
+  zero_cells_kernel<<<grid_for(ncells), kBlock, 0, stream>>>(d_counts, cursor, ncells);
+  TDMD_LAUNCH_CHECK();
   const DevBox db = make_devbox(box);
   if (natoms > 0) {
     assign_cells_kernel<<<grid_for(natoms), kBlock, 0, stream>>>(
         d_pos, natoms, db, cs[0], cs[1], cs[2], n[0], n[1], n[2], d_atom_cells, d_counts);
     TDMD_LAUNCH_CHECK();
   }
-  rc = scan_exclusive_i32(d_counts, d_offsets, ncells, nullptr, scan_work, stream);
+  const int rc = scan_exclusive_i32(d_counts, d_offsets, ncells, nullptr, scan_work, stream);
   if (rc) return rc;
   if (natoms > 0) {
     scatter_cells_kernel<<<grid_for(natoms), kBlock, 0, stream>>>(
         d_atom_cells, natoms, d_offsets, cursor, d_cell_atoms);
     TDMD_LAUNCH_CHECK();
-    order_cells_kernel<<<grid_for(ncells), kBlock, 0, stream>>>(d_offsets, d_counts, ncells,
-                                                                d_cell_atoms);
+    if (ncells <= 32768 || natoms >= 8 * static_cast<int64_t>(ncells))
+      order_cells_kernel<64><<<grid_for(ncells, kBlock / kWave), kBlock, 0, stream>>>(
+          d_offsets, d_counts, ncells, d_cell_atoms);
+    else
+      order_cells_kernel<1><<<grid_for(ncells), kBlock, 0, stream>>>(d_offsets, d_counts, ncells,
+                                                                     d_cell_atoms);
     TDMD_LAUNCH_CHECK();
   }
   return TDMD_OK;

@@ -98,6 +98,35 @@ __device__ __forceinline__ int wave_max_i(int v) {
   return v;
 }
 
+// Adds one to ctr[key] for each active lane of the wavefront with one atomic
+// per distinct key (atoms are in cell order from the previous sort, so a
+// wave's lanes share a few cells and per-lane atomics on one address
+// serialise); returns the counter's value before this lane's increment, in
+// lane order within each key. Every active lane of the wave must call it.
+// The keys are sorted out first and the atomics issued together, so a wave
+// waits for one round trip, not for one per key; lanes whose key has not come
+// up in kWaveKeys turns (atoms in no spatial order) add for themselves.
+constexpr int kWaveKeys = 12;
+__device__ __forceinline__ int wave_add_one(int32_t* ctr, int key) {
+  const int lane = static_cast<int>(threadIdx.x & 63);
+  unsigned long long todo = __ballot(1);
+  int first = lane, before = 0, sum = 1;
+  for (int t = 0; t < kWaveKeys && todo; ++t) {
+    const int leader = __ffsll(todo) - 1;
+    const int k = __shfl(key, leader, 64);
+    const unsigned long long same = __ballot(key == k) & todo;
+    if ((same >> lane) & 1ull) {
+      first = leader;
+      before = __popcll(same & ((1ull << lane) - 1ull));
+      sum = __popcll(same);
+    }
+    todo &= ~same;
+  }
+  int old = 0;
+  if (before == 0) old = atomicAdd(&ctr[key], sum);
+  return __shfl(old, first, 64) + before;
+}
+
 // Block reduction of a double into out[blockIdx.x] (fixed order: wave sums
 // then a serial sum of wave partials by thread 0). blockDim multiple of 64.
 template <int BLOCK>

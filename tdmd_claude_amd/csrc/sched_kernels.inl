@@ -775,28 +775,6 @@ __device__ __forceinline__ void cell_coords(const CellGrid& cg, double x, double
 // ---- per-item bodies, shared by the separate kernels (first build) and
 // the fused rebuild kernel ----
 
-// Adds one to ctr[key] for each active lane of the wavefront with one atomic
-// per distinct key (atoms are in cell order from the previous sort, so a
-// wave's lanes share a few cells and per-lane atomics on one address
-// serialise); returns the counter's value before this lane's increment, in
-// lane order within each key. Every active lane of the wave must call it.
-__device__ __forceinline__ int wave_add_one(int32_t* ctr, int key) {
-  const int lane = static_cast<int>(threadIdx.x & 63);
-  unsigned long long todo = __ballot(1);
-  int old = 0;
-  while (todo) {
-    const int leader = __ffsll(todo) - 1;
-    const int k = __shfl(key, leader, 64);
-    const unsigned long long same = __ballot(key == k) & todo;
-    int base = 0;
-    if (lane == leader) base = atomicAdd(&ctr[k], __popcll(same));
-    base = __shfl(base, leader, 64);
-    if ((same >> lane) & 1ull) old = base + __popcll(same & ((1ull << lane) - 1ull));
-    todo &= ~same;
-  }
-  return old;
-}
-
 template <class Mir>
 __device__ __forceinline__ void bin_atom(const StepArgs& a, const GridArgs& g, int i) {
   int c[3];
