@@ -82,6 +82,98 @@ def test_full_list_bitexact_vs_oracle(case):
         assert np.array_equal(np.sort(nb[off[i]:off[i] + cnt[i]]), rnb[roff[i]:roff[i] + rcnt[i]])
 
 
+def rows_reference(pos, lo, hi, periodic, r_list, nc):
+    """Rows in the order the list promises: the 27 stencil cells z, y, x outer
+    to inner, each cell's atoms by index; d = x_j - x_i in float64, one
+    conditional minimum image, r^2 summed unfused."""
+    L = hi - lo
+    cs = L / np.array(nc)
+    c = np.clip(np.trunc((pos - lo) / cs).astype(int), 0, np.array(nc) - 1)
+    cell = (c[:, 2] * nc[1] + c[:, 1]) * nc[0] + c[:, 0]
+    order = np.argsort(cell, kind="stable")
+    start = np.searchsorted(cell[order], np.arange(nc[0] * nc[1] * nc[2] + 1))
+    rows = []
+    for i in range(len(pos)):
+        cand = []
+        for dz in (-1, 0, 1):
+            for dy in (-1, 0, 1):
+                for dx in (-1, 0, 1):
+                    n = [(c[i, a] + d) % nc[a] for a, d in enumerate((dx, dy, dz))]
+                    k = (n[2] * nc[1] + n[1]) * nc[0] + n[0]
+                    cand.append(order[start[k]:start[k + 1]])
+        cand = np.concatenate(cand)
+        d = pos[cand] - pos[i]
+        for a in range(3):
+            if periodic[a]:
+                x, h = d[:, a].copy(), 0.5 * L[a]
+                d[:, a] = np.where(x > h, x - L[a], np.where(x < -h, x + L[a], x))
+        r2 = d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1] + d[:, 2] * d[:, 2]
+        rows.append(cand[(r2 < r_list * r_list) & (cand != i)])
+    return rows
+
+
+def list_edge_case(name):
+    """pos, lo, hi, periodic, r_list, max_neighbors (None: what the count says)."""
+    rng = np.random.Generator(np.random.PCG64(11))
+    lo = np.array([-3.0, 1.0, 0.5])
+    if name == "one":  # a single atom
+        return lo + [[1.0, 2.0, 3.0]], lo, lo + 30.0, (1, 1, 1), 4.0, None
+    if name == "sparse":  # fewer atoms than cells
+        return lo + rng.uniform(0, 40, (200, 3)), lo, lo + 40.0, (1, 1, 1), 4.0, None
+    if name == "box of 3 cells below r_list":  # the stencil covers the box
+        return lo + rng.uniform(0, 10, (150, 3)), lo, lo + 10.0, (1, 1, 1), 4.9, None
+    if name == "cluster":  # cells of hundreds of atoms, stencils beyond one chunk
+        p = np.concatenate([rng.normal(15.0, 2.0, (1500, 3)), rng.uniform(0, 30, (500, 3))])
+        return lo + np.clip(p, 0, 29.99), lo, lo + 30.0, (1, 1, 1), 4.0, None
+    if name == "cut rows":  # capacity below the longest row
+        return lo + rng.uniform(0, 14, (900, 3)), lo, lo + 14.0, (1, 1, 1), 4.0, 40
+    if name == "outside":  # atoms beyond the faces, some by more than a box
+        p = rng.uniform(-6, 18, (700, 3))
+        p[::40] += 30.0
+        return lo + p, lo, lo + 12.0, (1, 1, 1), 3.9, None
+    # open axes, atoms far outside them
+    p = rng.uniform(-4, 20, (700, 3))
+    p[::50] *= 40.0
+    return lo + p, lo, lo + 16.0, (1, 0, 0), 3.9, None
+
+
+@pytest.mark.parametrize("case", ["one", "sparse", "box of 3 cells below r_list", "cluster",
+                                  "cut rows", "outside", "open"])
+def test_list_rows_in_order_at_the_edges(case):
+    pos, lo, hi, per, r_list, cap = list_edge_case(case)
+    pos, hi, N = np.asarray(pos), np.asarray(hi), len(pos)
+    say("csr rows", case, N)
+    box = capi.Box.make(lo, hi, per)
+    n = (C.c_int32 * 3)()
+    capi.call("tdmd_cell_grid", C.byref(box), r_list, n, (C.c_double * 3)())
+    rows = rows_reference(pos, lo, hi, per, r_list, list(n))
+    ncells = n[0] * n[1] * n[2]
+    d_pos = D.from_host(np.ascontiguousarray(pos, dtype=np.float64))
+    cc, co, ca, ac = D(ncells, np.int32), D(ncells, np.int32), D(N, np.int32), D(N, np.int32)
+    wb = C.c_size_t()
+    capi.call("tdmd_cell_workspace_bytes", N, ncells, C.byref(wb))
+    work = D(wb.value, np.uint8)
+    cells = (cc.ptr, co.ptr, ca.ptr, ac.ptr)
+    capi.call("tdmd_cell_build", d_pos.ptr, N, C.byref(box), r_list, *cells, work.ptr, None)
+    counts, counts2 = D(N, np.int32), D(N, np.int32)
+    capi.call("tdmd_nlist_count", d_pos.ptr, N, C.byref(box), r_list, *cells, n, counts.ptr, None)
+    want = np.array([len(r) for r in rows])
+    assert np.array_equal(counts.download(), want)
+    cap = cap or int(want.max())
+    offs = np.concatenate([[0], np.cumsum(np.minimum(want, max(cap, 1)))[:-1]]).astype(np.int32)
+    d_off, ovf = D.from_host(offs), D(1, np.int32)
+    nb = D.from_host(np.full(int(np.minimum(want, cap).sum()) + 64, -7, dtype=np.int32))
+    ovf.zero()
+    capi.call("tdmd_nlist_fill", d_pos.ptr, N, C.byref(box), r_list, *cells, n, d_off.ptr, nb.ptr,
+              counts2.ptr, cap, ovf.ptr, None)
+    got = nb.download()
+    assert np.array_equal(counts2.download(), want)
+    assert int(ovf.download()[0]) == (int(want.max()) if want.max() > cap else 0)
+    for i, r in enumerate(rows):
+        assert np.array_equal(got[offs[i]:offs[i] + min(len(r), cap)], r[:cap]), i
+    assert np.all(got[-64:] == -7)
+
+
 @pytest.mark.parametrize("n", [1, 255, 4096, 4097, 100000, 1 << 20])
 def test_scan_exact(n):
     say("scan", n)
