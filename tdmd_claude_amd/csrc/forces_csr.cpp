@@ -2,27 +2,60 @@
 // compute_morse_gpu / DeviceEam::compute boundary
 // (src/potentials/device_morse.cu:32-170, src/potentials/device_eam.cu:72-421).
 //
-// One thread per atom. Pair geometry (difference, minimum image, r^2, cutoff,
-// r) in FP64, pair functions in R (pair_math.hpp). Per-atom sums (force,
-// density, energy) are FP64. Forces are stored, not accumulated
-// (device_morse.cu:110-117); energies are added to *d_energy: one FP64
-// atomic per block when no workspace is given, otherwise per-block partials
-// summed in a fixed order.
+// kRowLanes neighbouring lanes per atom: they read a row's consecutive slots
+// side by side and combine their sums by a butterfly, a fixed order. (One lane
+// per atom reads 64 rows ~400 bytes apart, a cache line for every slot, and
+// walks ~100 dependent slots in turn: 16,384 atoms filled 64 of 256 CUs.)
+// The next slot's index is loaded while a slot is evaluated. Pair geometry
+// (difference, minimum image, r^2, cutoff, r) in FP64, pair functions in R
+// (pair_math.hpp). Per-atom sums (force, density, energy) are FP64. Forces
+// are stored, not accumulated (device_morse.cu:110-117); energies are added
+// to *d_energy: one FP64 atomic per 256 atoms when no workspace is given,
+// otherwise partials, one per 256 atoms, summed in a fixed order.
+#include <algorithm>
+
 #include "pair_math.hpp"
 
 namespace tdmd_hip {
 
-constexpr int kMaxSplines = 64;  // 2*ntypes + ntypes(ntypes+1)/2 for ntypes <= 8
-
 namespace {
 
-__device__ __forceinline__ double pair_geom(const double* __restrict__ pos, double xi, double yi,
-                                            double zi, int j, const DevBox& box, double* dx,
-                                            double* dy, double* dz) {
-  *dx = min_image(xi - pos[3 * j], box.size[0], 0.5 * box.size[0], box.periodic[0]);
-  *dy = min_image(yi - pos[3 * j + 1], box.size[1], 0.5 * box.size[1], box.periodic[1]);
-  *dz = min_image(zi - pos[3 * j + 2], box.size[2], 0.5 * box.size[2], box.periodic[2]);
-  return *dx * *dx + *dy * *dy + *dz * *dz;
+// Lanes per row, and slots a lane takes at a time (kSlots of for_row). Rows of
+// a solid have ~90-120 slots. us without / with the energy, by lanes x slots:
+//   atoms                  4x4         8x1         8x2         8x4        16x2
+//   EAM mixed   16,384   22 / 39     17 / 36     17 / 36     18 / 37     17 / 39
+//   EAM mixed  131,072  110 / 112   116 / 117   108 / 110   101 / 105   105 / 110
+//   EAM mixed  1M      1057 / 1037 1201 / 1231 1086 / 1100  961 / 951   996 / 1035
+//   Morse FP64  16,384   14 / 34     12 / 36     12 / 36     12 / 37     12 / 40
+//   Morse FP64 131,072   70 / 79     68 / 83     71 / 82     72 / 85     74 / 89
+//   Morse FP64 1M       480 / 537   550 / 596   491 / 572   504 / 583   535 / 643
+//   Morse, 1M atoms of a gas, rows of ~4 slots:
+//                         38          46          49          66          91
+// (one lane: EAM mixed 167, 368, 5445; Morse FP64 105, 216, 4515; gas 64).
+// The passes are bound by their gathers (three 8-byte words of a position,
+// one or two table quads, F' per slot: ~20 lines of L1 a wave and slot).
+constexpr int kRowLanes = 8;
+constexpr int kMorseSlots = 2;
+constexpr int kEamSlots = 4;
+constexpr int kEnergyBlock = 1024;  // with the energy: 256 atoms a workgroup, in turns
+
+// Box of the pair geometry: half is infinite on an open axis.
+struct PairBox {
+  double size[3], half[3];
+};
+
+PairBox make_pair_box(const DevBox& b) {
+  PairBox p;
+  for (int a = 0; a < 3; ++a) {
+    p.size[a] = b.size[a];
+    p.half[a] = b.periodic[a] ? 0.5 * b.size[a] : __builtin_huge_val();
+  }
+  return p;
+}
+
+// min_image() (common.hpp) by one compare: the same values.
+__device__ __forceinline__ double image(double d, double size, double half) {
+  return d - (fabs(d) > half ? copysign(size, d) : 0.0);
 }
 
 // 0-based table index of a 1-based type. Types outside 1..ntypes (which the
@@ -32,34 +65,138 @@ __device__ __forceinline__ int clamp_type(int t, int ntypes) {
   return t < 0 ? 0 : (t >= ntypes ? ntypes - 1 : t);
 }
 
+// Sum over the kRowLanes lanes of a row, in every lane.
+__device__ __forceinline__ double row_sum(double v) {
+#pragma unroll
+  for (int w = kRowLanes / 2; w > 0; w >>= 1) v += __shfl_xor(v, w, 64);
+  return v;
+}
+
+// pair(j, dx, dy, dz, r2) for this lane's slots of a row, kSlots at a time:
+// the indices of the next turn are loaded before this turn's positions are
+// waited for, without a branch (past the row's end the last slot is read
+// again and not evaluated).
+template <int kSlots, class Pair>
+__device__ __forceinline__ void for_row(const double* __restrict__ pos,
+                                        const int32_t* __restrict__ nbrs, int off, int cnt,
+                                        double xi, double yi, double zi, const PairBox& box,
+                                        Pair&& pair) {
+  if (cnt <= 0) return;
+  const int32_t* row = nbrs + off;
+  const int part = static_cast<int>(threadIdx.x) % kRowLanes;
+  int j[kSlots];
+#pragma unroll
+  for (int u = 0; u < kSlots; ++u) j[u] = row[min(part + u * kRowLanes, cnt - 1)];
+  for (int k = part; k < cnt; k += kSlots * kRowLanes) {
+    double dx[kSlots], dy[kSlots], dz[kSlots], r2[kSlots];
+    double px[kSlots], py[kSlots], pz[kSlots];
+    int jn[kSlots];
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+      const double* p = pos + 3 * static_cast<int64_t>(j[u]);
+      px[u] = p[0];
+      py[u] = p[1];
+      pz[u] = p[2];
+    }
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u)
+      jn[u] = row[min(k + (kSlots + u) * kRowLanes, cnt - 1)];
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+      dx[u] = image(xi - px[u], box.size[0], box.half[0]);
+      dy[u] = image(yi - py[u], box.size[1], box.half[1]);
+      dz[u] = image(zi - pz[u], box.size[2], box.half[2]);
+      r2[u] = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
+    }
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u)
+      if (k + u * kRowLanes < cnt) pair(j[u], dx[u], dy[u], dz[u], r2[u]);
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) j[u] = jn[u];
+  }
+}
+
+// Blocks are dealt round-robin to the 8 XCDs: block b of `n` takes piece
+// piece_of(b, n) of the atoms, so that an XCD's pieces are consecutive and
+// their rows' positions stay in its L2.
+__device__ __forceinline__ int64_t piece_of(int b, int n) {
+  const int per = n >> 3;
+  return b < 8 * per ? static_cast<int64_t>(b & 7) * per + (b >> 3) : b;
+}
+
+// The workgroup's atoms [begin, end): kThreads / kRowLanes at a time. With
+// the energy a workgroup takes 256 atoms, whose sum is partial piece_of(b);
+// without, one turn's atoms (a grid of at most kMaxGrid strides over them).
+constexpr int kMaxGrid = 1 << 22;
+
+template <bool kEnergy, class Atom>
+__device__ __forceinline__ void for_atoms(int count, Atom&& atom) {
+  constexpr int kThreads = kEnergy ? kEnergyBlock : kBlock;
+  constexpr int kTurn = kThreads / kRowLanes;
+  const int64_t piece = piece_of(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  const int sub = static_cast<int>(threadIdx.x) / kRowLanes;
+  if (kEnergy) {
+    for (int t = 0; t < kBlock; t += kTurn) {
+      const int64_t i = piece * kBlock + t + sub;
+      if (i < count) atom(static_cast<int>(i));
+    }
+  } else {
+    for (int64_t i = piece * kTurn + sub; i < count;
+         i += static_cast<int64_t>(gridDim.x) * kTurn)
+      atom(static_cast<int>(i));
+  }
+}
+
 __device__ __forceinline__ void emit_energy(double e, double* __restrict__ partials,
                                             double* __restrict__ d_energy) {
-  const double t = block_sum<kBlock>(e);
+  const double t = block_sum<kEnergyBlock>(e);
   if (threadIdx.x == 0) {
     if (partials)
-      partials[blockIdx.x] = t;
+      partials[piece_of(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))] = t;
     else
       atomicAdd(d_energy, t);
   }
 }
 
-// Atoms [first, first + count); kAccum adds the forces to what `forces`
-// holds (the zone pass, device_morse_zone.cu:29-117) instead of storing them.
+int row_grid(int count, bool energy) {
+  if (energy) return grid_for(count);
+  return static_cast<int>(std::min<int64_t>(
+      (static_cast<int64_t>(count) * kRowLanes + kBlock - 1) / kBlock, kMaxGrid));
+}
+
+// Forces of one atom, by the first of its lanes; kAccum adds to what
+// `forces` holds (the zone pass, device_morse_zone.cu:29-117).
+template <class R, bool kAccum>
+__device__ __forceinline__ void put_force(R* __restrict__ forces, int i, double fx, double fy,
+                                          double fz) {
+  if (threadIdx.x % kRowLanes != 0) return;
+  R* f = forces + 3 * static_cast<int64_t>(i);
+  if (kAccum) {
+    f[0] += static_cast<R>(fx);
+    f[1] += static_cast<R>(fy);
+    f[2] += static_cast<R>(fz);
+  } else {
+    f[0] = static_cast<R>(fx);
+    f[1] = static_cast<R>(fy);
+    f[2] = static_cast<R>(fz);
+  }
+}
+
+// Atoms [first, first + count).
 template <class R, bool kEnergy, bool kAccum>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kEnergy ? kEnergyBlock : kBlock)
 morse_csr_kernel(const double* __restrict__ pos, R* __restrict__ forces,
                  const int32_t* __restrict__ nbrs, const int32_t* __restrict__ offsets,
-                 const int32_t* __restrict__ counts, int first, int count, DevBox box,
+                 const int32_t* __restrict__ counts, int first, int count, PairBox box,
                  MorseCoef p, double* __restrict__ partials, double* __restrict__ d_energy) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = first + t;
-  double fx = 0.0, fy = 0.0, fz = 0.0, pe = 0.0;
-  if (t < count) {
-    const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-    const int off = offsets[i], cnt = counts[i];
-    for (int k = 0; k < cnt; ++k) {
-      double dx, dy, dz;
-      const double r2 = pair_geom(pos, xi, yi, zi, nbrs[off + k], box, &dx, &dy, &dz);
+  double pe = 0.0;
+  for_atoms<kEnergy>(count, [&](int t) {
+    const int i = first + t;
+    const double* pi = pos + 3 * static_cast<int64_t>(i);
+    const double xi = pi[0], yi = pi[1], zi = pi[2];
+    double fx = 0.0, fy = 0.0, fz = 0.0;
+    for_row<kMorseSlots>(pos, nbrs, offsets[i], counts[i], xi, yi, zi, box,
+            [&](int j, double dx, double dy, double dz, double r2) {
       if (r2 < p.rc_sq) {
         const PairR<R> pr = pair_r<R>(r2);
         R e;
@@ -69,123 +206,122 @@ morse_csr_kernel(const double* __restrict__ pos, R* __restrict__ forces,
         fy = fma(fpair, dy, fy);
         fz = fma(fpair, dz, fz);
       }
-    }
-    if (kAccum) {
-      forces[3 * i] += static_cast<R>(fx);
-      forces[3 * i + 1] += static_cast<R>(fy);
-      forces[3 * i + 2] += static_cast<R>(fz);
-    } else {
-      forces[3 * i] = static_cast<R>(fx);
-      forces[3 * i + 1] = static_cast<R>(fy);
-      forces[3 * i + 2] = static_cast<R>(fz);
-    }
-  }
+    });
+    put_force<R, kAccum>(forces, i, row_sum(fx), row_sum(fy), row_sum(fz));
+  });
   if (kEnergy) emit_energy(pe, partials, d_energy);
 }
 
-__device__ __forceinline__ void load_meta(SplineMeta* sm, const SplineMeta* meta, int ns) {
-  for (int k = threadIdx.x; k < ns; k += blockDim.x) sm[k] = meta[k];
-  __syncthreads();
+// The tables' layout by value: the F splines share one grid, all r splines
+// another (setfl: one Nrho, drho, Nr, dr), every table starts at 0.
+struct EamLayout {
+  SplineMeta F, r;  // offset of element 0's F and rho
+  int ntypes;
+  double rc_sq;
+  __device__ __forceinline__ int f_at(int t) const { return t * (F.n - 1); }
+  __device__ __forceinline__ int rho_at(int t) const { return r.offset + t * (r.n - 1); }
+  __device__ __forceinline__ int phi_at(int p) const {
+    return r.offset + (ntypes + p) * (r.n - 1);
+  }
+};
+
+EamLayout eam_layout(const tdmd_eam_tables* t) {
+  EamLayout e;
+  e.F = SplineMeta{t->drho, 1.0 / t->drho, 0.0, t->nrho, 0};
+  e.r = SplineMeta{t->dr, 1.0 / t->dr, 0.0, t->nr, t->ntypes * (t->nrho - 1)};
+  e.ntypes = t->ntypes;
+  e.rc_sq = t->cutoff * t->cutoff;
+  return e;
 }
 
-// Pass 1: rho_i = sum_j rho_{t_j}(r_ij), FP64 sum (device_eam.cu:72-133).
-template <class R>
+// Derivative and value of one interval's cubic, spline_deriv's and
+// spline_value's expressions.
+template <class R, class Q>
+__device__ __forceinline__ R quad_deriv(const Q& c, R dx) {
+  return c.y + dx * (static_cast<R>(2) * c.z + dx * static_cast<R>(3) * c.w);
+}
+template <class R, class Q>
+__device__ __forceinline__ R quad_value(const Q& c, R dx) {
+  return c.x + dx * (c.y + dx * (c.z + dx * c.w));
+}
+
+// Passes 1 and 2: rho_i = sum_j rho_{t_j}(r_ij), FP64 sum
+// (device_eam.cu:72-133), and fp_i = F'_{t_i}(rho_i) (:137-162).
+template <class R, bool kOne>
 __global__ void __launch_bounds__(kBlock)
 eam_density_csr_kernel(const double* __restrict__ pos, const int32_t* __restrict__ types,
                        const int32_t* __restrict__ nbrs, const int32_t* __restrict__ offsets,
-                       const int32_t* __restrict__ counts, int natoms, int ntypes, DevBox box,
-                       double rc_sq, const SplineMeta* __restrict__ meta,
+                       const int32_t* __restrict__ counts, int natoms, EamLayout t, PairBox box,
                        const typename Quad<R>::type* __restrict__ coeff,
-                       double* __restrict__ rho) {
-  __shared__ SplineMeta smeta[kMaxSplines];
-  load_meta(smeta, meta, 2 * ntypes);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= natoms) return;
-  const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-  const int off = offsets[i], cnt = counts[i];
-  double rho_i = 0.0;
-  for (int k = 0; k < cnt; ++k) {
-    const int j = nbrs[off + k];
-    double dx, dy, dz;
-    const double r2 = pair_geom(pos, xi, yi, zi, j, box, &dx, &dy, &dz);
-    if (r2 >= rc_sq) continue;
-    const PairR<R> pr = pair_r<R>(r2);
-    rho_i += static_cast<double>(
-        spline_value<R>(smeta[ntypes + clamp_type(types[j], ntypes)], coeff, pr.r));
-  }
-  rho[i] = rho_i;
-}
-
-// Pass 2: fp_i = F'_{t_i}(rho_i); energy F(rho_i) (device_eam.cu:137-162).
-template <class R, bool kEnergy>
-__global__ void __launch_bounds__(kBlock)
-eam_embed_csr_kernel(const int32_t* __restrict__ types, int natoms, int ntypes,
-                     const SplineMeta* __restrict__ meta,
-                     const typename Quad<R>::type* __restrict__ coeff,
-                     const double* __restrict__ rho, R* __restrict__ fp,
-                     double* __restrict__ partials, double* __restrict__ d_energy) {
-  __shared__ SplineMeta smeta[kMaxSplines];
-  load_meta(smeta, meta, ntypes);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double e = 0.0;
-  if (i < natoms) {
-    const SplineVal<R> F = spline_both<R>(smeta[clamp_type(types[i], ntypes)], coeff, rho[i]);
-    fp[i] = F.df;
-    e = static_cast<double>(F.f);
-  }
-  if (kEnergy) emit_energy(e, partials, d_energy);
+                       double* __restrict__ rho, R* __restrict__ fp) {
+  for_atoms<false>(natoms, [&](int i) {
+    const double* pi = pos + 3 * static_cast<int64_t>(i);
+    const double xi = pi[0], yi = pi[1], zi = pi[2];
+    double rho_i = 0.0;
+    for_row<kEamSlots>(pos, nbrs, offsets[i], counts[i], xi, yi, zi, box,
+            [&](int j, double dx, double dy, double dz, double r2) {
+      if (r2 < t.rc_sq) {
+        R x;
+        const int k = spline_locate<R>(t.r, pair_r<R>(r2).r, &x);
+        const int tj = kOne ? 0 : clamp_type(types[j], t.ntypes);
+        rho_i += static_cast<double>(quad_value<R>(coeff[t.rho_at(tj) + k], x));
+      }
+    });
+    rho_i = row_sum(rho_i);
+    if (threadIdx.x % kRowLanes == 0) {
+      R x;
+      const int k = spline_locate<R>(t.F, rho_i, &x);
+      rho[i] = rho_i;
+      fp[i] = quad_deriv<R>(coeff[t.f_at(kOne ? 0 : clamp_type(types[i], t.ntypes)) + k], x);
+    }
+  });
 }
 
 // Pass 3: F_i = sum_j -(phi' + fp_i rho'_{t_j} + fp_j rho'_{t_i})/r * d
-// (device_eam.cu:176-278), plus 0.5 phi per pair of the full list.
-template <class R, bool kEnergy>
-__global__ void __launch_bounds__(kBlock)
+// (device_eam.cu:176-278); energy 0.5 phi per pair of the full list and
+// F(rho_i). One interval per pair: the three r splines share the grid.
+template <class R, bool kEnergy, bool kOne>
+__global__ void __launch_bounds__(kEnergy ? kEnergyBlock : kBlock)
 eam_force_csr_kernel(const double* __restrict__ pos, R* __restrict__ forces,
                      const int32_t* __restrict__ types, const int32_t* __restrict__ nbrs,
                      const int32_t* __restrict__ offsets, const int32_t* __restrict__ counts,
-                     int natoms, int ntypes, DevBox box, double rc_sq,
-                     const SplineMeta* __restrict__ meta,
+                     int natoms, EamLayout t, PairBox box,
                      const typename Quad<R>::type* __restrict__ coeff,
-                     const R* __restrict__ fp, double* __restrict__ partials,
-                     double* __restrict__ d_energy) {
-  __shared__ SplineMeta smeta[kMaxSplines];
-  const int np = ntypes * (ntypes + 1) / 2;
-  load_meta(smeta, meta, 2 * ntypes + np);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double fx = 0.0, fy = 0.0, fz = 0.0, pe = 0.0;
-  if (i < natoms) {
-    const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-    const int ti = clamp_type(types[i], ntypes);
+                     const double* __restrict__ rho, const R* __restrict__ fp,
+                     double* __restrict__ partials, double* __restrict__ d_energy) {
+  double pe = 0.0;
+  for_atoms<kEnergy>(natoms, [&](int i) {
+    const double* pi = pos + 3 * static_cast<int64_t>(i);
+    const double xi = pi[0], yi = pi[1], zi = pi[2];
+    const int ti = kOne ? 0 : clamp_type(types[i], t.ntypes);
     const R fpi = fp[i];
-    const int off = offsets[i], cnt = counts[i];
-    for (int k = 0; k < cnt; ++k) {
-      const int j = nbrs[off + k];
-      double dx, dy, dz;
-      const double r2 = pair_geom(pos, xi, yi, zi, j, box, &dx, &dy, &dz);
-      if (r2 >= rc_sq) continue;
-      const PairR<R> pr = pair_r<R>(r2);
-      const int tj = clamp_type(types[j], ntypes);
-      const int pidx = phi_index(ti, tj, ntypes);
-      R dphi;
-      if (kEnergy) {
-        const SplineVal<R> ph = spline_both<R>(smeta[2 * ntypes + pidx], coeff, pr.r);
-        pe += 0.5 * static_cast<double>(ph.f);
-        dphi = ph.df;
-      } else {
-        dphi = spline_deriv<R>(smeta[2 * ntypes + pidx], coeff, pr.r);
+    double fx = 0.0, fy = 0.0, fz = 0.0;
+    for_row<kEamSlots>(pos, nbrs, offsets[i], counts[i], xi, yi, zi, box,
+            [&](int j, double dx, double dy, double dz, double r2) {
+      if (r2 < t.rc_sq) {
+        const PairR<R> pr = pair_r<R>(r2);
+        const int tj = kOne ? 0 : clamp_type(types[j], t.ntypes);
+        R x;
+        const int k = spline_locate<R>(t.r, pr.r, &x);
+        const auto cphi = coeff[t.phi_at(kOne ? 0 : phi_index(ti, tj, t.ntypes)) + k];
+        const R dphi = quad_deriv<R>(cphi, x);
+        if (kEnergy) pe += 0.5 * static_cast<double>(quad_value<R>(cphi, x));
+        const R drho_j = quad_deriv<R>(coeff[t.rho_at(tj) + k], x);
+        const R drho_i = kOne ? drho_j : quad_deriv<R>(coeff[t.rho_at(ti) + k], x);
+        const double fpair =
+            static_cast<double>(-(dphi + fpi * drho_j + fp[j] * drho_i) * pr.rinv);
+        fx = fma(fpair, dx, fx);
+        fy = fma(fpair, dy, fy);
+        fz = fma(fpair, dz, fz);
       }
-      const R drho_j = spline_deriv<R>(smeta[ntypes + tj], coeff, pr.r);
-      const R drho_i = spline_deriv<R>(smeta[ntypes + ti], coeff, pr.r);
-      const double fpair =
-          static_cast<double>(-(dphi + fpi * drho_j + fp[j] * drho_i) * pr.rinv);
-      fx = fma(fpair, dx, fx);
-      fy = fma(fpair, dy, fy);
-      fz = fma(fpair, dz, fz);
+    });
+    put_force<R, false>(forces, i, row_sum(fx), row_sum(fy), row_sum(fz));
+    if (kEnergy && threadIdx.x % kRowLanes == 0) {
+      R x;
+      const int k = spline_locate<R>(t.F, rho[i], &x);
+      pe += static_cast<double>(quad_value<R>(coeff[t.f_at(ti) + k], x));
     }
-    forces[3 * i] = static_cast<R>(fx);
-    forces[3 * i + 1] = static_cast<R>(fy);
-    forces[3 * i + 2] = static_cast<R>(fz);
-  }
+  });
   if (kEnergy) emit_energy(pe, partials, d_energy);
 }
 
@@ -193,18 +329,46 @@ template <class R, bool kAccum>
 int morse_launch(const double* pos, void* forces, const int32_t* nbrs, const int32_t* offsets,
                  const int32_t* counts, int first, int count, const DevBox& box,
                  const tdmd_morse_params& p, double* d_energy, void* work, hipStream_t stream) {
-  const int grid = grid_for(count);
   double* partials = static_cast<double*>(work);
   const MorseCoef c{p.d, p.alpha, p.r0, p.rc_sq};
+  const PairBox pb = make_pair_box(box);
+  const int grid = row_grid(count, d_energy != nullptr);
   if (d_energy) {
-    morse_csr_kernel<R, true, kAccum><<<grid, kBlock, 0, stream>>>(
-        pos, static_cast<R*>(forces), nbrs, offsets, counts, first, count, box, c, partials,
+    morse_csr_kernel<R, true, kAccum><<<grid, kEnergyBlock, 0, stream>>>(
+        pos, static_cast<R*>(forces), nbrs, offsets, counts, first, count, pb, c, partials,
         d_energy);
     TDMD_LAUNCH_CHECK();
     if (partials) return launch_sum_partials(partials, grid, d_energy, 1, stream);
   } else {
     morse_csr_kernel<R, false, kAccum><<<grid, kBlock, 0, stream>>>(
-        pos, static_cast<R*>(forces), nbrs, offsets, counts, first, count, box, c, nullptr,
+        pos, static_cast<R*>(forces), nbrs, offsets, counts, first, count, pb, c, nullptr,
+        nullptr);
+    TDMD_LAUNCH_CHECK();
+  }
+  return TDMD_OK;
+}
+
+template <class R, bool kOne>
+int eam_passes(const tdmd_eam_tables* t, const double* pos, R* forces, const int32_t* types,
+               const int32_t* nbrs, const int32_t* offsets, const int32_t* counts, int natoms,
+               const PairBox& box, double* rho, R* fp, double* d_energy, double* partials,
+               hipStream_t stream) {
+  const auto* coeff = static_cast<const typename Quad<R>::type*>(t->d_coeff);
+  const EamLayout e = eam_layout(t);
+  const int grid = row_grid(natoms, false);
+  eam_density_csr_kernel<R, kOne><<<grid, kBlock, 0, stream>>>(
+      pos, types, nbrs, offsets, counts, natoms, e, box, coeff, rho, fp);
+  TDMD_LAUNCH_CHECK();
+  if (d_energy) {
+    const int ge = row_grid(natoms, true);
+    eam_force_csr_kernel<R, true, kOne><<<ge, kEnergyBlock, 0, stream>>>(
+        pos, forces, types, nbrs, offsets, counts, natoms, e, box, coeff, rho, fp, partials,
+        d_energy);
+    TDMD_LAUNCH_CHECK();
+    if (partials) return launch_sum_partials(partials, ge, d_energy, 1, stream);
+  } else {
+    eam_force_csr_kernel<R, false, kOne><<<grid, kBlock, 0, stream>>>(
+        pos, forces, types, nbrs, offsets, counts, natoms, e, box, coeff, rho, fp, nullptr,
         nullptr);
     TDMD_LAUNCH_CHECK();
   }
@@ -214,42 +378,16 @@ int morse_launch(const double* pos, void* forces, const int32_t* nbrs, const int
 template <class R>
 int eam_launch(const tdmd_eam_tables* t, const double* pos, void* forces, const int32_t* types,
                const int32_t* nbrs, const int32_t* offsets, const int32_t* counts, int natoms,
-               const DevBox& box, double* rho, void* fpv, double* d_energy, void* work,
+               const DevBox& box, double* rho, void* fp, double* d_energy, void* work,
                hipStream_t stream) {
-  using Q = typename Quad<R>::type;
-  const int grid = grid_for(natoms);
-  const double rc_sq = t->cutoff * t->cutoff;
-  const auto* meta = static_cast<const SplineMeta*>(t->d_meta);
-  const auto* coeff = static_cast<const Q*>(t->d_coeff);
-  R* fp = static_cast<R*>(fpv);
-  double* partials = static_cast<double*>(work);
-  eam_density_csr_kernel<R><<<grid, kBlock, 0, stream>>>(pos, types, nbrs, offsets, counts,
-                                                         natoms, t->ntypes, box, rc_sq, meta,
-                                                         coeff, rho);
-  TDMD_LAUNCH_CHECK();
-  if (d_energy) {
-    eam_embed_csr_kernel<R, true><<<grid, kBlock, 0, stream>>>(types, natoms, t->ntypes, meta,
-                                                               coeff, rho, fp, partials, d_energy);
-    TDMD_LAUNCH_CHECK();
-    if (partials) {
-      int rc = launch_sum_partials(partials, grid, d_energy, 1, stream);
-      if (rc) return rc;
-    }
-    eam_force_csr_kernel<R, true><<<grid, kBlock, 0, stream>>>(
-        pos, static_cast<R*>(forces), types, nbrs, offsets, counts, natoms, t->ntypes, box,
-        rc_sq, meta, coeff, fp, partials, d_energy);
-    TDMD_LAUNCH_CHECK();
-    if (partials) return launch_sum_partials(partials, grid, d_energy, 1, stream);
-  } else {
-    eam_embed_csr_kernel<R, false><<<grid, kBlock, 0, stream>>>(types, natoms, t->ntypes, meta,
-                                                                coeff, rho, fp, nullptr, nullptr);
-    TDMD_LAUNCH_CHECK();
-    eam_force_csr_kernel<R, false><<<grid, kBlock, 0, stream>>>(
-        pos, static_cast<R*>(forces), types, nbrs, offsets, counts, natoms, t->ntypes, box,
-        rc_sq, meta, coeff, fp, nullptr, nullptr);
-    TDMD_LAUNCH_CHECK();
-  }
-  return TDMD_OK;
+  const PairBox pb = make_pair_box(box);
+  auto* f = static_cast<R*>(forces);
+  auto* d = static_cast<R*>(fp);
+  auto* w = static_cast<double*>(work);
+  return t->ntypes == 1 ? eam_passes<R, true>(t, pos, f, types, nbrs, offsets, counts, natoms, pb,
+                                              rho, d, d_energy, w, stream)
+                        : eam_passes<R, false>(t, pos, f, types, nbrs, offsets, counts, natoms,
+                                               pb, rho, d, d_energy, w, stream);
 }
 
 // ---------------------------------------------------------------------------

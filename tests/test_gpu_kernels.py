@@ -285,6 +285,124 @@ def test_eam_multitype_vs_oracle():
         assert err < (1e-12 if prec == FP64 else MIXED_TOL)
 
 
+def cut_rows(natoms, periodic=(1, 1, 1)):
+    """The first `natoms` atoms of a jittered crystal with their rows cut to
+    lengths around the lane and turn sizes of the row passes (0 slots to all)."""
+    s = I.fcc_lattice(8, 8, 8, 3.615)
+    I.displace_gaussian(s, 0.05, 77)
+    i, j = [], []
+    L = s.hi - s.lo
+    lengths = [0, 1, 2, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 10 ** 6]
+    cnt = np.zeros(natoms, dtype=np.int32)
+    for a in range(natoms):
+        d = s.pos[a] - s.pos
+        d -= np.where(periodic, L, 0.0) * np.round(d / L)
+        nb = np.nonzero(((d * d).sum(1) < 6.5 ** 2) & (np.arange(s.natoms) != a))[0]
+        nb = nb[:lengths[a % len(lengths)]]
+        cnt[a] = len(nb)
+        i += [a] * len(nb)
+        j += list(nb)
+    off = np.concatenate([[0], np.cumsum(cnt)[:-1]]).astype(np.int32)
+    return s, cnt, off, np.array(i, dtype=np.int64), np.array(j, dtype=np.int32)
+
+
+@pytest.mark.parametrize("prec", [FP64, MIXED])
+@pytest.mark.parametrize("natoms,ntypes,work,per", [(1, 1, True, (1, 1, 1)),
+                                                    (129, 1, True, (1, 1, 1)),
+                                                    (256, 3, False, (1, 1, 1)),
+                                                    (257, 3, True, (1, 0, 1)),
+                                                    (1000, 1, None, (1, 1, 1))])
+def test_row_passes_at_the_edges(natoms, ntypes, work, per, prec):
+    """Morse and EAM over rows of every length class, partial workgroups, one
+    and several elements, an open axis; energy by workspace, by atomics and
+    absent, against the same sums in numpy float64 (the bounds of the other
+    force tests: 1e-12 / 1e-5 of the RMS force)."""
+    say("row passes", natoms, ntypes, work, per, prec)
+    s, cnt, off, i, j = cut_rows(natoms, per)
+    t = I.johnson_setfl(nr=500, nrho=500) if ntypes == 1 else I.johnson_alloy_setfl(nr=500,
+                                                                                   nrho=500)
+    types = np.random.Generator(np.random.PCG64(5)).integers(1, ntypes + 1, s.natoms)
+    L = s.hi - s.lo
+    d = s.pos[i] - s.pos[j]
+    d -= np.where(per, L, 0.0) * np.round(d / L)
+    r = np.sqrt((d * d).sum(1))
+
+    def cubic(v, h, x, deriv):
+        a, b, c, dd = O.spline_coeffs(v, h)
+        k = np.clip((x / h).astype(int), 0, len(a) - 1)
+        y = x - k * h
+        return (b[k] + y * (2 * c[k] + 3 * y * dd[k]) if deriv
+                else a[k] + y * (b[k] + y * (c[k] + y * dd[k])))
+
+    def pick(tables, which, h, x, deriv=False):  # table which[n] at x[n]
+        out = np.zeros(len(x))
+        for k in range(len(tables)):
+            out[which == k] = cubic(tables[k], h, x[which == k], deriv)
+        return out
+
+    rr = np.arange(t.nr) * t.dr
+    phi = np.zeros_like(t.rphi)
+    phi[:, 1:] = t.rphi[:, 1:] / rr[1:]
+    inside = r < t.cutoff
+    I_, J_, D_, R_ = i[inside], j[inside], d[inside], r[inside]
+    ti, tj = types[I_] - 1, types[J_] - 1
+    lo_, hi_ = np.minimum(ti, tj), np.maximum(ti, tj)
+    pair = lo_ * ntypes - lo_ * (lo_ + 1) // 2 + hi_
+    rho = np.bincount(I_, pick(t.rho, tj, t.dr, R_), natoms)
+    fp = np.zeros(s.natoms)  # rows of atoms beyond natoms are empty: rho = 0
+    allr = np.concatenate([rho, np.zeros(s.natoms - natoms)])
+    fp = pick(t.F, types - 1, t.drho, allr, True)
+    f = -(pick(phi, pair, t.dr, R_, True) + fp[I_] * pick(t.rho, tj, t.dr, R_, True)
+          + fp[J_] * pick(t.rho, ti, t.dr, R_, True)) / R_
+    eam_f = np.stack([np.bincount(I_, f * D_[:, k], natoms) for k in range(3)], 1)
+    eam_e = pick(t.F, types[:natoms] - 1, t.drho, rho).sum() + 0.5 * pick(phi, pair, t.dr, R_).sum()
+    De, al, r0, rc = MORSE_CU
+    inside = r < rc
+    e = np.exp(-al * (r - r0))
+    w = np.where(inside, -2 * De * al * (1 - e) * e / r, 0.0)
+    morse_f = np.stack([np.bincount(i, w * d[:, k], natoms) for k in range(3)], 1)
+    morse_e = 0.5 * np.where(inside, De * ((1 - e) ** 2 - 1), 0.0).sum()
+
+    rdt = np.float32 if prec == MIXED else np.float64
+    box = capi.Box.make(s.lo, s.hi, per)
+    # every atom of the crystal has a row in the arrays (empty beyond natoms),
+    # so F'(rho) exists for every neighbour
+    M = s.natoms
+    cnt_all = np.concatenate([cnt, np.zeros(M - natoms, np.int32)])
+    off_all = np.concatenate([off, np.full(M - natoms, len(j), np.int32)])
+    d_pos, d_t = D.from_host(s.pos), D.from_host(types.astype(np.int32))
+    d_cnt, d_off, d_nb = D.from_host(cnt_all), D.from_host(off_all), D.from_host(np.append(j, np.int32(0)).astype(np.int32))
+    tabs = EamTables(prec, t)
+    d_rho, d_fp, d_f = D(M, np.float64), D(M, rdt), D((M, 3), rdt)
+    d_w = D(M // 256 + 2, np.float64)
+    d_e = D.from_host(np.array([2.5]))
+    args = (None, None) if work is None else (d_e.ptr, d_w.ptr if work else None)
+    tol, etol = (1e-12, 1e-12) if prec == FP64 else (MIXED_TOL, 1e-6)
+    scale = max(np.sqrt((eam_f ** 2).sum(1).mean()), 1e-3)
+    f0 = pick(t.F, types[natoms:] - 1, t.drho, np.zeros(M - natoms)).sum()
+    capi.call("tdmd_eam_compute", tabs.h, d_pos.ptr, d_f.ptr, d_t.ptr, d_nb.ptr, d_off.ptr,
+              d_cnt.ptr, M, C.byref(box), d_rho.ptr, d_fp.ptr, *args, None)
+    got = d_f.download().astype(np.float64)
+    assert np.abs(got[:natoms] - eam_f).max() < tol * scale
+    assert np.all(got[natoms:] == 0.0)
+    assert np.allclose(d_rho.download()[:natoms], rho, rtol=1e-12 if prec == FP64 else 1e-6)
+    if work is not None:
+        assert d_e.download()[0] == pytest.approx(2.5 + eam_e + f0, rel=etol)
+    # Morse over the first natoms rows only
+    d_e = D.from_host(np.array([2.5]))
+    args = (None, None) if work is None else (d_e.ptr, d_w.ptr if work else None)
+    d_f = D.from_host(np.full((M, 3), 7.0, dtype=rdt))
+    p = capi.MorseParams.make(*MORSE_CU)
+    capi.call("tdmd_morse_force", prec, d_pos.ptr, d_f.ptr, d_nb.ptr, d_off.ptr, d_cnt.ptr, natoms,
+              C.byref(box), C.byref(p), *args, None)
+    got = d_f.download().astype(np.float64)
+    scale = max(np.sqrt((morse_f ** 2).sum(1).mean()), 1e-3)
+    assert np.abs(got[:natoms] - morse_f).max() < tol * scale
+    assert np.all(got[natoms:] == 7.0)
+    if work is not None:
+        assert d_e.download()[0] == pytest.approx(2.5 + morse_e, rel=etol)
+
+
 @pytest.mark.parametrize("prec", [FP64, MIXED])
 def test_velocity_verlet_kernels_vs_oracle(prec):
     s = c1()
