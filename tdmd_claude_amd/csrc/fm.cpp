@@ -7,8 +7,9 @@
 //
 // Layout: the snapshots are one concatenated system of nsnap * natoms atoms
 // (AoS FP64 positions) sharing one box; each snapshot's full CSR list is
-// built once at creation with global indices, so every pass is a single
-// launch over all snapshots.
+// built once at creation with global indices, and beside it the half list
+// (neighbours j > i), so every pass is a single launch over all snapshots.
+// Rows are read by eight lanes side by side (csr_rows.hpp).
 //
 // Adjoint (ordered pairs i -> j, d = x_i - x_j, u = d / r, g = F - T):
 //   Morse:  dL/dtheta = sum 2 (g_i . d) dfpair/dtheta        (one pass)
@@ -19,46 +20,58 @@
 //           F     coefficients  (b,c,d)[k(rho_i)] += lam_i (1, 2t, 3t^2),
 //           mu_i = lam_i F''(rho_i),
 //           rho   coefficients  (a,b,c,d)[k(r)] += mu_i (1, t, t^2, t^3).
-//   (w/2 per ordered pair: the two orderings of a pair give w in total.)
+//   (w/2 per ordered pair: the two orderings of a pair give w in total, and
+//   mu_i + mu_j: the histogram pass takes each pair once.)
 // Coefficient gradients go back to knot values through the transpose of the
 // FD-Hermite construction (eam_alloy.cpp:19-50).
 //
+// FP64 (and mixed tables of more points than seven FP32 histograms fit the
+// LDS for) takes three passes: lam_i over full rows; the F coefficients and
+// mu_i per atom; the phi and rho coefficients per unordered pair, seven adds
+// each, in FP64 histograms in LDS where they fit. (One pass over ordered
+// pairs, ten global FP64 atomics each: 21.3 ms an evaluation of 100 x 4,000
+// atoms, 5000 points, 0.8 ms so.)
+//
 // Mixed precision: pair geometry and r in FP64, spline and Morse arithmetic
-// in FP32 (as the forward kernels), per-atom sums FP64; coefficient
-// histograms are accumulated in FP32 in LDS per workgroup and flushed with
-// FP64 atomics, so the gradient is reproducible to FP32 rounding of the
-// per-workgroup partial sums, not bit for bit. FP64 mode accumulates straight
-// into FP64 (global atomics).
+// in FP32 (as the forward kernels), per-atom sums FP64; the r histograms are
+// accumulated in FP32 in LDS per workgroup and flushed with FP64 atomics, so
+// the gradient is reproducible to FP32 rounding of the per-workgroup partial
+// sums, not bit for bit (in FP64 to FP64 rounding).
+#include <cmath>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
-#include "pair_math.hpp"
+#include "csr_rows.hpp"
 
 struct tdmd_fm {
   int precision = TDMD_MIXED;
   int natoms = 0, nsnap = 0, ntot = 0;
   tdmd_box box{};
   double r_list = 0;
+  double r_min = 0;            // shortest listed pair
   double* d_pos = nullptr;     // [ntot][3]
   int32_t* d_cnt = nullptr;    // [ntot]
   int32_t* d_off = nullptr;    // [ntot]
+  int32_t* d_hcnt = nullptr;   // [ntot] half list: neighbours j > i
+  int32_t* d_hoff = nullptr;   // [ntot]
+  int32_t* d_hnbr = nullptr;   // [total / 2]
   int32_t* d_nbr = nullptr;    // [total]
   int32_t* d_types = nullptr;  // [ntot], all 1
   double* d_target = nullptr;  // [ntot][3]
-  double* d_g = nullptr;       // [ntot][3] residual F - T
+  double* d_rec = nullptr;     // [ntot] FmRec, what the adjoint passes gather
   void* d_force = nullptr;     // [ntot][3] in R
   double* d_rho = nullptr;     // [ntot]
   void* d_fp = nullptr;        // [ntot] in R
   double* d_partials = nullptr;
   int nparts = 0;
+  int ncu = 0, lds_max = 0;  // compute units, LDS bytes of a workgroup
   double* d_scalars = nullptr;  // [8]
   bool has_target = false;
   // EAM scratch
   tdmd_eam_tables* tables = nullptr;  // geometry + quads rewritten per call
-  double* d_coef = nullptr;           // [4 niF + 8 niR] FP64 coefficients
   double* d_gcoef = nullptr;          // [4 niF + 8 niR]
-  double* d_gS = nullptr;             // [niF + 2 niR]
   int nrho = 0, nr = 0;
   double drho = 0, dr = 0, cutoff = 0;
 };
@@ -67,17 +80,21 @@ namespace tdmd_hip {
 
 namespace {
 
-constexpr int kFmBlock = 1024;  // adjoint workgroup (LDS histograms)
-constexpr int kHist = 7;        // phi b,c,d; rho a,b,c,d
+// Slots a lane takes at a time; us at 1, 2, 4 (55M ordered pairs, FP32 pair
+// functions): the lambda pass 422, 373, 338; phi's FP64 histograms 233, 202,
+// 219; rho's 238, 226, 258. Bound by their 48- and 64-byte gathers from L2.
+constexpr int kLambdaSlots = 4;
+constexpr int kHistSlots = 2;
+constexpr int kFmBlock = 1024;  // workgroup of the histogram passes
+constexpr int kFmGrid = 2048;   // workgroups (and partials) of the Morse pass, at most
 
-__device__ __forceinline__ double fm_geom(const double* __restrict__ pos, double xi, double yi,
-                                          double zi, int j, const DevBox& box, double* dx,
-                                          double* dy, double* dz) {
-  *dx = min_image(xi - pos[3 * j], box.size[0], 0.5 * box.size[0], box.periodic[0]);
-  *dy = min_image(yi - pos[3 * j + 1], box.size[1], 0.5 * box.size[1], box.periodic[1]);
-  *dz = min_image(zi - pos[3 * j + 2], box.size[2], 0.5 * box.size[2], box.periodic[2]);
-  return *dx * *dx + *dy * *dy + *dz * *dz;
-}
+// What the adjoint passes gather of an atom, 64 bytes: half a cache line; the
+// lambda and phi passes want the first 48 (three 16-byte loads).
+struct alignas(64) FmRec {
+  double x, y, z;     // position
+  double gx, gy, gz;  // residual F - T
+  double fp, mu;      // F'(rho); lam, then mu
+};
 
 template <class R>
 __device__ __forceinline__ R fm_exp(R x);
@@ -91,67 +108,70 @@ __device__ __forceinline__ double fm_exp<double>(double x) {
 }
 
 // ---------------------------------------------------------------------------
-// Morse: forces, residual, loss and dL/d(D, alpha, r0) in one pass.
+// Morse: forces, residual, loss and dL/d(D, alpha, r0) in one sweep of the
+// rows: dL/dtheta = 2 g_i . sum_j d_ij dfpair/dtheta, so the three vectors are
+// summed beside the force and meet g_i at the row's end.
 // partials[blk * 4 + {0: L, 1: dD, 2: dalpha, 3: dr0}]
 // ---------------------------------------------------------------------------
-template <class R>
+template <class R, bool kTarget>
 __global__ void __launch_bounds__(kBlock)
 k_fm_morse(const double* __restrict__ pos, const int32_t* __restrict__ nbr,
-           const int32_t* __restrict__ off, const int32_t* __restrict__ cnt, int ntot, DevBox box,
-           MorseCoef p, const double* __restrict__ target, int has_target,
-           double* __restrict__ forces_out, double* __restrict__ partials) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+           const int32_t* __restrict__ off, const int32_t* __restrict__ cnt, int ntot, PairBox box,
+           MorseCoef p, const double* __restrict__ target, double* __restrict__ forces_out,
+           double* __restrict__ partials) {
   double l = 0.0, gD = 0.0, ga = 0.0, gr = 0.0;
-  if (i < ntot) {
-    const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-    const int o = off[i], c = cnt[i];
+  const R D = static_cast<R>(p.D), al = static_cast<R>(p.alpha);
+  for_atoms<false>(ntot, [&](int i) {
+    const Neighbour a = neighbour_at(pos, i);
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    for (int k = 0; k < c; ++k) {
-      double dx, dy, dz;
-      const double r2 = fm_geom(pos, xi, yi, zi, nbr[o + k], box, &dx, &dy, &dz);
+    double vD[3] = {0.0, 0.0, 0.0}, va[3] = {0.0, 0.0, 0.0}, vr[3] = {0.0, 0.0, 0.0};
+    auto load = [&](int j) { return neighbour_at(pos, j); };
+    for_row<kMorseSlots>(nbr, off[i], cnt[i], a.x, a.y, a.z, box, load,
+                         [&](int, const Neighbour&, double dx, double dy, double dz, double r2) {
       if (r2 < p.rc_sq) {
         const PairR<R> pr = pair_r<R>(r2);
-        R e;
-        const double fpair = static_cast<double>(morse_fpair<R>(p, pr, &e));
+        R en;
+        const double fpair = static_cast<double>(morse_fpair<R>(p, pr, &en));
         fx = fma(fpair, dx, fx);
         fy = fma(fpair, dy, fy);
         fz = fma(fpair, dz, fz);
-      }
-    }
-    // forces as the product path stores them (R)
-    const double Fx = static_cast<double>(static_cast<R>(fx));
-    const double Fy = static_cast<double>(static_cast<R>(fy));
-    const double Fz = static_cast<double>(static_cast<R>(fz));
-    if (forces_out) {
-      forces_out[3 * i] = Fx;
-      forces_out[3 * i + 1] = Fy;
-      forces_out[3 * i + 2] = Fz;
-    }
-    if (has_target) {
-      const double gx = Fx - target[3 * i], gy = Fy - target[3 * i + 1],
-                   gz = Fz - target[3 * i + 2];
-      l = gx * gx + gy * gy + gz * gz;
-      const R D = static_cast<R>(p.D), al = static_cast<R>(p.alpha);
-      for (int k = 0; k < c; ++k) {
-        double dx, dy, dz;
-        const double r2 = fm_geom(pos, xi, yi, zi, nbr[o + k], box, &dx, &dy, &dz);
-        if (r2 < p.rc_sq) {
-          const PairR<R> pr = pair_r<R>(r2);
+        if (kTarget) {
           const R x = static_cast<R>(pr.r - p.r0);
           const R e = fm_exp<R>(-al * x);
           const R one = static_cast<R>(1), two = static_cast<R>(2);
           const R ome = one - e, o2e = one - two * e;
-          const R dfdD = -two * al * ome * e * pr.rinv;
-          const R dfda = -two * D * e * (ome - al * o2e * x) * pr.rinv;
-          const R dfdr = -two * D * al * al * o2e * e * pr.rinv;
-          const double w = 2.0 * (gx * dx + gy * dy + gz * dz);
-          gD = fma(w, static_cast<double>(dfdD), gD);
-          ga = fma(w, static_cast<double>(dfda), ga);
-          gr = fma(w, static_cast<double>(dfdr), gr);
+          const double dfdD = static_cast<double>(-two * al * ome * e * pr.rinv);
+          const double dfda = static_cast<double>(-two * D * e * (ome - al * o2e * x) * pr.rinv);
+          const double dfdr = static_cast<double>(-two * D * al * al * o2e * e * pr.rinv);
+          const double d[3] = {dx, dy, dz};
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            vD[c] = fma(dfdD, d[c], vD[c]);
+            va[c] = fma(dfda, d[c], va[c]);
+            vr[c] = fma(dfdr, d[c], vr[c]);
+          }
         }
       }
+    });
+    // forces as the product path stores them (R)
+    const double F[3] = {static_cast<double>(static_cast<R>(row_sum(fx))),
+                         static_cast<double>(static_cast<R>(row_sum(fy))),
+                         static_cast<double>(static_cast<R>(row_sum(fz)))};
+    const bool first = threadIdx.x % kRowLanes == 0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const size_t at = 3 * static_cast<size_t>(i) + c;
+      if (forces_out && first) forces_out[at] = F[c];
+      if (kTarget) {
+        const double g = F[c] - target[at];
+        if (first) l += g * g;
+        gD = fma(2.0 * g, vD[c], gD);
+        ga = fma(2.0 * g, va[c], ga);
+        gr = fma(2.0 * g, vr[c], gr);
+      }
     }
-  }
+  });
+  if (!kTarget) return;
   const double s0 = block_sum<kBlock>(l);
   const double s1 = block_sum<kBlock>(gD);
   const double s2 = block_sum<kBlock>(ga);
@@ -164,22 +184,20 @@ k_fm_morse(const double* __restrict__ pos, const int32_t* __restrict__ nbr,
   }
 }
 
-// Fixed-order sum of `ncomp` interleaved partial streams.
+// Fixed-order sum of `ncomp` interleaved partial streams, one per workgroup.
 __global__ void k_fm_reduce(const double* __restrict__ partials, int nblk, int ncomp,
                             double* __restrict__ out) {
   __shared__ double s[256];
-  for (int c = 0; c < ncomp; ++c) {
-    double t = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += 256) t += partials[b * ncomp + c];
-    s[threadIdx.x] = t;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if (static_cast<int>(threadIdx.x) < w) s[threadIdx.x] += s[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[c] = s[0];
+  const int c = blockIdx.x;
+  double t = 0.0;
+  for (int b = threadIdx.x; b < nblk; b += 256) t += partials[b * ncomp + c];
+  s[threadIdx.x] = t;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (static_cast<int>(threadIdx.x) < w) s[threadIdx.x] += s[threadIdx.x + w];
     __syncthreads();
   }
+  if (threadIdx.x == 0) out[c] = s[0];
 }
 
 // ---------------------------------------------------------------------------
@@ -187,11 +205,12 @@ __global__ void k_fm_reduce(const double* __restrict__ partials, int nblk, int n
 // ---------------------------------------------------------------------------
 
 // FD-Hermite coefficients from knot values (build_fd_hermite on the device,
-// same operation order, no contraction): spline s = 0 F, 1 rho, 2 phi.
-// coef64: blocks [spline][4][ni]; quads: F, rho, phi intervals in a row.
+// same operation order, no contraction): spline s = 0 F, 1 rho, 2 phi; quads:
+// F, rho, phi intervals in a row. Clears the coefficient gradients (blocks
+// [spline][4][ni]) for the adjoint.
 template <class R>
 __global__ void k_fm_build_coeffs(const double* __restrict__ vals, int nrho, double drho, int nr,
-                                  double dr, double* __restrict__ coef64,
+                                  double dr, double* __restrict__ gcoef,
                                   typename Quad<R>::type* __restrict__ quads) {
 #pragma clang fp contract(off)
   const int s = blockIdx.y;
@@ -213,10 +232,7 @@ __global__ void k_fm_build_coeffs(const double* __restrict__ vals, int nrho, dou
   const int niF = nrho - 1, niR = nr - 1;
   const size_t base = s == 0 ? 0 : (s == 1 ? 4 * static_cast<size_t>(niF)
                                            : 4 * static_cast<size_t>(niF) + 4 * niR);
-  coef64[base + i] = a;
-  coef64[base + ni + i] = b;
-  coef64[base + 2 * ni + i] = c;
-  coef64[base + 3 * ni + i] = d;
+  for (int k = 0; k < 4; ++k) gcoef[base + static_cast<size_t>(k) * ni + i] = 0.0;
   const int qo = s == 0 ? 0 : (s == 1 ? niF : niF + niR);
   typename Quad<R>::type q;
   q.x = static_cast<R>(a);
@@ -229,147 +245,284 @@ __global__ void k_fm_build_coeffs(const double* __restrict__ vals, int nrho, dou
 // Residual g = F - T (F as stored, in R), loss partials (one per block).
 template <class R>
 __global__ void __launch_bounds__(kBlock)
-k_fm_residual(const R* __restrict__ f, const double* __restrict__ target, int ntot,
-              double* __restrict__ g, double* __restrict__ forces_out,
+k_fm_residual(const R* __restrict__ f, const R* __restrict__ fp, const double* __restrict__ target,
+              int ntot, FmRec* __restrict__ rec, double* __restrict__ forces_out,
               double* __restrict__ partials, int has_target) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   double l = 0.0;
   if (i < ntot) {
+    double g[3] = {0.0, 0.0, 0.0};
     for (int c = 0; c < 3; ++c) {
-      const double F = static_cast<double>(f[3 * i + c]);
-      if (forces_out) forces_out[3 * i + c] = F;
+      const size_t at = 3 * static_cast<size_t>(i) + c;
+      const double F = static_cast<double>(f[at]);
+      if (forces_out) forces_out[at] = F;
       if (has_target) {
-        const double gc = F - target[3 * i + c];
-        g[3 * i + c] = gc;
-        l += gc * gc;
+        g[c] = F - target[at];
+        l += g[c] * g[c];
       }
     }
+    rec[i].fp = static_cast<double>(fp[i]);
+    rec[i].gx = g[0];
+    rec[i].gy = g[1];
+    rec[i].gz = g[2];
   }
   const double s = block_sum<kBlock>(l);
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
-struct FmSplines {
-  SplineMeta F, rho, phi;
-  int niF, niR;
-};
+// 1 / r to FP64 rounding: as pair_r has it, or its float seed and one Newton
+// step (relative error ~1e-14).
+__device__ __forceinline__ double inverse(const PairR<double>& p) { return p.rinv; }
+__device__ __forceinline__ double inverse(const PairR<float>& p) {
+  const double y = static_cast<double>(p.rinv);
+  return fma(y, fma(-p.r, y, 1.0), y);
+}
 
-template <bool kLds>
-__device__ __forceinline__ void hist_add(float* hist, double* gglob, int which, int k, int ni,
-                                         double v) {
-  // which: 0..2 phi b,c,d ; 3..6 rho a,b,c,d
+// w_ij = -2 (g_i - g_j) . d_ij / r_ij
+__device__ __forceinline__ double fm_weight(const FmRec& a, const FmRec& b, double dx, double dy,
+                                            double dz, double rinv) {
+  return -2.0 * ((a.gx - b.gx) * dx + (a.gy - b.gy) * dy + (a.gz - b.gz) * dz) * rinv;
+}
+
+// lam_i = sum_j w_ij rho'(r_ij) over full rows, left in rec[i].mu.
+template <class R>
+__global__ void __launch_bounds__(kBlock)
+k_fm_eam_lambda(FmRec* rec, const int32_t* __restrict__ nbr, const int32_t* __restrict__ off,
+                const int32_t* __restrict__ cnt, int ntot, PairBox box, EamLayout t,
+                const typename Quad<R>::type* __restrict__ quads) {
+  for_atoms<false>(ntot, [&](int i) {
+    FmRec a = rec[i];
+    double lam = 0.0;
+    auto load = [&](int j) {
+      FmRec b;  // all but fp and mu, which other workgroups write
+      const FmRec* p = rec + j;
+      b.x = p->x;
+      b.y = p->y;
+      b.z = p->z;
+      b.gx = p->gx;
+      b.gy = p->gy;
+      b.gz = p->gz;
+      return b;
+    };
+    for_row<kLambdaSlots>(nbr, off[i], cnt[i], a.x, a.y, a.z, box, load,
+                         [&](int, const FmRec& b, double dx, double dy, double dz, double r2) {
+      if (r2 < t.rc_sq) {
+        const PairR<R> pr = pair_r<R>(r2);
+        R x;
+        const int k = spline_locate<R>(t.r, pr.r, &x);
+        const R drho = quad_deriv<R>(quads[t.rho_at(0) + k], x);
+        lam = fma(fm_weight(a, b, dx, dy, dz, inverse(pr)), static_cast<double>(drho), lam);
+      }
+    });
+    lam = row_sum(lam);
+    if (threadIdx.x % kRowLanes == 0) rec[i].mu = lam;
+  });
+}
+
+// F coefficients at rho_i and mu_i = lam_i F''(rho_i) (rec[i].mu: lam to mu).
+// The densities of a solid fall on a few hundred of F's intervals, so the
+// three adds an atom go to an LDS histogram first where it fits (kLds).
+template <class R, bool kLds>
+__global__ void __launch_bounds__(kFmBlock)
+k_fm_eam_embed(FmRec* __restrict__ rec, const double* __restrict__ rho, int ntot, EamLayout t,
+               const typename Quad<R>::type* __restrict__ quads, double* __restrict__ gF) {
+  extern __shared__ __align__(16) unsigned char fm_smem[];
+  double* hist = reinterpret_cast<double*>(fm_smem);  // b, c, d
+  const int ni = t.F.n - 1;
   if (kLds) {
-    atomicAdd(&hist[which * ni + k], static_cast<float>(v));
-  } else {
-    // global layout after the F block: rho{a,b,c,d}, phi{a,b,c,d}
-    const size_t blk = which < 3 ? static_cast<size_t>(4 + 1 + which) : static_cast<size_t>(which - 3);
-    atomicAdd(&gglob[blk * ni + k], v);
+    for (int q = threadIdx.x; q < 3 * ni; q += kFmBlock) hist[q] = 0.0;
+    __syncthreads();
+  }
+  double* out = kLds ? hist : gF + ni;  // gF[0, ni): the a block, untouched
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kFmBlock + threadIdx.x; i < ntot;
+       i += static_cast<int64_t>(gridDim.x) * kFmBlock) {
+    const double lam = rec[i].mu;
+    R x;
+    const int k = spline_locate<R>(t.F, rho[i], &x);
+    const double xd = static_cast<double>(x);
+    atomicAdd(&out[k], lam);
+    atomicAdd(&out[ni + k], 2.0 * xd * lam);
+    atomicAdd(&out[2 * ni + k], 3.0 * xd * xd * lam);
+    const auto c = quads[t.f_at(0) + k];
+    rec[i].mu = lam * static_cast<double>(static_cast<R>(2) * c.z + static_cast<R>(6) * c.w * x);
+  }
+  if (kLds) {
+    __syncthreads();
+    for (int q = threadIdx.x; q < 3 * ni; q += kFmBlock)
+      if (hist[q] != 0.0) atomicAdd(&gF[ni + q], hist[q]);
   }
 }
 
-template <class R, bool kLds>
+// phi (b, c, d) and rho (a, b, c, d) coefficients over unordered pairs, the
+// half list. kPhi / kRho: which of them this launch adds (both, or
+// one each where seven histograms do not fit the LDS together). kLds: in
+// LDS, intervals k_lo (that of the set's shortest pair) and up, flushed at
+// the end; else straight to gcoef. Workgroups are persistent, each over a
+// contiguous run of rows.
+template <class R, bool kPhi, bool kRho, bool kLds>
 __global__ void __launch_bounds__(kFmBlock)
-k_fm_eam_adjoint(const double* __restrict__ pos, const int32_t* __restrict__ nbr,
-                 const int32_t* __restrict__ off, const int32_t* __restrict__ cnt, int ntot,
-                 DevBox box, double rc_sq, const typename Quad<R>::type* __restrict__ quads,
-                 FmSplines sp, const double* __restrict__ g, const double* __restrict__ rho,
-                 const R* __restrict__ fp, double* __restrict__ gcoef) {
-  extern __shared__ float hist[];
-  const int niF = sp.niF, niR = sp.niR;
-  double* gF = gcoef;                                  // [4][niF]
-  double* gRP = gcoef + 4 * static_cast<size_t>(niF);  // rho[4][niR], phi[4][niR]
+k_fm_eam_hist(const FmRec* __restrict__ rec, const int32_t* __restrict__ nbr,
+              const int32_t* __restrict__ off, const int32_t* __restrict__ cnt, int ntot,
+              PairBox box, EamLayout t, int k_lo, double* __restrict__ gcoef) {
+  extern __shared__ __align__(16) unsigned char fm_smem[];
+  double* hist = reinterpret_cast<double*>(fm_smem);
+  const int ni = t.r.n - 1, nw = ni - k_lo;
+  constexpr int kN = (kPhi ? 3 : 0) + (kRho ? 4 : 0);
+  constexpr int kRhoAt = kPhi ? 3 : 0;
+  // gcoef after the F block: rho {a,b,c,d}, phi {a,b,c,d}
+  double* g = gcoef + 4 * static_cast<size_t>(t.F.n - 1);
+  auto home = [](int which) { return which < kRhoAt ? 5 + which : which - kRhoAt; };
   if (kLds) {
-    for (int q = threadIdx.x; q < kHist * niR; q += kFmBlock) hist[q] = 0.0f;
+    for (int q = threadIdx.x; q < kN * nw; q += kFmBlock) hist[q] = 0.0;
     __syncthreads();
   }
-  for (int base = blockIdx.x * kFmBlock; base < ntot; base += gridDim.x * kFmBlock) {
-    const int i = base + threadIdx.x;
-    if (i >= ntot) continue;
-    const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-    const double gix = g[3 * i], giy = g[3 * i + 1], giz = g[3 * i + 2];
-    const R fpi = fp[i];
-    const int o = off[i], c = cnt[i];
+  auto add = [&](int which, int k, double v) {
+    if (kLds)
+      atomicAdd(&hist[which * nw + (k - k_lo)], v);
+    else
+      atomicAdd(&g[static_cast<size_t>(home(which)) * ni + k], v);
+  };
+  constexpr int kTurn = kFmBlock / kRowLanes;
+  const int64_t piece = piece_of(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  const int64_t turns = (static_cast<int64_t>(ntot) + kTurn - 1) / kTurn;
+  const int64_t t1 = turns * (piece + 1) / gridDim.x;
+  for (int64_t tt = turns * piece / gridDim.x; tt < t1; ++tt) {
+    const int64_t ii = tt * kTurn + static_cast<int>(threadIdx.x) / kRowLanes;
+    if (ii >= ntot) continue;
+    const int i = static_cast<int>(ii);
+    const FmRec a = rec[i];
+    auto load = [&](int j) { return rec[j]; };
+    for_row<kHistSlots>(nbr, off[i], cnt[i], a.x, a.y, a.z, box, load,
+                         [&](int, const FmRec& b, double dx, double dy, double dz, double r2) {
+      if (r2 < t.rc_sq) {
+        const PairR<R> pr = pair_r<R>(r2);
+        R x;
+        const int k = spline_locate<R>(t.r, pr.r, &x);
+        const double w = fm_weight(a, b, dx, dy, dz, inverse(pr));
+        const double td = static_cast<double>(x);
+        if (kPhi) {
+          add(0, k, w);
+          add(1, k, 2.0 * td * w);
+          add(2, k, 3.0 * td * td * w);
+        }
+        if (kRho) {
+          const double m = a.mu + b.mu;
+          const double wp =
+              w * static_cast<double>(static_cast<R>(a.fp) + static_cast<R>(b.fp));
+          add(kRhoAt, k, m);
+          add(kRhoAt + 1, k, wp + m * td);
+          add(kRhoAt + 2, k, td * (2.0 * wp + m * td));
+          add(kRhoAt + 3, k, td * td * (3.0 * wp + m * td));
+        }
+      }
+    });
+  }
+  if (kLds) {
+    __syncthreads();
+    for (int which = 0; which < kN; ++which)
+      for (int k = threadIdx.x; k < nw; k += kFmBlock) {
+        const double v = hist[which * nw + k];
+        if (v != 0.0) atomicAdd(&g[static_cast<size_t>(home(which)) * ni + k_lo + k], v);
+      }
+  }
+}
+
+// Mixed precision where seven FP32 histograms fit the LDS: the whole adjoint
+// in one pass over ordered pairs, one lane per atom. An FP32 sum of ~100 terms
+// of either sign a bin carries a rounding error that its order decides
+// (1.5e-6 of the gradient), and the adds bound this pass so evenly that two
+// runs differ by less than half of that (0.6e-6): sums in another type or
+// order would move the gradients of existing mixed fits by more than they
+// move from run to run. ~200 cycles per ds_add_f32 of a wavefront, ten a pair,
+// are all of its time (2865 us at 55M ordered pairs of 1M atoms, 5000 points;
+// the FP64 passes take 800).
+__global__ void __launch_bounds__(kFmBlock)
+k_fm_eam_adjoint_f32(const FmRec* __restrict__ rec, const int32_t* __restrict__ nbr,
+                     const int32_t* __restrict__ off, const int32_t* __restrict__ cnt, int ntot,
+                     PairBox box, EamLayout tab, const float4* __restrict__ quads,
+                     const double* __restrict__ rho, double* __restrict__ gcoef) {
+  extern __shared__ __align__(16) unsigned char fm_smem[];
+  float* hist = reinterpret_cast<float*>(fm_smem);  // phi b,c,d; rho a,b,c,d
+  const int niF = tab.F.n - 1, niR = tab.r.n - 1;
+  double* gF = gcoef;                                  // [4][niF]
+  double* gRP = gcoef + 4 * static_cast<size_t>(niF);  // rho[4][niR], phi[4][niR]
+  for (int q = threadIdx.x; q < 7 * niR; q += kFmBlock) hist[q] = 0.0f;
+  __syncthreads();
+  auto add = [&](int which, int k, double v) {
+    atomicAdd(&hist[which * niR + k], static_cast<float>(v));
+  };
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kFmBlock + threadIdx.x; i < ntot;
+       i += static_cast<int64_t>(gridDim.x) * kFmBlock) {
+    const FmRec a = rec[i];
+    const int32_t* row = nbr + off[i];
+    const int c = cnt[i];
     double lam = 0.0;
     for (int k = 0; k < c; ++k) {
-      const int j = nbr[o + k];
-      double dx, dy, dz;
-      const double r2 = fm_geom(pos, xi, yi, zi, j, box, &dx, &dy, &dz);
-      if (r2 < rc_sq) {
-        const PairR<R> pr = pair_r<R>(r2);
-        R t;
-        const int q = spline_locate<R>(sp.rho, pr.r, &t);
-        const auto cr = quads[sp.rho.offset + q];
-        const R drho = cr.y + t * (static_cast<R>(2) * cr.z + t * static_cast<R>(3) * cr.w);
-        const double w = -2.0 *
-                         ((gix - g[3 * j]) * dx + (giy - g[3 * j + 1]) * dy +
-                          (giz - g[3 * j + 2]) * dz) /
-                         pr.r;
+      const FmRec b = rec[row[k]];
+      const double dx = image(a.x - b.x, box.size[0], box.half[0]);
+      const double dy = image(a.y - b.y, box.size[1], box.half[1]);
+      const double dz = image(a.z - b.z, box.size[2], box.half[2]);
+      const double r2 = dx * dx + dy * dy + dz * dz;
+      if (r2 < tab.rc_sq) {
+        const PairR<float> pr = pair_r<float>(r2);
+        float t;
+        const int q = spline_locate<float>(tab.r, pr.r, &t);
+        const float drho = quad_deriv<float>(quads[tab.rho_at(0) + q], t);
+        const double w = fm_weight(a, b, dx, dy, dz, inverse(pr));
         const double hw = 0.5 * w;  // the two orderings of the pair give w
-        const double P = static_cast<double>(fpi + fp[j]);
+        const double P = static_cast<double>(static_cast<float>(a.fp) + static_cast<float>(b.fp));
         const double td = static_cast<double>(t);
-        hist_add<kLds>(hist, gRP, 0, q, niR, hw);
-        hist_add<kLds>(hist, gRP, 1, q, niR, 2.0 * td * hw);
-        hist_add<kLds>(hist, gRP, 2, q, niR, 3.0 * td * td * hw);
-        hist_add<kLds>(hist, gRP, 4, q, niR, hw * P);
-        hist_add<kLds>(hist, gRP, 5, q, niR, 2.0 * td * hw * P);
-        hist_add<kLds>(hist, gRP, 6, q, niR, 3.0 * td * td * hw * P);
+        add(0, q, hw);
+        add(1, q, 2.0 * td * hw);
+        add(2, q, 3.0 * td * td * hw);
+        add(4, q, hw * P);
+        add(5, q, 2.0 * td * hw * P);
+        add(6, q, 3.0 * td * td * hw * P);
         lam = fma(w, static_cast<double>(drho), lam);
       }
     }
-    // F'(rho_i) coefficients and F''(rho_i)
-    R tF;
-    const int qF = spline_locate<R>(sp.F, rho[i], &tF);
+    float tF;
+    const int qF = spline_locate<float>(tab.F, rho[i], &tF);
     const double tFd = static_cast<double>(tF);
     atomicAdd(&gF[niF + qF], lam);
     atomicAdd(&gF[2 * niF + qF], 2.0 * tFd * lam);
     atomicAdd(&gF[3 * niF + qF], 3.0 * tFd * tFd * lam);
-    const auto cF = quads[sp.F.offset + qF];
-    const double mu =
-        lam * static_cast<double>(static_cast<R>(2) * cF.z + static_cast<R>(6) * cF.w * tF);
+    const float4 cF = quads[tab.f_at(0) + qF];
+    const double mu = lam * static_cast<double>(2.0f * cF.z + 6.0f * cF.w * tF);
     for (int k = 0; k < c; ++k) {
-      double dx, dy, dz;
-      const double r2 = fm_geom(pos, xi, yi, zi, nbr[o + k], box, &dx, &dy, &dz);
-      if (r2 < rc_sq) {
-        const PairR<R> pr = pair_r<R>(r2);
-        R t;
-        const int q = spline_locate<R>(sp.rho, pr.r, &t);
+      const FmRec* b = rec + row[k];
+      const double dx = image(a.x - b->x, box.size[0], box.half[0]);
+      const double dy = image(a.y - b->y, box.size[1], box.half[1]);
+      const double dz = image(a.z - b->z, box.size[2], box.half[2]);
+      const double r2 = dx * dx + dy * dy + dz * dz;
+      if (r2 < tab.rc_sq) {
+        float t;
+        const int q = spline_locate<float>(tab.r, pair_r<float>(r2).r, &t);
         const double td = static_cast<double>(t);
-        hist_add<kLds>(hist, gRP, 3, q, niR, mu);
-        hist_add<kLds>(hist, gRP, 4, q, niR, mu * td);
-        hist_add<kLds>(hist, gRP, 5, q, niR, mu * td * td);
-        hist_add<kLds>(hist, gRP, 6, q, niR, mu * td * td * td);
+        add(3, q, mu);
+        add(4, q, mu * td);
+        add(5, q, mu * td * td);
+        add(6, q, mu * td * td * td);
       }
     }
   }
-  if (kLds) {
-    __syncthreads();
-    for (int q = threadIdx.x; q < kHist * niR; q += kFmBlock) {
-      const float v = hist[q];
-      if (v != 0.0f) {
-        const int which = q / niR, k = q - which * niR;
-        const size_t blk = which < 3 ? static_cast<size_t>(4 + 1 + which)
-                                     : static_cast<size_t>(which - 3);
-        atomicAdd(&gRP[blk * niR + k], static_cast<double>(v));
-      }
+  __syncthreads();
+  for (int q = threadIdx.x; q < 7 * niR; q += kFmBlock) {
+    const float v = hist[q];
+    if (v != 0.0f) {
+      const int which = q / niR, k = q - which * niR;
+      atomicAdd(&gRP[static_cast<size_t>(which < 3 ? 5 + which : which - 3) * niR + k],
+                static_cast<double>(v));
     }
   }
 }
 
-// Transpose of the FD-Hermite map, step 1: gS[k] per interval.
-__global__ void k_fm_coef_grad_s(const double* __restrict__ gcoef, int nrho, double drho, int nr,
-                                 double dr, double* __restrict__ gS) {
-  const int s = blockIdx.y;
-  const int niF = nrho - 1, niR = nr - 1;
-  const int ni = s == 0 ? niF : niR;
-  const double h = s == 0 ? drho : dr;
-  const double* gc4 = gcoef + (s == 0 ? 0 : (s == 1 ? 4 * static_cast<size_t>(niF)
-                                                    : 4 * static_cast<size_t>(niF) + 4 * niR));
-  double* out = gS + (s == 0 ? 0 : (s == 1 ? niF : niF + niR));
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= ni) return;
-  const double* gb = gc4 + ni;
-  const double* gc = gc4 + 2 * ni;
-  const double* gd = gc4 + 3 * ni;
+// Transpose of the FD-Hermite map: the knot-value gradient from the
+// coefficient gradients, through S[k], the gradient of interval k's slope.
+__device__ __forceinline__ double fm_slope_grad(const double* __restrict__ gb,
+                                                const double* __restrict__ gc,
+                                                const double* __restrict__ gd, int k, int ni,
+                                                double h) {
   auto gm0 = [&](int q) { return gb[q] - 2.0 * gc[q] / h + gd[q] / (h * h); };
   auto gm1 = [&](int q) { return -gc[q] / h + gd[q] / (h * h); };
   double v = 3.0 * gc[k] / h - 2.0 * gd[k] / (h * h);
@@ -377,41 +530,94 @@ __global__ void k_fm_coef_grad_s(const double* __restrict__ gcoef, int nrho, dou
   if (k + 1 <= ni - 1) v += 0.5 * gm0(k + 1);
   v += (k == ni - 1) ? gm1(k) : 0.5 * gm1(k);
   if (k >= 1) v += 0.5 * gm1(k - 1);
-  out[k] = v;
+  return v;
 }
 
-// Step 2: knot-value gradient gv[m].
-__global__ void k_fm_coef_grad_v(const double* __restrict__ gcoef, const double* __restrict__ gS,
-                                 int nrho, double drho, int nr, double dr,
-                                 double* __restrict__ gv) {
+__global__ void k_fm_coef_grad(const double* __restrict__ gcoef, int nrho, double drho, int nr,
+                               double dr, double* __restrict__ gv) {
   const int s = blockIdx.y;
   const int niF = nrho - 1, niR = nr - 1;
   const int n = s == 0 ? nrho : nr, ni = n - 1;
   const double h = s == 0 ? drho : dr;
   const double* ga = gcoef + (s == 0 ? 0 : (s == 1 ? 4 * static_cast<size_t>(niF)
                                                    : 4 * static_cast<size_t>(niF) + 4 * niR));
-  const double* S = gS + (s == 0 ? 0 : (s == 1 ? niF : niF + niR));
+  const double *gb = ga + ni, *gc = ga + 2 * ni, *gd = ga + 3 * ni;
   double* out = gv + (s == 0 ? 0 : (s == 1 ? nrho : nrho + nr));
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= n) return;
   double v = 0.0;
-  if (m <= ni - 1) v += ga[m] - S[m] / h;
-  if (m >= 1) v += S[m - 1] / h;
+  if (m <= ni - 1) v += ga[m] - fm_slope_grad(gb, gc, gd, m, ni, h) / h;
+  if (m >= 1) v += fm_slope_grad(gb, gc, gd, m - 1, ni, h) / h;
   out[m] = v;
 }
 
-__global__ void k_fm_offset(int32_t* __restrict__ nbr, const int32_t* __restrict__ off,
-                            const int32_t* __restrict__ cnt, int n, int32_t shift) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
+// Rows from the snapshots' local indices to global ones, the half list's
+// counts, and *r2_min: the shortest pair's r^2 (non-negative doubles order as
+// their bits). One wavefront per row.
+__global__ void __launch_bounds__(kBlock)
+k_fm_rows(int32_t* __restrict__ nbr, const int32_t* __restrict__ off,
+          const int32_t* __restrict__ cnt, int ntot, int natoms, const double* __restrict__ pos,
+          PairBox box, int32_t* __restrict__ hcnt, unsigned long long* r2_min) {
+  const int64_t row = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) >> 6;
+  if (row >= ntot) return;
+  const int lane = threadIdx.x & 63;
+  const int i = static_cast<int>(row);
+  const int shift = i / natoms * natoms;
   const int o = off[i], c = cnt[i];
-  for (int k = 0; k < c; ++k) nbr[o + k] += shift;
+  const Neighbour a = neighbour_at(pos, i);
+  int nh = 0;
+  double r2 = __builtin_huge_val();
+  for (int q = lane; q < c; q += kWave) {
+    const int j = nbr[o + q] + shift;
+    nbr[o + q] = j;
+    nh += j > i ? 1 : 0;
+    const Neighbour b = neighbour_at(pos, j);
+    const double dx = image(a.x - b.x, box.size[0], box.half[0]);
+    const double dy = image(a.y - b.y, box.size[1], box.half[1]);
+    const double dz = image(a.z - b.z, box.size[2], box.half[2]);
+    r2 = fmin(r2, dx * dx + dy * dy + dz * dz);
+  }
+  for (int w = 32; w > 0; w >>= 1) {
+    nh += __shfl_xor(nh, w, 64);
+    r2 = fmin(r2, __shfl_xor(r2, w, 64));
+  }
+  if (lane == 0) {
+    hcnt[i] = nh;
+    const auto bits = static_cast<unsigned long long>(__double_as_longlong(r2));
+    if (bits < __hip_atomic_load(r2_min, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMin(r2_min, bits);
+  }
+}
+
+// The half list, each row's neighbours j > i in the row's order.
+__global__ void __launch_bounds__(kBlock)
+k_fm_half(const int32_t* __restrict__ nbr, const int32_t* __restrict__ off,
+          const int32_t* __restrict__ cnt, int ntot, const int32_t* __restrict__ hoff,
+          int32_t* __restrict__ hnbr) {
+  const int64_t row = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) >> 6;
+  if (row >= ntot) return;
+  const int lane = threadIdx.x & 63;
+  const int i = static_cast<int>(row);
+  const int o = off[i], c = cnt[i];
+  int at = hoff[i];
+  for (int k = 0; k < c; k += kWave) {
+    const int j = k + lane < c ? nbr[o + k + lane] : -1;
+    const unsigned long long m = __ballot(j > i);
+    if (j > i) hnbr[at + __popcll(m & ((1ull << lane) - 1ull))] = j;
+    at += __popcll(m);
+  }
+}
+
+__global__ void __launch_bounds__(kBlock)
+k_fm_records(const double* __restrict__ pos, int ntot, FmRec* __restrict__ rec) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (i >= ntot) return;
+  rec[i] = FmRec{pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], 0.0, 0.0, 0.0, 0.0, 0.0};
 }
 
 int fm_free(tdmd_fm* F) {
-  void* ptrs[] = {F->d_pos, F->d_cnt,  F->d_off,      F->d_nbr,     F->d_types,
-                  F->d_target, F->d_g, F->d_force,    F->d_rho,     F->d_fp,
-                  F->d_partials, F->d_scalars, F->d_coef, F->d_gcoef, F->d_gS};
+  void* ptrs[] = {F->d_pos,  F->d_cnt, F->d_off, F->d_nbr, F->d_hcnt, F->d_hoff, F->d_hnbr, F->d_types,
+                  F->d_target, F->d_rec, F->d_force, F->d_rho, F->d_fp, F->d_partials, F->d_scalars, F->d_gcoef};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (F->tables) eam_tables_destroy(F->tables);
@@ -425,6 +631,77 @@ int fm_alloc(T** p, size_t n) {
   const int rc = tdmd_malloc(&q, std::max<size_t>(n, 1) * sizeof(T));
   *p = static_cast<T*>(q);
   return rc;
+}
+
+// The adjoint passes: coefficient gradients in F->d_gcoef (cleared before).
+template <class R>
+int fm_eam_adjoint(tdmd_fm* F, hipStream_t s) {
+  const int N = F->ntot;
+  const size_t niF = static_cast<size_t>(F->nrho - 1), niR = static_cast<size_t>(F->nr - 1);
+  const size_t lmax = static_cast<size_t>(F->lds_max);
+  const PairBox box = make_pair_box(make_devbox(F->box));
+  const EamLayout t = eam_layout(F->tables);
+  const auto* quads = static_cast<const typename Quad<R>::type*>(F->tables->d_coeff);
+  auto* rec = reinterpret_cast<FmRec*>(F->d_rec);
+  // Persistent workgroups of `lds` bytes: as many as the CUs hold (two of
+  // 1024 threads at most), no more than there is work for.
+  auto persistent = [&](size_t lds, int64_t threads) {
+    const int64_t per_cu = 2 * lds <= lmax ? 2 : 1;
+    return static_cast<int>(std::max<int64_t>(
+        1, std::min<int64_t>(per_cu * F->ncu, (threads + kFmBlock - 1) / kFmBlock)));
+  };
+  // (the same limit for every handle: no call lowers another's)
+  auto allow = [&](const void* kernel, size_t lds) -> int {
+    if (lds <= 65536) return TDMD_OK;
+    TDMD_HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     F->lds_max));
+    return TDMD_OK;
+  };
+  if constexpr (std::is_same_v<R, float>) {
+    const size_t lds = 7 * niR * sizeof(float);
+    if (lds + 1024 <= lmax) {
+      if (const int r = allow(reinterpret_cast<const void*>(&k_fm_eam_adjoint_f32), lds)) return r;
+      k_fm_eam_adjoint_f32<<<std::max(1, std::min(grid_for(N, kFmBlock), F->ncu)), kFmBlock, lds,
+                             s>>>(rec, F->d_nbr, F->d_off, F->d_cnt, N, box, t, quads, F->d_rho,
+                                  F->d_gcoef);
+      TDMD_LAUNCH_CHECK();
+      return TDMD_OK;
+    }
+  }
+  k_fm_eam_lambda<R><<<row_grid(N, false), kBlock, 0, s>>>(rec, F->d_nbr, F->d_off, F->d_cnt, N,
+                                                           box, t, quads);
+  TDMD_LAUNCH_CHECK();
+  int rc;
+  const size_t lf = 3 * niF * sizeof(double);
+  if (lf <= lmax) {
+    if ((rc = allow(reinterpret_cast<const void*>(&k_fm_eam_embed<R, true>), lf))) return rc;
+    k_fm_eam_embed<R, true><<<persistent(lf, N), kFmBlock, lf, s>>>(rec, F->d_rho, N, t, quads,
+                                                                    F->d_gcoef);
+  } else {
+    k_fm_eam_embed<R, false><<<persistent(0, N), kFmBlock, 0, s>>>(rec, F->d_rho, N, t, quads,
+                                                                   F->d_gcoef);
+  }
+  TDMD_LAUNCH_CHECK();
+  // no pair of the set lies below interval k_lo (r is exact to rounding; one
+  // interval of margin)
+  const int k_lo = std::max(0, std::min(static_cast<int>(F->r_min / F->dr) - 1, F->nr - 2));
+  const size_t nw = niR - static_cast<size_t>(k_lo);
+  const int64_t threads = static_cast<int64_t>(N) * kRowLanes;
+  auto hist = [&](auto* kernel, size_t lds) -> int {
+    const int r = allow(reinterpret_cast<const void*>(kernel), lds);
+    if (r) return r;
+    kernel<<<persistent(lds, threads), kFmBlock, lds, s>>>(
+        rec, F->d_hnbr, F->d_hoff, F->d_hcnt, N, box, t, k_lo, F->d_gcoef);
+    TDMD_LAUNCH_CHECK();
+    return TDMD_OK;
+  };
+  constexpr size_t d = sizeof(double);
+  if (7 * nw * d <= lmax) return hist(&k_fm_eam_hist<R, true, true, true>, 7 * nw * d);
+  if (4 * nw * d <= lmax) {  // phi's three histograms, then rho's four
+    rc = hist(&k_fm_eam_hist<R, true, false, true>, 3 * nw * d);
+    return rc ? rc : hist(&k_fm_eam_hist<R, false, true, true>, 4 * nw * d);
+  }
+  return hist(&k_fm_eam_hist<R, true, true, false>, 0);
 }
 
 }  // namespace
@@ -454,8 +731,9 @@ int tdmd_fm_create(tdmd_fm** out, int32_t precision, const tdmd_box* box, int32_
   int rc = 0;
   if ((rc = fm_alloc(&F->d_pos, 3 * static_cast<size_t>(N))) ||
       (rc = fm_alloc(&F->d_cnt, N)) || (rc = fm_alloc(&F->d_off, N)) ||
+      (rc = fm_alloc(&F->d_hcnt, N)) || (rc = fm_alloc(&F->d_hoff, N)) ||
       (rc = fm_alloc(&F->d_types, N)) || (rc = fm_alloc(&F->d_target, 3 * static_cast<size_t>(N))) ||
-      (rc = fm_alloc(&F->d_g, 3 * static_cast<size_t>(N))) ||
+      (rc = fm_alloc(&F->d_rec, 8 * static_cast<size_t>(N))) ||
       (rc = fm_alloc(reinterpret_cast<char**>(&F->d_force), 3 * rsz * N)) ||
       (rc = fm_alloc(&F->d_rho, N)) ||
       (rc = fm_alloc(reinterpret_cast<char**>(&F->d_fp), rsz * N)) ||
@@ -464,7 +742,8 @@ int tdmd_fm_create(tdmd_fm** out, int32_t precision, const tdmd_box* box, int32_
     return rc;
   }
   F->nparts = (N + kBlock - 1) / kBlock;
-  if ((rc = fm_alloc(&F->d_partials, 4 * static_cast<size_t>(F->nparts) + 64))) {
+  if ((rc = fm_alloc(&F->d_partials, std::max(4 * static_cast<size_t>(kFmGrid),
+                                              static_cast<size_t>(F->nparts))))) {
     fm_free(F);
     return rc;
   }
@@ -479,8 +758,18 @@ int tdmd_fm_create(tdmd_fm** out, int32_t precision, const tdmd_box* box, int32_
     fm_free(F);
     return hip_fail(e, "hipMemcpy", __FILE__, __LINE__);
   }
+  int dev = 0;
+  e = hipGetDevice(&dev);
+  if (e == hipSuccess)
+    e = hipDeviceGetAttribute(&F->ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e == hipSuccess)
+    e = hipDeviceGetAttribute(&F->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+  if (e != hipSuccess) {
+    fm_free(F);
+    return hip_fail(e, "hipDeviceGetAttribute", __FILE__, __LINE__);
+  }
   // Per-snapshot full lists (cell build + count), one global scan, fill,
-  // then shift each snapshot's indices to global numbering.
+  // then all rows to their global form at once.
   int32_t ncells[3];
   double cs[3];
   if ((rc = tdmd_cell_grid(box, r_cut, ncells, cs))) {
@@ -488,73 +777,66 @@ int tdmd_fm_create(tdmd_fm** out, int32_t precision, const tdmd_box* box, int32_
     return rc;
   }
   const int nc = ncells[0] * ncells[1] * ncells[2];
-  size_t wb = 0;
+  size_t wb = 0, sb = 0;
   tdmd_cell_workspace_bytes(natoms, nc, &wb);
-  std::vector<int32_t*> cc(static_cast<size_t>(nsnap)), co(static_cast<size_t>(nsnap)),
-      ca(static_cast<size_t>(nsnap)), ac(static_cast<size_t>(nsnap));
-  void* work = nullptr;
-  auto cleanup_cells = [&]() {
-    for (int s = 0; s < nsnap; ++s) {
-      for (int32_t* p : {cc[static_cast<size_t>(s)], co[static_cast<size_t>(s)],
-                         ca[static_cast<size_t>(s)], ac[static_cast<size_t>(s)]})
-        if (p) (void)hipFree(p);
-    }
-    if (work) (void)hipFree(work);
+  tdmd_scan_workspace_bytes(N, &sb);
+  const size_t S = static_cast<size_t>(nsnap);
+  int32_t *cc = nullptr, *co = nullptr, *ca = nullptr, *ac = nullptr, *meta = nullptr;
+  char *work = nullptr, *swork = nullptr;
+  if (!(rc = fm_alloc(&cc, S * nc)) && !(rc = fm_alloc(&co, S * nc)) && !(rc = fm_alloc(&ca, N)) &&
+      !(rc = fm_alloc(&ac, N)) && !(rc = fm_alloc(&meta, 4)) && !(rc = fm_alloc(&work, wb)))
+    rc = fm_alloc(&swork, sb);
+  auto cells = [&](int s, auto&& call) {  // call(positions, first atom, cells of snapshot s)
+    const size_t a0 = static_cast<size_t>(s) * natoms, c0 = static_cast<size_t>(s) * nc;
+    return call(F->d_pos + 3 * a0, a0, cc + c0, co + c0, ca + a0, ac + a0);
   };
-  if ((rc = tdmd_malloc(&work, wb))) {
-    fm_free(F);
-    return rc;
-  }
-  for (int s = 0; s < nsnap && !rc; ++s) {
-    const size_t si = static_cast<size_t>(s);
-    const double* ps = F->d_pos + 3 * static_cast<size_t>(s) * natoms;
-    if ((rc = fm_alloc(&cc[si], nc)) || (rc = fm_alloc(&co[si], nc)) ||
-        (rc = fm_alloc(&ca[si], natoms)) || (rc = fm_alloc(&ac[si], natoms)))
-      break;
-    if ((rc = tdmd_cell_build(ps, natoms, box, r_cut, cc[si], co[si], ca[si], ac[si], work,
-                              nullptr)))
-      break;
-    rc = tdmd_nlist_count(ps, natoms, box, r_cut, cc[si], co[si], ca[si], ac[si], ncells,
-                          F->d_cnt + static_cast<size_t>(s) * natoms, nullptr);
-  }
-  size_t sb = 0;
-  void* swork = nullptr;
-  int32_t* meta = nullptr;
-  if (!rc) {
-    tdmd_scan_workspace_bytes(N, &sb);
-    if (!(rc = tdmd_malloc(&swork, sb)) && !(rc = fm_alloc(&meta, 2)))
-      rc = tdmd_scan_exclusive_i32(F->d_cnt, F->d_off, N, meta, swork, nullptr);
-  }
+  for (int s = 0; s < nsnap && !rc; ++s)
+    rc = cells(s, [&](const double* ps, size_t a0, int32_t* c, int32_t* o, int32_t* a, int32_t* k) {
+      const int r = tdmd_cell_build(ps, natoms, box, r_cut, c, o, a, k, work, nullptr);
+      return r ? r
+               : tdmd_nlist_count(ps, natoms, box, r_cut, c, o, a, k, ncells, F->d_cnt + a0,
+                                  nullptr);
+    });
+  if (!rc) rc = tdmd_scan_exclusive_i32(F->d_cnt, F->d_off, N, meta, swork, nullptr);
   int32_t hm[2] = {0, 0};
   if (!rc) {
     e = hipMemcpy(hm, meta, 8, hipMemcpyDeviceToHost);
     if (e != hipSuccess) rc = hip_fail(e, "hipMemcpy", __FILE__, __LINE__);
   }
-  int32_t* ovf = nullptr;
-  if (!rc && !(rc = fm_alloc(&F->d_nbr, std::max(hm[0], 1))) && !(rc = fm_alloc(&ovf, 1))) {
-    (void)hipMemset(ovf, 0, 4);
-    for (int s = 0; s < nsnap && !rc; ++s) {
-      const size_t si = static_cast<size_t>(s);
-      const size_t a0 = static_cast<size_t>(s) * natoms;
-      rc = tdmd_nlist_fill(F->d_pos + 3 * a0, natoms, box, r_cut, cc[si], co[si], ca[si], ac[si],
-                           ncells, F->d_off + a0, F->d_nbr, F->d_cnt + a0, hm[1], ovf, nullptr);
-      if (!rc && s > 0) {
-        k_fm_offset<<<(natoms + kBlock - 1) / kBlock, kBlock>>>(F->d_nbr, F->d_off + a0,
-                                                                F->d_cnt + a0, natoms,
-                                                                static_cast<int32_t>(a0));
-        const hipError_t le = hipGetLastError();
-        if (le != hipSuccess) rc = hip_fail(le, "k_fm_offset", __FILE__, __LINE__);
-      }
+  const size_t total = static_cast<size_t>(std::max(hm[0], 1));
+  if (!rc && !(rc = fm_alloc(&F->d_nbr, total)) &&
+      !(rc = fm_alloc(&F->d_hnbr, total / 2 + 1))) {
+    (void)hipMemset(meta + 2, 0, 4);  // overflow: cannot happen, the rows were counted
+    for (int s = 0; s < nsnap && !rc; ++s)
+      rc = cells(s, [&](const double* ps, size_t a0, int32_t* c, int32_t* o, int32_t* a, int32_t* k) {
+        return tdmd_nlist_fill(ps, natoms, box, r_cut, c, o, a, k, ncells, F->d_off + a0, F->d_nbr,
+                               F->d_cnt + a0, hm[1], meta + 2, nullptr);
+      });
+    if (!rc) {
+      const double none = __builtin_huge_val();
+      e = hipMemcpy(F->d_scalars, &none, sizeof(none), hipMemcpyHostToDevice);
+      if (e != hipSuccess) rc = hip_fail(e, "hipMemcpy", __FILE__, __LINE__);
+      const int rows = grid_for(N, kBlock / kWave);
+      k_fm_rows<<<rows, kBlock>>>(F->d_nbr, F->d_off, F->d_cnt, N, natoms, F->d_pos,
+                                  make_pair_box(make_devbox(*box)), F->d_hcnt,
+                                  reinterpret_cast<unsigned long long*>(F->d_scalars));
+      if (!rc) rc = tdmd_scan_exclusive_i32(F->d_hcnt, F->d_hoff, N, nullptr, swork, nullptr);
+      k_fm_half<<<rows, kBlock>>>(F->d_nbr, F->d_off, F->d_cnt, N, F->d_hoff, F->d_hnbr);
+      k_fm_records<<<grid_for(N), kBlock>>>(F->d_pos, N, reinterpret_cast<FmRec*>(F->d_rec));
+      e = hipGetLastError();
+      if (e != hipSuccess) rc = hip_fail(e, "fm_create rows", __FILE__, __LINE__);
     }
   }
   if (!rc) {
-    e = hipDeviceSynchronize();
-    if (e != hipSuccess) rc = hip_fail(e, "hipDeviceSynchronize", __FILE__, __LINE__);
+    double r2 = 0.0;  // (waits for the launches above)
+    e = hipMemcpy(&r2, F->d_scalars, sizeof(r2), hipMemcpyDeviceToHost);
+    if (e != hipSuccess) rc = hip_fail(e, "hipMemcpy", __FILE__, __LINE__);
+    F->r_min = r2 < r_cut * r_cut ? std::sqrt(r2) : 0.0;
   }
-  cleanup_cells();
-  if (swork) (void)hipFree(swork);
-  if (meta) (void)hipFree(meta);
-  if (ovf) (void)hipFree(ovf);
+  for (void* p : {static_cast<void*>(cc), static_cast<void*>(co), static_cast<void*>(ca),
+                  static_cast<void*>(ac), static_cast<void*>(meta),
+                  static_cast<void*>(work), static_cast<void*>(swork)})
+    if (p) (void)hipFree(p);
   if (rc) {
     fm_free(F);
     return rc;
@@ -595,26 +877,30 @@ int tdmd_fm_morse(tdmd_fm* F, const double params[3], double rc, double* loss, d
   if (rc > F->r_list) return fail(TDMD_E_INVALID, "fm_morse: cutoff beyond the list cutoff");
   if ((loss || grad) && !F->has_target) return fail(TDMD_E_STATE, "fm_morse: no targets set");
   const int N = F->ntot;
-  const DevBox box = make_devbox(F->box);
+  const PairBox box = make_pair_box(make_devbox(F->box));
   const MorseCoef p{params[0], params[1], params[2], rc * rc};
   double* d_fout = nullptr;
   if (forces_out) {
     const int rc2 = fm_alloc(&d_fout, 3 * static_cast<size_t>(N));
     if (rc2) return rc2;
   }
-  const int nb = F->nparts;
+  const int nb = std::min(row_grid(N, false), kFmGrid);
+  const bool want = F->has_target && (loss || grad);
+  auto go = [&](auto kernel) {
+    kernel<<<nb, kBlock>>>(F->d_pos, F->d_nbr, F->d_off, F->d_cnt, N, box, p, F->d_target, d_fout,
+                           F->d_partials);
+  };
   if (F->precision == TDMD_MIXED)
-    k_fm_morse<float><<<nb, kBlock>>>(F->d_pos, F->d_nbr, F->d_off, F->d_cnt, N, box, p,
-                                      F->d_target, F->has_target ? 1 : 0, d_fout, F->d_partials);
+    want ? go(&k_fm_morse<float, true>) : go(&k_fm_morse<float, false>);
   else
-    k_fm_morse<double><<<nb, kBlock>>>(F->d_pos, F->d_nbr, F->d_off, F->d_cnt, N, box, p,
-                                       F->d_target, F->has_target ? 1 : 0, d_fout,
-                                       F->d_partials);
+    want ? go(&k_fm_morse<double, true>) : go(&k_fm_morse<double, false>);
   TDMD_LAUNCH_CHECK();
-  k_fm_reduce<<<1, 256>>>(F->d_partials, nb, 4, F->d_scalars);
-  TDMD_LAUNCH_CHECK();
-  double h[4];
-  TDMD_HIP_TRY(hipMemcpy(h, F->d_scalars, sizeof(h), hipMemcpyDeviceToHost));
+  if (want) {
+    k_fm_reduce<<<4, 256>>>(F->d_partials, nb, 4, F->d_scalars);
+    TDMD_LAUNCH_CHECK();
+  }
+  double h[4] = {0.0, 0.0, 0.0, 0.0};
+  if (want) TDMD_HIP_TRY(hipMemcpy(h, F->d_scalars, sizeof(h), hipMemcpyDeviceToHost));
   if (loss) *loss = h[0];
   if (grad) {
     grad[0] = h[1];
@@ -642,10 +928,8 @@ int tdmd_fm_eam(tdmd_fm* F, int32_t nrho, double drho, int32_t nr, double dr, do
       F->cutoff != cutoff) {
     if (F->tables) eam_tables_destroy(F->tables);
     F->tables = nullptr;
-    for (double** p : {&F->d_coef, &F->d_gcoef, &F->d_gS}) {
-      if (*p) (void)hipFree(*p);
-      *p = nullptr;
-    }
+    if (F->d_gcoef) (void)hipFree(F->d_gcoef);
+    F->d_gcoef = nullptr;
     SetflData sd;
     sd.ntypes = 1;
     sd.nrho = nrho;
@@ -659,9 +943,7 @@ int tdmd_fm_eam(tdmd_fm* F, int32_t nrho, double drho, int32_t nr, double dr, do
     sd.rphi.assign(static_cast<size_t>(nr), 0.0);
     int rc = eam_tables_create(&F->tables, F->precision, sd);
     if (rc) return rc;
-    if ((rc = fm_alloc(&F->d_coef, 4 * static_cast<size_t>(niF) + 8 * static_cast<size_t>(niR))) ||
-        (rc = fm_alloc(&F->d_gcoef, 4 * static_cast<size_t>(niF) + 8 * static_cast<size_t>(niR))) ||
-        (rc = fm_alloc(&F->d_gS, static_cast<size_t>(niF) + 2 * static_cast<size_t>(niR))))
+    if ((rc = fm_alloc(&F->d_gcoef, 4 * static_cast<size_t>(niF) + 8 * static_cast<size_t>(niR))))
       return rc;
     F->nrho = nrho;
     F->nr = nr;
@@ -671,13 +953,12 @@ int tdmd_fm_eam(tdmd_fm* F, int32_t nrho, double drho, int32_t nr, double dr, do
   }
   const bool mixed = F->precision == TDMD_MIXED;
   // FD-Hermite coefficients from the knot values, and the kernels' quads
-  double* d_coef = F->d_coef;
   const dim3 gc((std::max(niF, niR) + 255) / 256, 3);
   if (mixed)
-    k_fm_build_coeffs<float><<<gc, 256, 0, s>>>(d_values, nrho, drho, nr, dr, d_coef,
+    k_fm_build_coeffs<float><<<gc, 256, 0, s>>>(d_values, nrho, drho, nr, dr, F->d_gcoef,
                                                 static_cast<float4*>(F->tables->d_coeff));
   else
-    k_fm_build_coeffs<double><<<gc, 256, 0, s>>>(d_values, nrho, drho, nr, dr, d_coef,
+    k_fm_build_coeffs<double><<<gc, 256, 0, s>>>(d_values, nrho, drho, nr, dr, F->d_gcoef,
                                                  static_cast<double4*>(F->tables->d_coeff));
   TDMD_LAUNCH_CHECK();
   // forward: density, embedding, forces (the drop-in EAM path)
@@ -685,66 +966,25 @@ int tdmd_fm_eam(tdmd_fm* F, int32_t nrho, double drho, int32_t nr, double dr, do
                             F->d_cnt, N, &F->box, F->d_rho, F->d_fp, nullptr, nullptr, stream);
   if (rc) return rc;
   const int nb = F->nparts;
+  auto* rec = reinterpret_cast<FmRec*>(F->d_rec);
   if (mixed)
-    k_fm_residual<float><<<nb, kBlock, 0, s>>>(static_cast<const float*>(F->d_force), F->d_target,
-                                              N, F->d_g, d_forces, F->d_partials,
-                                              F->has_target ? 1 : 0);
+    k_fm_residual<float><<<nb, kBlock, 0, s>>>(
+        static_cast<const float*>(F->d_force), static_cast<const float*>(F->d_fp), F->d_target, N,
+        rec, d_forces, F->d_partials, F->has_target ? 1 : 0);
   else
-    k_fm_residual<double><<<nb, kBlock, 0, s>>>(static_cast<const double*>(F->d_force),
-                                               F->d_target, N, F->d_g, d_forces, F->d_partials,
-                                               F->has_target ? 1 : 0);
+    k_fm_residual<double><<<nb, kBlock, 0, s>>>(
+        static_cast<const double*>(F->d_force), static_cast<const double*>(F->d_fp), F->d_target,
+        N, rec, d_forces, F->d_partials, F->has_target ? 1 : 0);
   TDMD_LAUNCH_CHECK();
   if (d_loss) {
     k_fm_reduce<<<1, 256, 0, s>>>(F->d_partials, nb, 1, d_loss);
     TDMD_LAUNCH_CHECK();
   }
   if (d_grad) {
-    rc = tdmd_fill_u32(F->d_gcoef, 0u,
-                       2 * (4 * static_cast<size_t>(niF) + 8 * static_cast<size_t>(niR)), stream);
+    rc = mixed ? fm_eam_adjoint<float>(F, s) : fm_eam_adjoint<double>(F, s);
     if (rc) return rc;
-    FmSplines sp;
-    SplineMeta m3[3];
-    TDMD_HIP_TRY(hipMemcpy(m3, F->tables->d_meta, sizeof(m3), hipMemcpyDeviceToHost));
-    sp.F = m3[0];
-    sp.rho = m3[1];
-    sp.phi = m3[2];
-    sp.niF = niF;
-    sp.niR = niR;
-    const DevBox box = make_devbox(F->box);
-    int dev = 0, ncu = 0, lmax = 0;
-    TDMD_HIP_TRY(hipGetDevice(&dev));
-    TDMD_HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    TDMD_HIP_TRY(hipDeviceGetAttribute(&lmax, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    const int tiles = (N + kFmBlock - 1) / kFmBlock;
-    const int grid = std::max(1, std::min(tiles, ncu));
-    const size_t lds = static_cast<size_t>(kHist) * niR * sizeof(float);
-    const bool use_lds = mixed && lds + 1024 <= static_cast<size_t>(lmax);
-    const double rc_sq = cutoff * cutoff;
-    if (use_lds) {
-      TDMD_HIP_TRY(hipFuncSetAttribute(
-          reinterpret_cast<const void*>(&k_fm_eam_adjoint<float, true>),
-          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-      k_fm_eam_adjoint<float, true><<<grid, kFmBlock, lds, s>>>(
-          F->d_pos, F->d_nbr, F->d_off, F->d_cnt, N, box, rc_sq,
-          static_cast<const float4*>(F->tables->d_coeff), sp, F->d_g, F->d_rho,
-          static_cast<const float*>(F->d_fp), F->d_gcoef);
-    } else if (mixed) {
-      k_fm_eam_adjoint<float, false><<<grid, kFmBlock, 0, s>>>(
-          F->d_pos, F->d_nbr, F->d_off, F->d_cnt, N, box, rc_sq,
-          static_cast<const float4*>(F->tables->d_coeff), sp, F->d_g, F->d_rho,
-          static_cast<const float*>(F->d_fp), F->d_gcoef);
-    } else {
-      k_fm_eam_adjoint<double, false><<<grid, kFmBlock, 0, s>>>(
-          F->d_pos, F->d_nbr, F->d_off, F->d_cnt, N, box, rc_sq,
-          static_cast<const double4*>(F->tables->d_coeff), sp, F->d_g, F->d_rho,
-          static_cast<const double*>(F->d_fp), F->d_gcoef);
-    }
-    TDMD_LAUNCH_CHECK();
-    const dim3 gs((std::max(niF, niR) + 255) / 256, 3);
-    k_fm_coef_grad_s<<<gs, 256, 0, s>>>(F->d_gcoef, nrho, drho, nr, dr, F->d_gS);
-    TDMD_LAUNCH_CHECK();
     const dim3 gv((std::max(nrho, nr) + 255) / 256, 3);
-    k_fm_coef_grad_v<<<gv, 256, 0, s>>>(F->d_gcoef, F->d_gS, nrho, drho, nr, dr, d_grad);
+    k_fm_coef_grad<<<gv, 256, 0, s>>>(F->d_gcoef, nrho, drho, nr, dr, d_grad);
     TDMD_LAUNCH_CHECK();
   }
   TDMD_HIP_TRY(hipStreamSynchronize(s));

@@ -111,9 +111,10 @@ class ForceMatchSet:
         v = values.detach().contiguous()
         if v.dtype != torch.float64 or not v.is_cuda or v.numel() != grid.nvalues:
             raise ValueError("values must be a float64 CUDA tensor of nrho + 2 nr entries")
-        loss = torch.zeros(1, dtype=torch.float64, device=v.device) if want_loss else None
-        grad = torch.zeros_like(v) if want_grad else None
-        forces = (torch.zeros((self.ntot, 3), dtype=torch.float64, device=v.device)
+        # every element is written by the call
+        loss = torch.empty(1, dtype=torch.float64, device=v.device) if want_loss else None
+        grad = torch.empty_like(v) if want_grad else None
+        forces = (torch.empty((self.ntot, 3), dtype=torch.float64, device=v.device)
                   if want_forces else None)
         stream = torch.cuda.current_stream(v.device).cuda_stream
         capi.call("tdmd_fm_eam", self._h, grid.nrho, grid.drho, grid.nr, grid.dr, grid.cutoff,

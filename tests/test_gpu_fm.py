@@ -112,6 +112,38 @@ def test_fm_eam_loss_and_gradient_vs_oracle(prec, nr):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("prec,nr,cells,nsnap", [("fp64", 5000, 3, 2), ("fp64", 2000, 3, 1),
+                                                 ("fp64", 12000, 3, 2), ("mixed", 12000, 3, 2),
+                                                 ("mixed", 2000, 5, 3)])
+def test_fm_eam_gradient_by_every_histogram_path(prec, nr, cells, nsnap):
+    """Seven histograms in LDS at once, phi's and rho's in turn, and straight
+    to memory where neither fits (12,000 points); F's in LDS and, at 12,000
+    points, in memory. Bounds of the test above."""
+    import torch
+
+    say(f"fm eam paths {prec} nr={nr} {nsnap}x{4 * cells ** 3}")
+    base, snaps = snapshots(n=nsnap, cells=cells)
+    t, values, grid, (F, rho, phi) = eam_case(nr)
+    _, _, _, targets = oracle_eam(base, snaps, grid, F * 1.03, rho * 0.98, phi * 1.05)
+    L0, G0, C0, _ = oracle_eam(base, snaps, grid, F, rho, phi, targets)
+    fm = fitting.ForceMatchSet(base.lo, base.hi, snaps, grid.cutoff, prec)
+    fm.set_targets(targets)
+    v = torch.tensor(values, dtype=torch.float64, device="cuda")
+    for _ in range(2):  # the second call finds used buffers
+        loss, grad, _ = fm.eam(v, grid)
+        torch.cuda.synchronize()
+        gerr = np.linalg.norm(grad.cpu().numpy() - G0) / np.linalg.norm(G0)
+        cerr = np.linalg.norm(fm.eam_coef_grad(grid) - C0) / np.linalg.norm(C0)
+        lerr = abs(float(loss.cpu()[0]) / L0 - 1)
+        say(f"  loss err {lerr:.2e}, grad err {gerr:.2e}, coef err {cerr:.2e}")
+        if prec == "fp64":
+            assert lerr < 1e-10 and gerr < 1e-9 and cerr < 1e-9
+        else:
+            assert lerr < 2e-4 and gerr < 2e-3 and cerr < 2e-3
+    fm.close()
+
+
+@pytest.mark.gpu
 def test_fm_eam_fp64_gradient_matches_its_finite_differences():
     import torch
 
