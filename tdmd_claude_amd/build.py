@@ -29,6 +29,12 @@ SOURCES = [
     "forces_csr.cpp",
     "integrate.cpp",
     "scheduler.cpp",
+    "sched_engine_fixed.cpp",
+    "sched_engine_mixed_f64.cpp",
+    "sched_engine_fp64.cpp",
+    "sched_engine_batch_fixed.cpp",
+    "sched_engine_batch_mixed_f64.cpp",
+    "sched_engine_batch_fp64.cpp",
     "fm.cpp",
     "pipeline.cpp",
 ]

@@ -291,6 +291,53 @@ struct StepArgs {
   int pair_nint;  // r intervals per element pair
 };
 
+struct GridArgs {
+  int n[3];
+  double inv_cs[3];
+  int ncells;
+  const int32_t* rank_of;  // linear cell id -> Morton rank
+  const int32_t* around;   // [ncells][27] by rank: ranks of the 27 cells
+                           // around the cell (periodic wrap), increasing
+  const uint8_t* around_img;  // the same entries' periodic images: 2 bits per
+                              // axis, 1 = +box length, 2 = -box length
+  int images;  // 1: every periodic axis has >= 3 cells no smaller than r_list,
+               // so a stencil entry's image is the minimum image of any pair
+               // within r_list that it holds (batches: per box, BoxGeo)
+  int nl_split;  // 1: the fused rebuild searches each atom's cells with 32 lanes
+  int32_t* ccount;         // [ncells] by rank; zero between rebuilds
+  int32_t* cstart;         // [ncells + 1] by rank: cell r's slots [cstart[r], cstart[r + 1])
+  int32_t* cursor;         // [ncells] by rank; zero between rebuilds
+  int32_t* key;            // [N] rank of each atom's cell (old order)
+  int32_t* sidx;           // [N] new slot -> old index
+  int32_t* orig;           // [N] upload index
+  int32_t* done;           // completion counter
+  int32_t* wsum;           // [kMaxScanGroups] per-workgroup cell sums (fused rebuild)
+};
+
+constexpr int kMaxScanGroups = 4096;  // workgroups of the fused rebuild, at most
+// Up to this many cells every workgroup of the fused rebuild scans them for
+// itself, into LDS, instead of the whole grid around two more barriers.
+constexpr int kScanOwn = 4096;
+
+struct PermArgs {
+  // scratch arrays the permutation gathers into
+  double *px, *py, *pz, *vx, *vy, *vz;
+  void *fx, *fy, *fz;
+  int32_t *types, *orig;
+};
+
+// Arrival is two-level: the workgroups of XCD group x (blockIdx % 8 == x)
+// count at sub[32 x], and the last of each group counts at `count`; the
+// last of those bumps `gen`. Arrivals on one address are serialised, so 512
+// workgroups on a single counter took ~30 us a barrier; eight counters of
+// at most 64 arrivals each, on separate 128-byte lines, take a fraction.
+struct GridBarrier {
+  unsigned int count;  // groups arrived
+  unsigned int gen;    // generation: bumped when every group has arrived
+  unsigned int pad[30];
+  unsigned int sub[8 * 32];  // workgroups arrived in group x: sub[32 x]
+};
+
 // Pass clock: every workgroup stamps the device wall clock at entry; the
 // last workgroup to finish a launch adds the span from the earliest stamp
 // to its own finish to the running total and re-arms the words for the

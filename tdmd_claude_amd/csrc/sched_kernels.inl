@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(kBlock) k_ke_partials(StepArgs a) {
   emit_partial(e, a.partials, blockIdx.x);
 }
 
-__global__ void k_scale_v(StepArgs a) {
+static __global__ void k_scale_v(StepArgs a) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= a.natoms) return;
   const double s = a.nhc[24];
@@ -211,7 +211,7 @@ __global__ void k_scale_v(StepArgs a) {
 
 // Before the VV step: half-step on the KE of the actual velocities
 // (vscale^2 * stored KE), kick scale = s1 * vscale.
-__global__ void k_nhc_pre(double* nhc, NhcParams p) {
+static __global__ void k_nhc_pre(double* nhc, NhcParams p) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   const double ke = nhc[24] * nhc[24] * nhc[25];
   const double s1 = nhc_half_step(p.M, nhc, nhc + 8, nhc + 16, p.t_target, p.t_period, p.dt,
@@ -251,7 +251,7 @@ __global__ void k_nhc_post(double* nhc, const double* partials, int n, NhcParams
 }
 
 // Stored-KE refresh (after upload, or after the pending scale was applied).
-__global__ void k_nhc_set_ke(double* nhc, const double* partials, int n, int commit_scale) {
+static __global__ void k_nhc_set_ke(double* nhc, const double* partials, int n, int commit_scale) {
   __shared__ double s[256];
   double t = 0.0;
   for (int k = threadIdx.x; k < n; k += 256) t += partials[k];
@@ -268,7 +268,7 @@ __global__ void k_nhc_set_ke(double* nhc, const double* partials, int n, int com
 }
 
 // Window end: the pending factor has been applied to v by k_scale_v.
-__global__ void k_nhc_commit(double* nhc) {
+static __global__ void k_nhc_commit(double* nhc) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   nhc[25] *= nhc[24] * nhc[24];
   nhc[24] = 1.0;
@@ -684,47 +684,11 @@ __global__ void __launch_bounds__(kBlock) k_morse_force(StepArgs a, MorseCoef p)
 // sit in a captured graph and only does work on steps that need it.
 // ---------------------------------------------------------------------------
 
-struct GridArgs {
-  int n[3];
-  double inv_cs[3];
-  int ncells;
-  const int32_t* rank_of;  // linear cell id -> Morton rank
-  const int32_t* around;   // [ncells][27] by rank: ranks of the 27 cells
-                           // around the cell (periodic wrap), increasing
-  const uint8_t* around_img;  // the same entries' periodic images: 2 bits per
-                              // axis, 1 = +box length, 2 = -box length
-  int images;  // 1: every periodic axis has >= 3 cells no smaller than r_list,
-               // so a stencil entry's image is the minimum image of any pair
-               // within r_list that it holds (batches: per box, BoxGeo)
-  int nl_split;  // 1: the fused rebuild searches each atom's cells with 32 lanes
-  int32_t* ccount;         // [ncells] by rank
-  int32_t* cstart;         // [ncells] by rank
-  int32_t* cursor;         // [ncells] by rank
-  int32_t* key;            // [N] rank of each atom's cell (old order)
-  int32_t* sidx;           // [N] new slot -> old index
-  int32_t* orig;           // [N] upload index
-  int32_t* done;           // completion counter
-  int32_t* wsum;           // [kMaxScanGroups] per-workgroup cell sums (fused rebuild)
-};
-
-constexpr int kMaxScanGroups = 4096;  // workgroups of the fused rebuild, at most
-// Up to this many cells the fused rebuild scans them with one workgroup
-// (~1.6 ns a cell) instead of the whole grid around one more barrier.
-constexpr int kScanOneGroup = 4096;
-
-
-struct PermArgs {
-  // scratch arrays the permutation gathers into
-  double *px, *py, *pz, *vx, *vy, *vz;
-  void *fx, *fy, *fz;
-  int32_t *types, *orig;
-};
-
-__global__ void k_set_flag(int32_t* flags) {
+static __global__ void k_set_flag(int32_t* flags) {
   if (threadIdx.x == 0 && blockIdx.x == 0) flags[0] = 1;
 }
 
-__global__ void __launch_bounds__(kBlock) k_zero_cells(const int32_t* flags, GridArgs g) {
+static __global__ void __launch_bounds__(kBlock) k_zero_cells(const int32_t* flags, GridArgs g) {
   if (!flags[0]) return;
   const int r = blockIdx.x * kBlock + threadIdx.x;
   if (r >= g.ncells) return;
@@ -787,9 +751,10 @@ __device__ __forceinline__ void bin_atom(const StepArgs& a, const GridArgs& g, i
 
 // Exclusive scan of the cell counts by one workgroup of BLOCK threads
 // (atomics-free): thread t owns a contiguous chunk of cells, sums it, the
-// workgroup scans the chunk sums, and each thread writes its chunk's starts.
+// workgroup scans the chunk sums, and each thread writes its chunk's starts;
+// out[ncells] = N.
 template <int BLOCK>
-__device__ __forceinline__ void scan_cells(const GridArgs& g) {
+__device__ __forceinline__ void scan_cells(const GridArgs& g, int32_t* out) {
   __shared__ int wsum[BLOCK / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int chunk = (g.ncells + BLOCK - 1) / BLOCK;
@@ -807,16 +772,17 @@ __device__ __forceinline__ void scan_cells(const GridArgs& g) {
   int base = incl - v;
   for (int k = 0; k < w; ++k) base += wsum[k];
   for (int c = c0; c < c1; ++c) {
-    g.cstart[c] = base;
+    out[c] = base;
     base += g.ccount[c];
   }
+  if (threadIdx.x == BLOCK - 1) out[g.ncells] = base;
 }
 
 // (The order of a cell's atoms after the scatter is the atomics' order;
 // the ordering pass then sorts each cell by upload index.)
-__device__ __forceinline__ void scatter_atom(const GridArgs& g, int i) {
+__device__ __forceinline__ void scatter_atom(const GridArgs& g, int i, const int32_t* cstart) {
   const int r = g.key[i];
-  g.sidx[g.cstart[r] + wave_add_one(g.cursor, r)] = i;
+  g.sidx[cstart[r] + wave_add_one(g.cursor, r)] = i;
 }
 
 // Inclusive scan of v over the workgroup (BLOCK threads); *total gets the
@@ -873,12 +839,11 @@ __device__ __forceinline__ void scan_cells_grid(const GridArgs& g, int phase) {
     if (cc < c1) g.cstart[cc] = run + incl - n;
     run += total;
   }
+  if (c1 == g.ncells && c0 < c1 && threadIdx.x == 0) g.cstart[g.ncells] = run;
 }
 
 // Deterministic order inside a cell: by upload index.
-__device__ __forceinline__ void order_cell(const GridArgs& g, int r) {
-  int32_t* seg = g.sidx + g.cstart[r];
-  const int n = g.ccount[r];
+__device__ __forceinline__ void order_cell(const GridArgs& g, int32_t* seg, int n) {
   for (int x = 1; x < n; ++x) {
     const int32_t v = seg[x];
     const int32_t kv = g.orig[v];
@@ -893,38 +858,46 @@ __device__ __forceinline__ void order_cell(const GridArgs& g, int r) {
 
 // The same order by one wavefront: lane l takes the cell's l-th atom and
 // counts the atoms with a smaller upload index (indices are unique, so the
-// counts are the sorted positions); all lanes read before any writes.
-// Cells of more than 64 atoms fall back to one lane's insertion sort.
-__device__ __forceinline__ void order_cell_wave(const GridArgs& g, int r) {
+// counts are the sorted positions); put(old index, new slot) for each atom.
+// Cells of more than 64 atoms are sorted in place by one lane first.
+template <class Put>
+__device__ __forceinline__ void order_cell_wave(const GridArgs& g, int r, Put&& put) {
   const int lane = static_cast<int>(threadIdx.x & 63);
-  int32_t* seg = g.sidx + g.cstart[r];
-  const int n = g.ccount[r];
+  const int start = g.cstart[r], n = g.cstart[r + 1] - start;
+  int32_t* seg = g.sidx + start;
   if (n > 64) {
-    if (lane == 0) order_cell(g, r);
+    if (lane == 0) order_cell(g, seg, n);
+    // lane 0's stores are complete before the other lanes read them
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    for (int k = lane; k < n; k += 64) put(seg[k], start + k);
     return;
   }
   const int32_t v = lane < n ? seg[lane] : 0;
   const int32_t kv = lane < n ? g.orig[v] : 0x7fffffff;
   int pos = 0;
   for (int m = 0; m < n; ++m) pos += __shfl(kv, m, 64) < kv ? 1 : 0;
-  if (lane < n) seg[pos] = v;
+  if (lane < n) put(v, start + pos);
 }
 
-template <class R>
+// Atom o (old slot) to slot s of the scratch arrays, and its gather record.
+template <class R, class Mir>
 __device__ __forceinline__ void permute_atom(const StepArgs& a, const GridArgs& g,
-                                             const PermArgs& t, int s) {
-  const int o = g.sidx[s];
-  t.px[s] = a.px[o];
-  t.py[s] = a.py[o];
-  t.pz[s] = a.pz[o];
+                                             const PermArgs& t, int o, int s) {
+  const double x = a.px[o], y = a.py[o], z = a.pz[o];
+  const int32_t ty = a.types[o];
+  t.px[s] = x;
+  t.py[s] = y;
+  t.pz[s] = z;
   t.vx[s] = a.vx[o];
   t.vy[s] = a.vy[o];
   t.vz[s] = a.vz[o];
   rp<R>(t.fx)[s] = rp<R>(a.fx)[o];
   rp<R>(t.fy)[s] = rp<R>(a.fy)[o];
   rp<R>(t.fz)[s] = rp<R>(a.fz)[o];
-  t.types[s] = a.types[o];
+  t.types[s] = ty;
   t.orig[s] = g.orig[o];
+  static_cast<typename Mir::T*>(a.M)[s] = Mir::encode(mp_of<Mir>(a, s), x, y, z, ty - 1);
 }
 
 template <class R, class Mir>
@@ -950,10 +923,8 @@ __device__ __forceinline__ void copyback_atom(const StepArgs& a, const GridArgs&
   rp<R>(a.fx)[s] = rp<R>(t.fx)[s];
   rp<R>(a.fy)[s] = rp<R>(t.fy)[s];
   rp<R>(a.fz)[s] = rp<R>(t.fz)[s];
-  const int ty = t.types[s];
-  const_cast<int32_t*>(a.types)[s] = ty;
+  const_cast<int32_t*>(a.types)[s] = t.types[s];
   g.orig[s] = t.orig[s];
-  static_cast<typename Mir::T*>(a.M)[s] = Mir::encode(mp_of<Mir>(a, s), x, y, z, ty - 1);
 }
 
 // Candidate prefilter of the list search with the 32-bit fixed-point
@@ -1003,7 +974,9 @@ __device__ __forceinline__ float pre_r2(const int4& mj, const int4& mi, const Pr
   return dx * dx + dy * dy + dz * dz;
 }
 
-// ELL row of atom i over the sorted atoms; returns the true count. Inclusion
+// ELL row of atom i over the sorted atoms, whose positions are read from the
+// sort's scratch arrays (the state's own are being written back beside the
+// search); returns the true count. Inclusion
 // exactly as the CPU list (neighbor_list.cpp:58-62): d = x_j - x_i in FP64,
 // single minimum image, unfused r2 < r_list^2. kCount: only count.
 //
@@ -1015,12 +988,13 @@ __device__ __forceinline__ float pre_r2(const int4& mj, const int4& mi, const Pr
 // shell. Near entries are written from the front and shell entries from the
 // back of the row; the shell block is then moved down behind the near block.
 template <bool kCount, class Mir>
-__device__ __forceinline__ int nlist_atom(const StepArgs& a, const GridArgs& g, int i,
+__device__ __forceinline__ int nlist_atom(const StepArgs& a, const GridArgs& g, const PermArgs& p,
+                                          int i,
                                           double r_list_sq, double near_sq, int32_t* nbr,
                                           int32_t* cnt) {
   int count = 0, nn = 0, nf = 0;
   const int cap = a.cap;
-  const double xi = a.px[i], yi = a.py[i], zi = a.pz[i];
+  const double xi = p.px[i], yi = p.py[i], zi = p.pz[i];
   const MirrorParams& mp = mp_of<Mir>(a, i);
   const CellGrid cg = grid_of<Mir>(a, g, i);
   int c[3];
@@ -1050,7 +1024,7 @@ __device__ __forceinline__ int nlist_atom(const StepArgs& a, const GridArgs& g, 
     constexpr bool kIsoU = decltype(iso_units)::value;
     for (int t = 0; t < 27; ++t) {
       const int r = around[t];
-      const int start = g.cstart[r], end = start + g.ccount[r];
+      const int start = g.cstart[r], end = g.cstart[r + 1];
       // kImg: the cell's image offset replaces the per-candidate minimum
       // image test: x_j - x_i then +-L, the same two roundings, so r2 is
       // bit for bit that of the test for every pair within r_list
@@ -1066,7 +1040,7 @@ __device__ __forceinline__ int nlist_atom(const StepArgs& a, const GridArgs& g, 
         sz = ((img >> 4) & 3) == 1 ? mp.L[2] : -mp.L[2];
       }
       auto exact_r2 = [&](int j) {
-        double ddx = a.px[j] - xi, ddy = a.py[j] - yi, ddz = a.pz[j] - zi;
+        double ddx = p.px[j] - xi, ddy = p.py[j] - yi, ddz = p.pz[j] - zi;
         if constexpr (kImg) {
           ddx = ix ? ddx + sx : ddx;
           ddy = iy ? ddy + sy : ddy;
@@ -1142,10 +1116,11 @@ __device__ __forceinline__ int nlist_atom(const StepArgs& a, const GridArgs& g, 
         double px[4], py[4], pz[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int j = min(j0 + q, end - 1);
-          px[q] = a.px[j];
-          py[q] = a.py[j];
-          pz[q] = a.pz[j];
+          // an FP64 record holds the position itself
+          const typename Mir::T m = static_cast<const typename Mir::T*>(a.M)[min(j0 + q, end - 1)];
+          px[q] = m.x;
+          py[q] = m.y;
+          pz[q] = m.z;
         }
         double r2q[4];
 #pragma unroll
@@ -1223,15 +1198,16 @@ __device__ __forceinline__ int nlist_atom(const StepArgs& a, const GridArgs& g, 
 // Distance arithmetic is nlist_atom's, so the row is bit for bit the same.
 // Every lane of the wave runs the loop (the ballots and shuffles need
 // them); `act` is false for a half with no atom, whose i is any valid atom.
-template <class Mir>
-__device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArgs& g, int i,
+template <bool kCount, class Mir>
+__device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArgs& g,
+                                                const PermArgs& p, int i,
                                                 bool act, double r_list_sq, double near_sq,
                                                 int32_t* nbr, int32_t* cnt) {
   const int lane = static_cast<int>(threadIdx.x & 63);
   const int l = lane & 31, sh = lane & 32;
   const uint32_t lt = (1u << l) - 1u;
   const int cap = a.cap;
-  const double xi = a.px[i], yi = a.py[i], zi = a.pz[i];
+  const double xi = p.px[i], yi = p.py[i], zi = p.pz[i];
   const MirrorParams& mp = mp_of<Mir>(a, i);
   const CellGrid cg = grid_of<Mir>(a, g, i);
   int c[3];
@@ -1247,7 +1223,7 @@ __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArg
   if (act && l < 27) {
     const int r = g.around[row + l];
     my_start = g.cstart[r];
-    my_end = my_start + g.ccount[r];
+    my_end = g.cstart[r + 1];
     my_img = g.around_img[row + l];
   }
   int4 mi_rec = make_int4(0, 0, 0, 0);
@@ -1272,7 +1248,17 @@ __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArg
       const bool valid = j < end;
       const int jj = valid ? j : i;
       auto exact_r2 = [&]() {
-        double ddx = a.px[jj] - xi, ddy = a.py[jj] - yi, ddz = a.pz[jj] - zi;
+        double ddx, ddy, ddz;
+        if constexpr (Mir::kFixed) {
+          ddx = p.px[jj] - xi;
+          ddy = p.py[jj] - yi;
+          ddz = p.pz[jj] - zi;
+        } else {  // an FP64 record holds the position itself
+          const typename Mir::T m = static_cast<const typename Mir::T*>(a.M)[jj];
+          ddx = m.x - xi;
+          ddy = m.y - yi;
+          ddz = m.z - zi;
+        }
         if (images) {
           ddx = ix ? ddx + sx : ddx;
           ddy = iy ? ddy + sy : ddy;
@@ -1305,6 +1291,10 @@ __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArg
       }
       const bool hit = valid && j != i && in_list;
       const uint32_t hg = static_cast<uint32_t>(__ballot(hit) >> sh);
+      if constexpr (kCount) {
+        count += __popc(hg);
+        continue;
+      }
       const bool kept = hit && count + __popc(hg & lt) < cap;
       const bool near = kept && in_near;
       const uint32_t kg = static_cast<uint32_t>(__ballot(kept) >> sh);
@@ -1320,6 +1310,7 @@ __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArg
       nf += __popc(kg & ~ng);
     }
   }
+  if constexpr (kCount) return act ? count : 0;
   // the row stores above are complete before the shell entries are read back
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -1365,31 +1356,25 @@ __global__ void __launch_bounds__(kBlock) k_bin(StepArgs a, GridArgs g) {
   bin_atom<Mir>(a, g, i);
 }
 
-__global__ void __launch_bounds__(1024) k_cell_scan(const int32_t* flags, GridArgs g) {
+static __global__ void __launch_bounds__(1024) k_cell_scan(const int32_t* flags, GridArgs g) {
   if (!flags[0]) return;
-  scan_cells<1024>(g);
+  scan_cells<1024>(g, g.cstart);
 }
 
-__global__ void __launch_bounds__(kBlock) k_scatter(StepArgs a, GridArgs g) {
+static __global__ void __launch_bounds__(kBlock) k_scatter(StepArgs a, GridArgs g) {
   if (!a.flags[0]) return;
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= a.natoms) return;
-  scatter_atom(g, i);
+  scatter_atom(g, i, g.cstart);
 }
 
-__global__ void __launch_bounds__(kBlock) k_order(StepArgs a, GridArgs g) {
+// One wavefront per cell.
+template <class R, class Mir>
+__global__ void __launch_bounds__(kBlock) k_order_permute(StepArgs a, GridArgs g, PermArgs t) {
   if (!a.flags[0]) return;
-  const int r = blockIdx.x * kBlock + threadIdx.x;
+  const int r = blockIdx.x * (kBlock / 64) + static_cast<int>(threadIdx.x >> 6);
   if (r >= g.ncells) return;
-  order_cell(g, r);
-}
-
-template <class R>
-__global__ void __launch_bounds__(kBlock) k_permute(StepArgs a, GridArgs g, PermArgs t) {
-  if (!a.flags[0]) return;
-  const int s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= a.natoms) return;
-  permute_atom<R>(a, g, t, s);
+  order_cell_wave(g, r, [&](int o, int s) { permute_atom<R, Mir>(a, g, t, o, s); });
 }
 
 template <class R, class Mir>
@@ -1400,20 +1385,30 @@ __global__ void __launch_bounds__(kBlock) k_copyback(StepArgs a, GridArgs g, Per
   copyback_atom<R, Mir>(a, g, t, s);
 }
 
-template <bool kCount, class Mir>
+// kSplit: two atoms per wavefront (nlist_atom_group).
+template <bool kCount, bool kSplit, class Mir>
 __global__ void __launch_bounds__(kBlock)
-k_nlist_ell(StepArgs a, GridArgs g, double r_list_sq, double near_sq, int32_t* nbr, int32_t* cnt,
-            int32_t* maxcnt) {
+k_nlist_ell(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double near_sq, int32_t* nbr,
+            int32_t* cnt, int32_t* maxcnt) {
   if (!kCount && !a.flags[0]) return;
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const int gi = blockIdx.x * kBlock + threadIdx.x;
   int count = 0;
-  if (i < a.natoms) count = nlist_atom<kCount, Mir>(a, g, i, r_list_sq, near_sq, nbr, cnt);
+  if constexpr (kSplit) {
+    const int i = gi >> 5, base = (gi >> 6) * 2;
+    if (base < a.natoms) {
+      const bool act = i < a.natoms;
+      count = nlist_atom_group<kCount, Mir>(a, g, t, act ? i : base, act, r_list_sq, near_sq, nbr,
+                                            cnt);
+    }
+  } else if (gi < a.natoms) {
+    count = nlist_atom<kCount, Mir>(a, g, t, gi, r_list_sq, near_sq, nbr, cnt);
+  }
   report_count<kCount>(a, count, maxcnt);
 }
 
 // End of a rebuild: the last block to finish clears the flag (every block has
 // read it by then), so the next step's kernels see a clean state.
-__global__ void __launch_bounds__(kBlock) k_rebuild_done(int32_t* flags, int32_t* done,
+static __global__ void __launch_bounds__(kBlock) k_rebuild_done(int32_t* flags, int32_t* done,
                                                          int nblocks, int64_t* rebuilds) {
   if (!flags[0]) return;
   __syncthreads();
@@ -1690,7 +1685,7 @@ __device__ __forceinline__ void build_halos(const StepArgs& a, int nblocks, Halo
 }
 
 // Standalone halo build after a rebuild by separate kernels (flags[4]).
-__global__ void __launch_bounds__(kHaloBlock) k_halo(StepArgs a, int nblocks, int32_t* done) {
+static __global__ void __launch_bounds__(kHaloBlock) k_halo(StepArgs a, int nblocks, int32_t* done) {
   if (!a.flags[4]) return;
   __shared__ HaloLds L;
   build_halos(a, nblocks, L);
@@ -1706,7 +1701,10 @@ __global__ void __launch_bounds__(kHaloBlock) k_halo(StepArgs a, int nblocks, in
 // ---------------------------------------------------------------------------
 // Fused rebuild: the whole sort + list sequence in one launch, its phases
 // separated by a grid barrier, so a step that needs no rebuild costs one
-// early-returning launch instead of nine.
+// early-returning launch instead of seven. The phases: bin | scan + scatter |
+// order + permute (records, scratch arrays) | copy back + list (| halos); a
+// barrier costs 3-7 us, so work moves into a neighbouring phase where its
+// inputs allow.
 //
 // The grid is sized by the host to what the device holds resident at once
 // (occupancy x CUs), so every workgroup of the launch runs concurrently and
@@ -1724,18 +1722,6 @@ __global__ void __launch_bounds__(kHaloBlock) k_halo(StepArgs a, int nblocks, in
 // (phases such as the cell scan run on one workgroup), and polls back off
 // with a growing sleep.
 // ---------------------------------------------------------------------------
-
-// Arrival is two-level: the workgroups of XCD group x (blockIdx % 8 == x)
-// count at sub[32 x], and the last of each group counts at `count`; the
-// last of those bumps `gen`. Arrivals on one address are serialised, so 512
-// workgroups on a single counter took ~30 us a barrier; eight counters of
-// at most 64 arrivals each, on separate 128-byte lines, take a fraction.
-struct GridBarrier {
-  unsigned int count;  // groups arrived
-  unsigned int gen;    // generation: bumped when every group has arrived
-  unsigned int pad[30];
-  unsigned int sub[8 * 32];  // workgroups arrived in group x: sub[32 x]
-};
 
 constexpr long kBarrierSpins = 1L << 22;
 
@@ -1800,35 +1786,40 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
   const int tid = blockIdx.x * kRebuildBlock + threadIdx.x;
   const int nthr = gridDim.x * kRebuildBlock;
   const int N = a.natoms;
-  for (int r = tid; r < g.ncells; r += nthr) {
-    g.ccount[r] = 0;
-    g.cursor[r] = 0;
-  }
-  if (!grid_barrier(bar, a.flags)) return;
+  // (the cell counters are clear: the phase that last reads them clears them)
   for (int i = tid; i < N; i += nthr) bin_atom<Mir>(a, g, i);
   if (!grid_barrier(bar, a.flags)) return;
-  if (g.ncells <= kScanOneGroup) {
-    // few cells: one workgroup scans them faster than a second barrier
-    if (blockIdx.x == 0) scan_cells<kRebuildBlock>(g);
+  if (g.ncells <= kScanOwn) {
+    // few cells: every workgroup scans them for itself, without a barrier
+    __shared__ int32_t cstart[kScanOwn + 1];
+    scan_cells<kRebuildBlock>(g, cstart);
+    __syncthreads();
+    if (blockIdx.x == 0)
+      for (int r = threadIdx.x; r <= g.ncells; r += kRebuildBlock) g.cstart[r] = cstart[r];
+    for (int i = tid; i < N; i += nthr) scatter_atom(g, i, cstart);
   } else {
     scan_cells_grid<kRebuildBlock>(g, 1);
     if (!grid_barrier(bar, a.flags)) return;
     scan_cells_grid<kRebuildBlock>(g, 2);
+    if (!grid_barrier(bar, a.flags)) return;
+    for (int i = tid; i < N; i += nthr) scatter_atom(g, i, g.cstart);
   }
-  if (!grid_barrier(bar, a.flags)) return;
-  for (int i = tid; i < N; i += nthr) scatter_atom(g, i);
   if (!grid_barrier(bar, a.flags)) return;
   {
     // one cell per wavefront, cells dealt to the workgroups wave by wave
     const int nw = gridDim.x * (kRebuildBlock / 64);
     const int wv = (threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-    for (int r = wv; r < g.ncells; r += nw) order_cell_wave(g, r);
+    for (int r = wv; r < g.ncells; r += nw)
+      order_cell_wave(g, r, [&](int o, int s) { permute_atom<R, Mir>(a, g, t, o, s); });
+    for (int r = tid; r < g.ncells; r += nthr) {
+      g.ccount[r] = 0;
+      g.cursor[r] = 0;
+    }
   }
   if (!grid_barrier(bar, a.flags)) return;
-  for (int s = tid; s < N; s += nthr) permute_atom<R>(a, g, t, s);
-  if (!grid_barrier(bar, a.flags)) return;
+  // the state's arrays back from the scratch ones, beside the list search,
+  // which reads the scratch arrays and the records
   for (int s = tid; s < N; s += nthr) copyback_atom<R, Mir>(a, g, t, s);
-  if (!grid_barrier(bar, a.flags)) return;
   int count = 0;
   if (g.nl_split) {
     // two atoms per wavefront, 32 lanes each; the loop bound is uniform per wave
@@ -1836,13 +1827,13 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
     for (int base = 2 * gw; base < N; base += 2 * nw) {
       const int i = base + static_cast<int>((threadIdx.x >> 5) & 1);
       const bool act = i < N;
-      const int c = nlist_atom_group<Mir>(a, g, act ? i : base, act, r_list_sq, near_sq, nbr,
-                                          cnt);
+      const int c = nlist_atom_group<false, Mir>(a, g, t, act ? i : base, act, r_list_sq, near_sq,
+                                                 nbr, cnt);
       count = c > count ? c : count;
     }
   } else {
     for (int i = tid; i < N; i += nthr) {
-      const int c = nlist_atom<false, Mir>(a, g, i, r_list_sq, near_sq, nbr, cnt);
+      const int c = nlist_atom<false, Mir>(a, g, t, i, r_list_sq, near_sq, nbr, cnt);
       count = c > count ? c : count;
     }
   }
