@@ -326,16 +326,22 @@ struct PermArgs {
   int32_t *types, *orig;
 };
 
-// Arrival is two-level: the workgroups of XCD group x (blockIdx % 8 == x)
-// count at sub[32 x], and the last of each group counts at `count`; the
-// last of those bumps `gen`. Arrivals on one address are serialised, so 512
-// workgroups on a single counter took ~30 us a barrier; eight counters of
-// at most 64 arrivals each, on separate 128-byte lines, take a fraction.
+// Grid barrier of the fused rebuild: arrivals counted without end (mod 2^32),
+// so nothing is reset between barriers; `gen` holds the barriers passed before
+// this launch. Up to kBarrierFlat workgroups arrive on `count`; more arrive on
+// their XCD group's counter (blockIdx % 8, each on its own 128-byte line), and
+// the last of each group on `count`. us a barrier, all on one counter / by
+// groups: 8 workgroups 1.3 / 1.7, 32 1.9 / 2.8, 128 3.9 / 4.3, 256 9.6 / 6.7,
+// 512 34 / 14 (with an acquire and a release at every arrival and a reset by
+// the last one 2.7, 3.9, 5.7, 9.0, 17.8).
+constexpr unsigned int kBarrierFlat = 128;
+
 struct GridBarrier {
-  unsigned int count;  // groups arrived
-  unsigned int gen;    // generation: bumped when every group has arrived
-  unsigned int pad[30];
-  unsigned int sub[8 * 32];  // workgroups arrived in group x: sub[32 x]
+  unsigned int count;
+  unsigned int pad0[31];
+  unsigned int gen;
+  unsigned int pad1[31];
+  unsigned int sub[8 * 32];  // group x: sub[32 x]
 };
 
 // Pass clock: every workgroup stamps the device wall clock at entry; the

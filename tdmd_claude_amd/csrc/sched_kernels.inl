@@ -1703,7 +1703,7 @@ static __global__ void __launch_bounds__(kHaloBlock) k_halo(StepArgs a, int nblo
 // separated by a grid barrier, so a step that needs no rebuild costs one
 // early-returning launch instead of seven. The phases: bin | scan + scatter |
 // order + permute (records, scratch arrays) | copy back + list (| halos); a
-// barrier costs 3-7 us, so work moves into a neighbouring phase where its
+// barrier costs 1.3-7 us, so work moves into a neighbouring phase where its
 // inputs allow.
 //
 // The grid is sized by the host to what the device holds resident at once
@@ -1713,58 +1713,57 @@ static __global__ void __launch_bounds__(kHaloBlock) k_halo(StepArgs a, int nblo
 // polls sets flags[3] and the kernel returns (the host reports the error)
 // instead of hanging.
 //
-// Only thread 0 of each workgroup touches the barrier. Its arrival is a
-// release and its wait ends with an acquire fence at agent scope, and the
-// workgroup barriers on either side extend both to the other threads: one
-// L2 write-back and one invalidate per workgroup and phase, not one per
-// wave. The polls themselves are relaxed loads: an acquiring poll would
-// invalidate the XCD's L2 at every poll, under the workgroups still working
-// (phases such as the cell scan run on one workgroup), and polls back off
-// with a growing sleep.
+// Only thread 0 of each workgroup touches the barrier: one release fence, a
+// relaxed arrival, relaxed polls, one acquire fence, all at agent scope, and
+// the workgroup barriers on either side extend them to the other threads: one
+// L2 write-back and one invalidate per workgroup and phase. (An acquiring poll
+// would invalidate the XCD's L2 at every poll, under the workgroups still
+// working.) Polls back off with a growing sleep.
 // ---------------------------------------------------------------------------
 
 constexpr long kBarrierSpins = 1L << 22;
 
-__device__ __forceinline__ bool grid_barrier(GridBarrier* b, int32_t* flags) {
+// `passed`: barriers this workgroup has passed (GridBarrier::gen at the
+// launch's start, counted on here).
+__device__ __forceinline__ bool grid_barrier(GridBarrier* b, unsigned int* passed,
+                                             int32_t* flags) {
   __shared__ int ok;
   __syncthreads();
+  const unsigned int n = ++*passed;
   if (threadIdx.x == 0) {
     ok = 1;
-    const unsigned int gen =
-        __hip_atomic_load(&b->gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned int x = blockIdx.x & 7u;
-    const unsigned int nx = (gridDim.x - x + 7u) >> 3;  // workgroups in group x
-    const unsigned int ngroups = gridDim.x < 8u ? gridDim.x : 8u;
-    unsigned int* sub = &b->sub[32u * x];
-    const unsigned int arrived =
-        __hip_atomic_fetch_add(sub, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-    bool last = false;
-    if (arrived == nx - 1u) {  // last of its group: arrive at the top
-      __hip_atomic_store(sub, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const unsigned int top =
-          __hip_atomic_fetch_add(&b->count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-      last = top == ngroups - 1u;
-    }
-    if (last) {
-      __hip_atomic_store(&b->count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(&b->gen, gen + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned int target = n * gridDim.x;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    if (gridDim.x <= kBarrierFlat) {
+      __hip_atomic_fetch_add(&b->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else {
-      long spins = 0;
-      while (__hip_atomic_load(&b->gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gen) {
-        if (spins < 16)
-          __builtin_amdgcn_s_sleep(2);
-        else if (spins < 256)
-          __builtin_amdgcn_s_sleep(16);
-        else
-          __builtin_amdgcn_s_sleep(64);
-        if (++spins > kBarrierSpins) {
-          ok = 0;
-          atomicExch(&flags[3], 1);
-          break;
-        }
+      const unsigned int x = blockIdx.x & 7u;
+      const unsigned int nx = (gridDim.x - x + 7u) >> 3;  // workgroups in group x
+      target = n * 8u;
+      if (__hip_atomic_fetch_add(&b->sub[32u * x], 1u, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT) == n * nx - 1u) {
+        // last of its group: passes on what the group's arrivals released
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
+        __hip_atomic_fetch_add(&b->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
+    long spins = 0;
+    while (static_cast<int>(__hip_atomic_load(&b->count, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT) -
+                            target) < 0) {
+      if (spins < 64)
+        __builtin_amdgcn_s_sleep(1);
+      else if (spins < 256)
+        __builtin_amdgcn_s_sleep(16);
+      else
+        __builtin_amdgcn_s_sleep(64);
+      if (++spins > kBarrierSpins) {
+        ok = 0;
+        atomicExch(&flags[3], 1);
+        break;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();
   return ok != 0;
@@ -1786,9 +1785,10 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
   const int tid = blockIdx.x * kRebuildBlock + threadIdx.x;
   const int nthr = gridDim.x * kRebuildBlock;
   const int N = a.natoms;
+  unsigned int passed = bar->gen;  // written below once every workgroup has read it
   // (the cell counters are clear: the phase that last reads them clears them)
   for (int i = tid; i < N; i += nthr) bin_atom<Mir>(a, g, i);
-  if (!grid_barrier(bar, a.flags)) return;
+  if (!grid_barrier(bar, &passed, a.flags)) return;
   if (g.ncells <= kScanOwn) {
     // few cells: every workgroup scans them for itself, without a barrier
     __shared__ int32_t cstart[kScanOwn + 1];
@@ -1799,12 +1799,12 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
     for (int i = tid; i < N; i += nthr) scatter_atom(g, i, cstart);
   } else {
     scan_cells_grid<kRebuildBlock>(g, 1);
-    if (!grid_barrier(bar, a.flags)) return;
+    if (!grid_barrier(bar, &passed, a.flags)) return;
     scan_cells_grid<kRebuildBlock>(g, 2);
-    if (!grid_barrier(bar, a.flags)) return;
+    if (!grid_barrier(bar, &passed, a.flags)) return;
     for (int i = tid; i < N; i += nthr) scatter_atom(g, i, g.cstart);
   }
-  if (!grid_barrier(bar, a.flags)) return;
+  if (!grid_barrier(bar, &passed, a.flags)) return;
   {
     // one cell per wavefront, cells dealt to the workgroups wave by wave
     const int nw = gridDim.x * (kRebuildBlock / 64);
@@ -1816,7 +1816,7 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
       g.cursor[r] = 0;
     }
   }
-  if (!grid_barrier(bar, a.flags)) return;
+  if (!grid_barrier(bar, &passed, a.flags)) return;
   // the state's arrays back from the scratch ones, beside the list search,
   // which reads the scratch arrays and the records
   for (int s = tid; s < N; s += nthr) copyback_atom<R, Mir>(a, g, t, s);
@@ -1841,7 +1841,7 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
   if constexpr (Mir::kFixed) {
     if (a.stage_cap > 0) {  // halos of the staged passes, from the new rows
       __shared__ HaloLds L;
-      if (!grid_barrier(bar, a.flags)) return;
+      if (!grid_barrier(bar, &passed, a.flags)) return;
       static_assert(kRebuildBlock == kHaloBlock, "halos are built by whole workgroups");
       build_halos(a, (N + kHaloBlock - 1) / kHaloBlock, L);
     }
@@ -1850,6 +1850,7 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
   if (tid == 0) {
     a.flags[0] = 0;
     *rebuilds += 1;
+    bar->gen = passed;
   }
 }
 
