@@ -32,9 +32,6 @@ using namespace sched;
 constexpr int kSplitLanes = 8;
 constexpr int kSplitMax = 131072;     // Morse
 constexpr int kEamSplitMax = 65536;   // EAM
-// The fused rebuild's list search takes 32 lanes per atom up to this size.
-constexpr int kNlistSplitMax = 131072;
-
 // Operation codes of a step sequence (also the graph-cache key alphabet).
 enum Op : char {
   OP_BOOT = 'b',        // half kick + drift (window start, NVE)
@@ -307,6 +304,18 @@ struct Engine final : EngineBase {
     S->nb_force = lds ? nb_lds : S->nblocks * lanes;
   }
 
+  // Workgroups of the list search and of the fused rebuild: a cell each up to
+  // 64, two each beyond (the rebuild of 864 atoms in 27 cells: 30.9 us with 27,
+  // 34.6 with 14; of 10,976 in 216: 50.4 with 216, 45.7 with 108: a barrier
+  // costs more the more arrive at it); one a CU and one per 32 atoms at most, so
+  // that several small systems can be resident together. Under the displacement
+  // policy the launch is a no-op check on nearly every step: one per 512 atoms.
+  int list_grid(int ncu) const {
+    const int per = S->cfg.rebuild_policy == TDMD_REBUILD_DISPLACEMENT ? 512 : 32;
+    const int cells = std::min(S->g.ncells, std::max(64, (S->g.ncells + 1) / 2));
+    return std::max(1, std::min({ncu, (S->natoms + per - 1) / per, cells}));
+  }
+
   int init() override {
     // rows split over kSplitLanes lanes when one lane per atom would leave
     // the chip mostly idle (partials: one per block of the larger grid)
@@ -322,23 +331,8 @@ struct Engine final : EngineBase {
       TDMD_HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
       TDMD_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(
           &per_cu, reinterpret_cast<const void*>(&k_rebuild_fused<R, Mir>), kRebuildBlock, 0));
-      // at most two workgroups per CU: a margin under the occupancy limit.
-      // Small systems search each atom's cells with 32 lanes (one lane per
-      // atom leaves the search a chain of dependent loads on a few CUs) --
-      // under the fixed-interval policy. Under the displacement policy the
-      // launch is a no-op check on nearly every step (a 32,000-atom Morse
-      // system rebuilds once in 10,000 steps), and a grid sized for 32
-      // lanes per atom makes every check dispatch 16 times more workgroups:
-      // there the search takes one lane per atom.
-      const bool split = S->natoms <= kNlistSplitMax &&
-                         S->cfg.rebuild_policy != TDMD_REBUILD_DISPLACEMENT;
-      const int64_t lanes = static_cast<int64_t>(S->natoms) * (split ? 32 : 1);
-      const int need = static_cast<int>(
-          std::max<int64_t>((lanes + kRebuildBlock - 1) / kRebuildBlock, 1));
-      S->nb_rebuild = std::max(1, std::min(std::min(per_cu, 2) * ncu, need));
-      S->nb_rebuild = std::min(S->nb_rebuild, sched::kMaxScanGroups);
+      S->nb_rebuild = list_grid(ncu);
       if (per_cu < 1) S->nb_rebuild = 0;  // cannot guarantee residency: separate kernels
-      S->g.nl_split = split && S->nb_rebuild > 0 ? 1 : 0;
     }
     if (S->kind == 1 && S->tables->ntypes > 1) return build_pair_table();
     if (S->kind != 1 || S->tables->ntypes != 1) return TDMD_OK;
@@ -643,20 +637,13 @@ struct Engine final : EngineBase {
     TDMD_LAUNCH_CHECK();
     return TDMD_OK;
   }
-  // Counts (into *d_max) or rows of the sorted atoms; 32 lanes an atom for
-  // systems that one lane an atom would leave most of the chip idle for.
+  // Counts (into *d_max) or rows of the sorted atoms.
   template <bool kCount>
   void nlist(hipStream_t s, int32_t* d_max) {
-    const double rl2 = S->r_list * S->r_list, rc2 = S->cutoff * S->cutoff;
-    int32_t* nbr = kCount ? nullptr : const_cast<int32_t*>(S->a.nbr);
-    int32_t* cnt = kCount ? nullptr : const_cast<int32_t*>(S->a.cnt);
-    if (S->natoms <= kNlistSplitMax)
-      k_nlist_ell<kCount, true, Mir>
-          <<<grid_for(static_cast<int64_t>(S->natoms) * 32), kBlock, 0, s>>>(
-              S->a, S->g, S->t, rl2, rc2, nbr, cnt, d_max);
-    else
-      k_nlist_ell<kCount, false, Mir><<<grid_for(S->natoms), kBlock, 0, s>>>(
-          S->a, S->g, S->t, rl2, rc2, nbr, cnt, d_max);
+    k_nlist_ell<kCount, Mir><<<std::min(256, (S->g.ncells + 1) / 2), kListBlock, 0, s>>>(
+        S->a, S->g, S->t, S->r_list * S->r_list, S->cutoff * S->cutoff,
+        kCount ? nullptr : const_cast<int32_t*>(S->a.nbr),
+        kCount ? nullptr : const_cast<int32_t*>(S->a.cnt), d_max);
   }
   int fill_pass(hipStream_t s) override {
     const int gb = grid_for(S->natoms);

@@ -45,11 +45,6 @@ constexpr int kMaxSplines = 64;
 // for the atom's own term and its neighbours'.
 constexpr int kPackedTypes = 4;
 
-// Spare records allocated past the last atom in each gather-record buffer:
-// the list search loads a cell's candidates in whole groups of eight from
-// the cell's first atom, masking the slots past the cell's end.
-constexpr int kRecPad = 8;
-
 struct MirrorParams {
   double lo[3];
   double q[3];     // fixed-point units per A (MirrorFixed)
@@ -303,7 +298,6 @@ struct GridArgs {
   int images;  // 1: every periodic axis has >= 3 cells no smaller than r_list,
                // so a stencil entry's image is the minimum image of any pair
                // within r_list that it holds (batches: per box, BoxGeo)
-  int nl_split;  // 1: the fused rebuild searches each atom's cells with 32 lanes
   int32_t* ccount;         // [ncells] by rank; zero between rebuilds
   int32_t* cstart;         // [ncells + 1] by rank: cell r's slots [cstart[r], cstart[r + 1])
   int32_t* cursor;         // [ncells] by rank; zero between rebuilds

@@ -974,228 +974,29 @@ __device__ __forceinline__ float pre_r2(const int4& mj, const int4& mi, const Pr
   return dx * dx + dy * dy + dz * dz;
 }
 
-// ELL row of atom i over the sorted atoms, whose positions are read from the
-// sort's scratch arrays (the state's own are being written back beside the
-// search); returns the true count. Inclusion
-// exactly as the CPU list (neighbor_list.cpp:58-62): d = x_j - x_i in FP64,
-// single minimum image, unfused r2 < r_list^2. kCount: only count.
+// The list search. ELL rows over the sorted atoms, whose positions are read
+// from the sort's scratch arrays (the state's own are being written back
+// beside the search). Inclusion exactly as the CPU list
+// (neighbor_list.cpp:58-62): d = x_j - x_i in FP64, single minimum image,
+// unfused r2 < r_list^2. kCount: only count.
 //
 // Each row is partitioned: neighbours inside the interaction cutoff at build
 // time first, the skin shell (rc <= r < r_list) after them. Atoms move less
 // than half the skin between builds, so in the force passes the in-cutoff
 // test is true for the leading slots and false for the trailing ones in
 // nearly every lane of a wave, and whole waves skip the pair work of the
-// shell. Near entries are written from the front and shell entries from the
-// back of the row; the shell block is then moved down behind the near block.
-template <bool kCount, class Mir>
-__device__ __forceinline__ int nlist_atom(const StepArgs& a, const GridArgs& g, const PermArgs& p,
-                                          int i,
-                                          double r_list_sq, double near_sq, int32_t* nbr,
-                                          int32_t* cnt) {
-  int count = 0, nn = 0, nf = 0;
-  const int cap = a.cap;
-  const double xi = p.px[i], yi = p.py[i], zi = p.pz[i];
-  const MirrorParams& mp = mp_of<Mir>(a, i);
-  const CellGrid cg = grid_of<Mir>(a, g, i);
-  int c[3];
-  cell_coords(cg, xi, yi, zi, c);
-  // The 27 cells around c, visited in increasing rank. Atoms are sorted by
-  // cell rank, so each row comes out in increasing atom index, and the
-  // lanes of a wave (neighbouring atoms with overlapping neighbourhoods)
-  // reach the same stretch of the record array at the same slot.
-  const int32_t* __restrict__ around =
-      g.around + 27 * static_cast<size_t>(
-                          g.rank_of[cg.off + (c[2] * cg.n[1] + c[1]) * cg.n[0] + c[0]]);
-  const size_t row = static_cast<size_t>(around - g.around);
-  int4 mi_rec = make_int4(0, 0, 0, 0);
-  PreBounds pb{};
-  if constexpr (Mir::kFixed) {
-    mi_rec = static_cast<const int4*>(a.M)[i];
-    pb = pre_bounds(mp, r_list_sq, near_sq);
-  }
-  // One copy of the search per image mode, so the loop body has no branch
-  // between a group's coordinate loads and they issue together.
-  // Row slots are addressed from the row's first slot: slot k is
-  // (k / 4) * 256 + k % 4 elements on (the ELL layout of ell()).
-  int32_t* const rowp = kCount ? nullptr : nbr + ell(i, 0, cap);
-  auto slot = [&](int k) -> int32_t& { return rowp[(k >> 2) * 256 + (k & 3)]; };
-  auto search = [&](auto images, auto iso_units) {
-    constexpr bool kImg = decltype(images)::value;
-    constexpr bool kIsoU = decltype(iso_units)::value;
-    for (int t = 0; t < 27; ++t) {
-      const int r = around[t];
-      const int start = g.cstart[r], end = g.cstart[r + 1];
-      // kImg: the cell's image offset replaces the per-candidate minimum
-      // image test: x_j - x_i then +-L, the same two roundings, so r2 is
-      // bit for bit that of the test for every pair within r_list
-      double sx = 0.0, sy = 0.0, sz = 0.0;
-      bool ix = false, iy = false, iz = false;
-      if constexpr (kImg) {
-        const int img = g.around_img[row + t];
-        ix = (img & 3) != 0;
-        iy = ((img >> 2) & 3) != 0;
-        iz = ((img >> 4) & 3) != 0;
-        sx = (img & 3) == 1 ? mp.L[0] : -mp.L[0];
-        sy = ((img >> 2) & 3) == 1 ? mp.L[1] : -mp.L[1];
-        sz = ((img >> 4) & 3) == 1 ? mp.L[2] : -mp.L[2];
-      }
-      auto exact_r2 = [&](int j) {
-        double ddx = p.px[j] - xi, ddy = p.py[j] - yi, ddz = p.pz[j] - zi;
-        if constexpr (kImg) {
-          ddx = ix ? ddx + sx : ddx;
-          ddy = iy ? ddy + sy : ddy;
-          ddz = iz ? ddz + sz : ddz;
-        } else {
-          ddx = min_image(ddx, mp.L[0], mp.hL[0], mp.periodic[0]);
-          ddy = min_image(ddy, mp.L[1], mp.hL[1], mp.periodic[1]);
-          ddz = min_image(ddz, mp.L[2], mp.hL[2], mp.periodic[2]);
-        }
-        return r2_unfused(ddx, ddy, ddz);
-      };
-      if constexpr (Mir::kFixed) {
-        // one 16-byte record per candidate, prefiltered in FP32; the exact
-        // test where the prefilter is too close to call
-        const char* __restrict__ Mb = static_cast<const char*>(a.M);
-        for (int j0 = start; j0 < end; j0 += 8) {
-          // A group of eight candidates: their prefilter decisions in
-          // straight-line code, so the eight record loads are issued together
-          // and consumed there (with the distance computed under each
-          // candidate's branch the compiler re-issued the first load inside
-          // its branch and waited on it); the exact test of the rare in-band
-          // candidates and the appends follow. (Groups of four: 1M-atom
-          // rebuild 2.09 ms; eight 2.00; sixteen 2.06.) The eight records
-          // are read from the group's first at fixed offsets, also past the
-          // cell's end (the buffer has kRecPad spare records at its end);
-          // those slots are masked.
-          const int4* __restrict__ g8 =
-              reinterpret_cast<const int4*>(Mb + (static_cast<uint32_t>(j0) << 4));
-          bool in[8], near[8], band[8];
-          bool any_band = false;
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            const int j = j0 + q;
-            const float r2f = pre_r2<kIsoU>(g8[q], mi_rec, pb);
-            // bitwise, not short-circuit, so no branch splits the group;
-            // a band is [lo, hi] around a bound: below hi and not below lo
-            const bool valid = (j < end) & (j != i);
-            const bool list_lo = r2f < pb.lo_list, list_hi = r2f <= pb.hi_list;
-            const bool near_lo = r2f < pb.lo_near, near_hi = r2f <= pb.hi_near;
-            band[q] = valid & ((list_hi & !list_lo) | (near_hi & !near_lo));
-            in[q] = valid & list_lo;
-            near[q] = valid & near_lo;
-            any_band |= band[q];
-          }
-          if (any_band) {
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-              if (band[q]) {
-                const double r2 = exact_r2(j0 + q);
-                in[q] = r2 < r_list_sq;
-                near[q] = r2 < near_sq;
-              }
-            }
-          }
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            if (in[q]) {
-              if (!kCount && nn + nf < cap) {
-                if (near[q])
-                  slot(nn++) = j0 + q;
-                else
-                  slot(cap - 1 - nf++) = j0 + q;
-              }
-              ++count;
-            }
-          }
-        }
-        continue;
-      }
-      // candidates in groups of four: the group's coordinates are loaded
-      // together, then tested and appended in index order
-      for (int j0 = start; j0 < end; j0 += 4) {
-        double px[4], py[4], pz[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          // an FP64 record holds the position itself
-          const typename Mir::T m = static_cast<const typename Mir::T*>(a.M)[min(j0 + q, end - 1)];
-          px[q] = m.x;
-          py[q] = m.y;
-          pz[q] = m.z;
-        }
-        double r2q[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          double ddx = px[q] - xi, ddy = py[q] - yi, ddz = pz[q] - zi;
-          if constexpr (kImg) {
-            ddx = ix ? ddx + sx : ddx;
-            ddy = iy ? ddy + sy : ddy;
-            ddz = iz ? ddz + sz : ddz;
-          } else {
-            ddx = min_image(ddx, mp.L[0], mp.hL[0], mp.periodic[0]);
-            ddy = min_image(ddy, mp.L[1], mp.hL[1], mp.periodic[1]);
-            ddz = min_image(ddz, mp.L[2], mp.hL[2], mp.periodic[2]);
-          }
-          r2q[q] = r2_unfused(ddx, ddy, ddz);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int j = j0 + q;
-          if (j < end && j != i && r2q[q] < r_list_sq) {
-            if (!kCount && nn + nf < cap) {
-              if (r2q[q] < near_sq)
-                slot(nn++) = j;
-              else
-                slot(cap - 1 - nf++) = j;
-            }
-            ++count;
-          }
-        }
-      }
-    }
-  };
-  bool images;
-  if constexpr (Mir::kMB)
-    images = a.boxes[a.rep[i]].images != 0;
-  else
-    images = g.images != 0;
-  // (pb.iso is false unless the records are fixed-point)
-  if (images) {
-    if (pb.iso)
-      search(std::true_type{}, std::true_type{});
-    else
-      search(std::true_type{}, std::false_type{});
-  } else {
-    if (pb.iso)
-      search(std::false_type{}, std::true_type{});
-    else
-      search(std::false_type{}, std::false_type{});
-  }
-  if (!kCount) {
-    // Shell entries sit at [cap - nf, cap); the gap [nn, cap - nf) has
-    // room for the m that must move (the rest already lie in [nn, nn+nf)).
-    const int gap = cap - nn - nf;
-    const int m = nf < gap ? nf : gap;
-    for (int q = 0; q < m; ++q) slot(nn + q) = slot(cap - 1 - q);
-    const int n = nn + nf;  // == min(count, cap)
-    cnt[i] = n;
-    a.cntn[i] = nn;
-    // Pad the row to a multiple of 8 with the atom itself, so unrolled
-    // readers can load whole groups of slots (cap is a multiple of 8).
-    for (int k = n; k < ((n + 7) & ~7); ++k) slot(k) = i;
-  }
-  return count;
-}
-
-// nlist_atom with 32 lanes per atom (two atoms per wavefront), for systems
-// too small to fill the chip one lane per atom. Lane t < 27 of a group loads
+// shell. Candidates are taken cell by cell in increasing rank, so both parts
+// come out in increasing atom index. A row over the capacity keeps its first
+// `cap` hits, and its true count is reported.
+//
+// nlist_atom_group: 32 lanes per atom, two atoms per wavefront, straight from
+// memory: for what nlist_cells leaves (below). Lane t < 27 of a group loads
 // stencil entry t's cell range and image, shared by shuffles; each cell's
 // candidates are then tested 32 at a time, and a hit's place in the row is
 // its rank among the hits in candidate order (ballot, then a prefix count):
-// hit k is kept when k < cap, near entries go to the front and shell entry
-// q to cap - 1 - q, as in nlist_atom. After a workgroup-scope fence (this
-// wave's row stores complete before it reads them back) the shell block is
-// moved behind the near block and the row padded, as nlist_atom does.
-// Distance arithmetic is nlist_atom's, so the row is bit for bit the same.
+// near entries go to the front and shell entries to the back; after a
+// workgroup-scope fence (this wave's row stores complete before it reads them
+// back) the shell block is moved behind the near block and the row padded.
 // Every lane of the wave runs the loop (the ballots and shuffles need
 // them); `act` is false for a half with no atom, whose i is any valid atom.
 template <bool kCount, class Mir>
@@ -1272,7 +1073,7 @@ __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArg
       };
       bool in_list, in_near;
       if constexpr (Mir::kFixed) {
-        // the record prefilter of nlist_atom, the exact test in its band
+        // the record prefilter, the exact test in its band
         const float r2f = pb.iso ? pre_r2<true>(static_cast<const int4*>(a.M)[jj], mi_rec, pb)
                                  : pre_r2<false>(static_cast<const int4*>(a.M)[jj], mi_rec, pb);
         if ((r2f >= pb.lo_list && r2f <= pb.hi_list) ||
@@ -1331,6 +1132,406 @@ __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArg
   return act ? count : 0;
 }
 
+// The rows of all cells, dealt to teams of wavefronts: the whole 1024-thread
+// workgroup, or halves or quarters of it where there are more cells than
+// workgroups. A team stages its cell's candidates -- the atoms of the 27
+// stencil cells, in rank order -- in LDS once: FP32 offsets from the cell's
+// centre, from the wrapping difference of the fixed-point records or from the
+// FP64 position with the stencil entry's image. Then, in three steps:
+//
+// 1. r^2 of all home atoms against all candidates on the matrix cores, 16 x 16
+//    at a time, as |a|^2 - 2 a.b + |b|^2 with r_list^2 taken off the
+//    accumulator's start: a sign bit is a hit, and a lane collects 16
+//    candidates' signs, for either radius, into masks. A pair closer to a
+//    radius than the FP32 error takes the exact test (loads of the positions,
+//    which the whole workgroup waits for: a wider band costs time). That error,
+//    with S = 2 |a| + r_list >= |a| + |b| near a radius: the offsets' rounding,
+//    2^-22 r_list S; the squares', products' and sum's, 6.5 2^-24 S^2; and a
+//    unit of the records on each axis, 3.5 r_list units.
+// 2. Half a wavefront turns a row's masks into the list of its candidates, near
+//    ones first: a popcount prefix over the words, then each lane its own bits.
+// 3. It writes the row, one quad of slots a lane.
+//
+// Boxes where the offsets' image could differ from the minimum image (under
+// three cells of r_list on a periodic axis) take r^2 from the records'
+// wrapping differences in step 1 (fixed point). nlist_atom_group takes such
+// boxes with FP64 records, cells whose stencil or masks do not fit, and rows
+// over the capacity.
+//
+// A round of cells (18-32 atoms, 500-860 candidates each) costs about 2.5 us of
+// load latency for the tables and candidates, 3-6 us in the masks and 3-6 us in
+// the rows, both of them VALU issue. List phase of a rebuild, us, against 32
+// lanes an atom (up to 131,072 atoms) or one straight from memory: 256 EAM atoms
+// 17.5 -> 10.8, 4,000 Morse 21 -> 16, 32,000 EAM 64 -> 41, 32,000 Morse in FP64
+// 80 -> 32, 256,000 EAM in FP64 232 -> 195, 1,048,576 EAM 776 -> 764.
+constexpr int kListBlock = 1024;
+constexpr int kListCand = 4096;   // candidates staged by a workgroup
+constexpr int kListMask = 8192;   // mask words (32 candidates) of a workgroup
+constexpr int kListRow = 1024;    // entries of a row in LDS
+constexpr float kSumError = 6.5e-7f;
+
+struct ListLds {
+  union {
+    float rel[4 * (kListCand + 16)];  // per team: x, y, z, |.|^2 of tcand + 4 each
+    uint16_t row[kListBlock / 32][kListRow];
+  };
+  int32_t idx[kListCand];
+  uint32_t in[kListMask];
+  uint32_t near[kListMask];
+  int32_t start[2][4][27];  // two rounds' tables
+  int32_t end[2][4][27];    // run t of team w: candidates [end[w][t - 1], end[w][t])
+  uint8_t img[2][4][28];
+  int32_t home[2][4][2];  // the cell's first atom and atom count
+};
+
+// Inclusive sum over the 32 lanes of a wavefront's half.
+__device__ __forceinline__ int half_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, true);  // row_bcast:15
+  return v;
+}
+
+// Returns the largest count this lane's rows had.
+template <bool kCount, class Mir>
+__device__ __forceinline__ int nlist_cells(const StepArgs& a, const GridArgs& g, const PermArgs& p,
+                                           double r_list_sq, double near_sq, int32_t* nbr,
+                                           int32_t* cnt, ListLds& L) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int kWaves = kListBlock / 64;
+  const int lane = static_cast<int>(threadIdx.x & 63);
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int grid = static_cast<int>(gridDim.x);
+  const int tsh = g.ncells > 2 * grid ? 2 : g.ncells > grid ? 1 : 0;
+  const int teams = 1 << tsh;
+  const int tw = kWaves >> tsh;                           // wavefronts of a team
+  const int team = w >> (4 - tsh), wt = w & (tw - 1);     // this one's team and place in it
+  const int tcand = kListCand >> tsh;
+  const int cs4 = tcand + 4;  // a component's stride: four in different LDS banks
+  float* const rel = L.rel + team * 4 * cs4;
+  int32_t* const idx = L.idx + team * tcand;
+  uint32_t* const m_in = L.in + team * (kListMask >> tsh);
+  uint32_t* const m_near = L.near + team * (kListMask >> tsh);
+  const int cap = a.cap;
+  const float rl2 = static_cast<float>(r_list_sq);
+  const float gap = static_cast<float>(r_list_sq - near_sq);
+  const float rl = sqrtf(rl2);
+  const float pre = static_cast<float>(r_list_sq * kPreMargin);
+  int most = 0;
+  // groups of `teams` consecutive cells, dealt so that an XCD's are consecutive
+  const int ngroups = (g.ncells + teams - 1) >> tsh;
+  const int xcds = grid >= 8 ? 8 : 1;
+  const int per = (ngroups + xcds - 1) / xcds;
+  const int x = static_cast<int>(blockIdx.x) % xcds;
+  const int step = (grid - x + xcds - 1) / xcds;  // workgroups that share these groups
+  // the stencil's runs of this team's cell in group m0, by one wavefront
+  auto table = [&](int m0, int buf) {
+    const int c = ((x * per + m0) << tsh) + team;
+    const bool in_grid = m0 < per && x * per + m0 < ngroups && c < g.ncells;
+    int n = 0;
+    if (in_grid && lane < 27) {
+      const int r = g.around[27 * static_cast<size_t>(c) + lane];
+      const int s = g.cstart[r];
+      n = g.cstart[r + 1] - s;
+      L.start[buf][team][lane] = s;
+      L.img[buf][team][lane] = g.around_img[27 * static_cast<size_t>(c) + lane];
+      if (r == c) {
+        L.home[buf][team][0] = s;
+        L.home[buf][team][1] = n;
+      }
+    }
+    if (!in_grid && lane == 0) L.home[buf][team][1] = 0;
+    n = half_scan(n);
+    if (lane < 27) L.end[buf][team][lane] = n;
+  };
+  if (wt == 0) table(static_cast<int>(blockIdx.x) / xcds, 0);
+  int buf = 0;
+  for (int m0 = static_cast<int>(blockIdx.x) / xcds; m0 < per; m0 += step, buf ^= 1) {
+    __syncthreads();  // the table stands, the LDS of the previous cells is done with
+    const int nh = __builtin_amdgcn_readfirstlane(L.home[buf][team][1]);
+    const int h0 = nh > 0 ? __builtin_amdgcn_readfirstlane(L.home[buf][team][0]) : 0;
+    const int m = nh > 0 ? __builtin_amdgcn_readfirstlane(L.end[buf][team][26]) : 0;
+    const int nch = (m + 63) >> 6;
+    const MirrorParams& mp = mp_of<Mir>(a, h0);
+    bool images = false, flat = false;  // flat: offsets carry the image
+    double ctr[3] = {0.0, 0.0, 0.0};
+    int ref[3] = {0, 0, 0};  // the centre as a record
+    float u[3] = {0.0f, 0.0f, 0.0f}, unit_err = 0.0f;
+    auto shift = [&](int img, int d) {
+      const int s = (img >> (2 * d)) & 3;
+      return s == 0 ? 0.0 : s == 1 ? mp.L[d] : -mp.L[d];
+    };
+    if (nh > 0) {
+      if constexpr (Mir::kMB)
+        images = a.boxes[a.rep[h0]].images != 0;
+      else
+        images = g.images != 0;
+      flat = images;
+      const CellGrid cg = grid_of<Mir>(a, g, h0);
+      const double at[3] = {p.px[h0], p.py[h0], p.pz[h0]};
+      int cc[3];
+      cell_coords(cg, at[0], at[1], at[2], cc);
+      for (int d = 0; d < 3; ++d) {
+        const double cs = 1.0 / cg.inv_cs[d];
+        ctr[d] = cg.lo[d] + (cc[d] + 0.5) * cs;
+        if constexpr (Mir::kFixed) {
+          // half a cell and r_list stay within half the box
+          flat = flat && (!mp.periodic[d] || cs * cs >= r_list_sq * 1.00001);
+          u[d] = static_cast<float>(mp.unit[d]);
+          unit_err = fmaxf(unit_err, 4.0f * rl * u[d]);
+          const double o = (ctr[d] - at[d]) / mp.unit[d];
+          const int4 r0 = static_cast<const int4*>(a.M)[h0];
+          ref[d] = static_cast<int>(static_cast<unsigned>(d == 0 ? r0.x : d == 1 ? r0.y : r0.z) +
+                                    static_cast<unsigned>(static_cast<int>(
+                                        fmin(fmax(o, -2147483647.0), 2147483647.0))));
+        } else {
+          // FP64 itself resolves 1e-7 r_list there
+          flat = flat && (fabs(ctr[d]) + mp.L[d]) * (fabs(ctr[d]) + mp.L[d]) < 1e16 * r_list_sq;
+        }
+      }
+    }
+    const bool staged =
+        m <= tcand && nh * nch * 2 <= (kListMask >> tsh) && (Mir::kFixed || flat);
+    // the run that candidate q lies in: the first that ends beyond it
+    auto run_of = [&](int q) {
+      int t = 0;
+#pragma unroll
+      for (int s = 16; s > 0; s >>= 1)
+        if (t + s <= 26 && L.end[buf][team][t + s - 1] <= q) t += s;
+      return t;
+    };
+    if (staged) {
+      for (int q = wt * 64 + lane; q < m; q += tw * 64) {
+        const int t = run_of(q);
+        const int j = L.start[buf][team][t] + (q - (t > 0 ? L.end[buf][team][t - 1] : 0));
+        const typename Mir::T v = static_cast<const typename Mir::T*>(a.M)[j];
+        idx[q] = j;
+        float o[3];
+        if constexpr (Mir::kFixed) {
+          if (flat) {
+            o[0] = static_cast<float>(MirrorFixed::wdiff(v.x, ref[0])) * u[0];
+            o[1] = static_cast<float>(MirrorFixed::wdiff(v.y, ref[1])) * u[1];
+            o[2] = static_cast<float>(MirrorFixed::wdiff(v.z, ref[2])) * u[2];
+          } else {
+            o[0] = __int_as_float(v.x);
+            o[1] = __int_as_float(v.y);
+            o[2] = __int_as_float(v.z);
+          }
+        } else {
+          const int img = L.img[buf][team][t];
+          o[0] = static_cast<float>(v.x + shift(img, 0) - ctr[0]);
+          o[1] = static_cast<float>(v.y + shift(img, 1) - ctr[1]);
+          o[2] = static_cast<float>(v.z + shift(img, 2) - ctr[2]);
+        }
+        float n2 = o[0] * o[0] + o[1] * o[1] + o[2] * o[2];
+        if (!Mir::kFixed && !(n2 < 1e30f)) {  // far out or not finite: no hit, or asked for
+          o[0] = o[1] = o[2] = 0.0f;
+          n2 = __builtin_huge_valf();
+        }
+        rel[q] = o[0];
+        rel[cs4 + q] = o[1];
+        rel[2 * cs4 + q] = o[2];
+        rel[3 * cs4 + q] = n2;
+      }
+    }
+    __syncthreads();
+    if (wt == tw - 1) table(m0 + step, buf ^ 1);
+    if (staged && nh > 0) {
+      // the first candidate of the home cell's own run: there an atom meets itself
+      int lo = 0;
+      bool own = false;
+      if (lane < 27) {
+        lo = lane > 0 ? L.end[buf][team][lane - 1] : 0;
+        own = L.start[buf][team][lane] == h0 && L.end[buf][team][lane] > lo;
+      }
+      const unsigned long long home = __builtin_amdgcn_ballot_w64(own);
+      const int self0 = __builtin_amdgcn_readlane(lo, home != 0 ? __builtin_ctzll(home) : 0);
+      // lane (piece s of the chunk, home atom b + col): bit e of its piece is
+      // candidate 64 ch + 16 s + e
+      const int col = lane & 15, s = lane >> 4;
+      for (int b = 0; b < nh; b += 16) {
+        const int h = self0 + min(b + col, nh - 1);
+        float width = pre, bv = 0.0f;
+        f32x4 c_list{};
+        if (!Mir::kFixed || flat) {
+          const float a2 = rel[3 * cs4 + h];
+          const float span = 2.0f * sqrtf(a2) + rl;
+          width = kSumError * span * span + unit_err;
+          bv = s < 3 ? -2.0f * rel[s * cs4 + h] : 1.0f;
+          c_list = f32x4{1.0f, 1.0f, 1.0f, 1.0f} * (a2 - rl2);
+        }
+        for (int ch = wt; ch < nch; ch += tw) {
+          const int q0 = 64 * ch + 16 * s;
+          unsigned in = 0, near = 0;
+          float v[16], f[16];  // r^2 - r_list^2, r^2 - r_near^2 of the piece
+          if (!Mir::kFixed || flat) {
+            // rows 4 s + e of product t: candidates 64 ch + 16 s + 4 t + e
+            const float* const from = rel + s * cs4 + 64 * ch + 16 * (col >> 2) + (col & 3);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              const f32x4 r = __builtin_amdgcn_mfma_f32_16x16x4f32(from[4 * t], bv, c_list, 0, 0, 0);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                v[4 * t + e] = r[e];
+                f[4 * t + e] = r[e] + gap;
+              }
+            }
+          } else {
+            const int ax = __float_as_int(rel[h]), ay = __float_as_int(rel[cs4 + h]),
+                      az = __float_as_int(rel[2 * cs4 + h]);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+              const float dx =
+                  u[0] * static_cast<float>(MirrorFixed::wdiff(__float_as_int(rel[q0 + e]), ax));
+              const float dy = u[1] * static_cast<float>(
+                                          MirrorFixed::wdiff(__float_as_int(rel[cs4 + q0 + e]), ay));
+              const float dz = u[2] * static_cast<float>(MirrorFixed::wdiff(
+                                          __float_as_int(rel[2 * cs4 + q0 + e]), az));
+              const float r2 = dx * dx + dy * dy + dz * dz;
+              v[e] = r2 - rl2;
+              f[e] = v[e] + gap;
+            }
+          }
+          float closest = __builtin_huge_valf();
+#pragma unroll
+          for (int e = 15; e >= 0; --e) {
+            in = __builtin_amdgcn_alignbit(in, __float_as_uint(v[e]), 31);
+            near = __builtin_amdgcn_alignbit(near, __float_as_uint(f[e]), 31);
+            closest = fminf(fminf(fabsf(v[e]), fabsf(f[e])), closest);
+          }
+          unsigned valid = 0xffffu;
+          if (ch == nch - 1) {
+            const int left = m - q0;
+            valid = left >= 16 ? 0xffffu : left > 0 ? (1u << left) - 1u : 0u;
+          }
+          if (self0 + b < 64 * ch + 64 && self0 + b + 16 > 64 * ch) {
+            const int self = h - q0;
+            if (self >= 0 && self < 16) valid &= ~(1u << self);
+          }
+          if (!(closest > width) && valid != 0) {
+            unsigned ask = 0;
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+              if (!(fabsf(v[e]) > width && fabsf(f[e]) > width)) ask |= 1u << e;
+            const int i = h0 + h - self0;
+            for (ask &= valid; ask != 0; ask &= ask - 1) {
+              const int e = __builtin_ctz(ask);
+              const int j = idx[q0 + e];
+              const int img = L.img[buf][team][run_of(q0 + e)];
+              double dx, dy, dz;
+              if constexpr (Mir::kFixed) {
+                dx = p.px[j] - p.px[i];
+                dy = p.py[j] - p.py[i];
+                dz = p.pz[j] - p.pz[i];
+              } else {  // an FP64 record holds the position itself
+                const typename Mir::T rj = static_cast<const typename Mir::T*>(a.M)[j];
+                const typename Mir::T ri = static_cast<const typename Mir::T*>(a.M)[i];
+                dx = rj.x - ri.x;
+                dy = rj.y - ri.y;
+                dz = rj.z - ri.z;
+              }
+              if (images) {
+                dx = (img & 3) ? dx + shift(img, 0) : dx;
+                dy = ((img >> 2) & 3) ? dy + shift(img, 1) : dy;
+                dz = ((img >> 4) & 3) ? dz + shift(img, 2) : dz;
+              } else {
+                dx = min_image(dx, mp.L[0], mp.hL[0], mp.periodic[0]);
+                dy = min_image(dy, mp.L[1], mp.hL[1], mp.periodic[1]);
+                dz = min_image(dz, mp.L[2], mp.hL[2], mp.periodic[2]);
+              }
+              const double r2 = r2_unfused(dx, dy, dz);
+              in = (in & ~(1u << e)) | ((r2 < r_list_sq ? 1u : 0u) << e);
+              near = (near & ~(1u << e)) | ((r2 < near_sq ? 1u : 0u) << e);
+            }
+          }
+          if (b + col < nh) {
+            const int o = ((b + col) * nch + ch) * 4 + s;
+            reinterpret_cast<uint16_t*>(m_in)[o] = static_cast<uint16_t>(in & valid);
+            reinterpret_cast<uint16_t*>(m_near)[o] = static_cast<uint16_t>(in & near & valid);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    // rows, one to a half wavefront
+    const int hl = lane & 31;
+    uint16_t* const list = L.row[2 * w + (lane >> 5)];
+    for (int b = 2 * wt; b < nh; b += 2 * tw) {
+      const int h = b + (lane >> 5);
+      const bool act = h < nh;
+      const int i = h0 + (act ? h : b);
+      int n = 0, nn = 0;
+      bool slow = !staged;
+      if (staged) {
+        const uint32_t* const in = m_in + (act ? h : b) * nch * 2;
+        const uint32_t* const near = m_near + (act ? h : b) * nch * 2;
+        int sum = 0;  // in | near << 16: a row has at most kListCand
+        for (int q = hl; q < 2 * nch; q += 32) sum += __popc(in[q]) | (__popc(near[q]) << 16);
+        sum = __shfl(half_scan(sum), lane | 31);
+        n = sum & 0xffff;
+        nn = sum >> 16;
+        if constexpr (kCount) {
+          if (act) most = max(most, n);
+          continue;
+        }
+        slow = __any(act && n > min(cap, kListRow));
+      }
+      if (slow) {
+        const int got =
+            nlist_atom_group<kCount, Mir>(a, g, p, i, act, r_list_sq, near_sq, nbr, cnt);
+        if (act) most = max(most, got);
+        continue;
+      }
+      if constexpr (!kCount) {
+        const uint32_t* const in = m_in + (act ? h : b) * nch * 2;
+        const uint32_t* const near = m_near + (act ? h : b) * nch * 2;
+        int base = 0;
+        for (int q0 = 0; q0 < 2 * nch; q0 += 32) {
+          const int q = q0 + hl;
+          const uint32_t bits = q < 2 * nch ? in[q] : 0u;
+          const uint32_t nb = q < 2 * nch ? near[q] : 0u;
+          const int own = __popc(bits) | (__popc(nb) << 16);
+          const int incl = base + half_scan(own);
+          const int before = incl - own;
+          base = __shfl(incl, lane | 31);
+          const int before_near = before >> 16;
+          uint16_t* to = list + before_near;
+          for (uint32_t left = nb; left != 0; left &= left - 1)
+            *to++ = static_cast<uint16_t>(32 * q + __builtin_ctz(left));
+          to = list + nn + (before & 0xffff) - before_near;
+          for (uint32_t left = bits ^ nb; left != 0; left &= left - 1)
+            *to++ = static_cast<uint16_t>(32 * q + __builtin_ctz(left));
+        }
+        // the wave's own LDS stores, read by its other lanes
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (act) {
+          // padded to a multiple of 8 with the atom itself, so unrolled readers
+          // can load whole groups of slots (cap is a multiple of 8)
+          int32_t* const row = nbr + ell(i, 0, cap);
+          for (int q = hl; q < 2 * ((n + 7) >> 3); q += 32) {
+            int4 v;
+            v.x = 4 * q < n ? idx[list[4 * q]] : i;
+            v.y = 4 * q + 1 < n ? idx[list[4 * q + 1]] : i;
+            v.z = 4 * q + 2 < n ? idx[list[4 * q + 2]] : i;
+            v.w = 4 * q + 3 < n ? idx[list[4 * q + 3]] : i;
+            *reinterpret_cast<int4*>(row + 256 * q) = v;
+          }
+          if (hl == 0) {
+            cnt[i] = n;
+            a.cntn[i] = nn;
+          }
+          most = max(most, n);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      }
+    }
+  }
+  return most;
+}
+
 // Largest row count of the wave: recorded for sizing (kCount) or flagged as
 // an overflow of the capacity.
 template <bool kCount>
@@ -1385,24 +1586,13 @@ __global__ void __launch_bounds__(kBlock) k_copyback(StepArgs a, GridArgs g, Per
   copyback_atom<R, Mir>(a, g, t, s);
 }
 
-// kSplit: two atoms per wavefront (nlist_atom_group).
-template <bool kCount, bool kSplit, class Mir>
-__global__ void __launch_bounds__(kBlock)
+template <bool kCount, class Mir>
+__global__ void __launch_bounds__(kListBlock)
 k_nlist_ell(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double near_sq, int32_t* nbr,
             int32_t* cnt, int32_t* maxcnt) {
   if (!kCount && !a.flags[0]) return;
-  const int gi = blockIdx.x * kBlock + threadIdx.x;
-  int count = 0;
-  if constexpr (kSplit) {
-    const int i = gi >> 5, base = (gi >> 6) * 2;
-    if (base < a.natoms) {
-      const bool act = i < a.natoms;
-      count = nlist_atom_group<kCount, Mir>(a, g, t, act ? i : base, act, r_list_sq, near_sq, nbr,
-                                            cnt);
-    }
-  } else if (gi < a.natoms) {
-    count = nlist_atom<kCount, Mir>(a, g, t, gi, r_list_sq, near_sq, nbr, cnt);
-  }
+  __shared__ ListLds L;
+  const int count = nlist_cells<kCount, Mir>(a, g, t, r_list_sq, near_sq, nbr, cnt, L);
   report_count<kCount>(a, count, maxcnt);
 }
 
@@ -1771,11 +1961,7 @@ __device__ __forceinline__ bool grid_barrier(GridBarrier* b, unsigned int* passe
 
 constexpr int kRebuildBlock = 1024;  // workgroup of the fused rebuild
 
-// Registers are not capped: the list search's candidate groups need more
-// than the 64 VGPRs that eight waves per SIMD (two workgroups per CU) would
-// leave, and spilled under that cap (1M-atom rebuild 2.14 ms capped, 2.10
-// uncapped; 0.67 / 0.58 ms at 256,000 atoms). The grid is as many
-// workgroups as the device holds at once (one or two per CU).
+// The grid is at most as many workgroups as the device holds at once.
 template <class R, class Mir>
 __global__ void __launch_bounds__(kRebuildBlock)
 k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double near_sq,
@@ -1785,13 +1971,18 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
   const int tid = blockIdx.x * kRebuildBlock + threadIdx.x;
   const int nthr = gridDim.x * kRebuildBlock;
   const int N = a.natoms;
+  __shared__ union {  // one phase's at a time, a grid barrier between them
+    int32_t cstart[kScanOwn + 1];
+    ListLds list;
+    HaloLds halo;
+  } lds;
   unsigned int passed = bar->gen;  // written below once every workgroup has read it
   // (the cell counters are clear: the phase that last reads them clears them)
   for (int i = tid; i < N; i += nthr) bin_atom<Mir>(a, g, i);
   if (!grid_barrier(bar, &passed, a.flags)) return;
   if (g.ncells <= kScanOwn) {
     // few cells: every workgroup scans them for itself, without a barrier
-    __shared__ int32_t cstart[kScanOwn + 1];
+    int32_t* const cstart = lds.cstart;
     scan_cells<kRebuildBlock>(g, cstart);
     __syncthreads();
     if (blockIdx.x == 0)
@@ -1820,30 +2011,13 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
   // the state's arrays back from the scratch ones, beside the list search,
   // which reads the scratch arrays and the records
   for (int s = tid; s < N; s += nthr) copyback_atom<R, Mir>(a, g, t, s);
-  int count = 0;
-  if (g.nl_split) {
-    // two atoms per wavefront, 32 lanes each; the loop bound is uniform per wave
-    const int gw = tid >> 6, nw = nthr >> 6;
-    for (int base = 2 * gw; base < N; base += 2 * nw) {
-      const int i = base + static_cast<int>((threadIdx.x >> 5) & 1);
-      const bool act = i < N;
-      const int c = nlist_atom_group<false, Mir>(a, g, t, act ? i : base, act, r_list_sq, near_sq,
-                                                 nbr, cnt);
-      count = c > count ? c : count;
-    }
-  } else {
-    for (int i = tid; i < N; i += nthr) {
-      const int c = nlist_atom<false, Mir>(a, g, t, i, r_list_sq, near_sq, nbr, cnt);
-      count = c > count ? c : count;
-    }
-  }
+  const int count = nlist_cells<false, Mir>(a, g, t, r_list_sq, near_sq, nbr, cnt, lds.list);
   report_count<false>(a, count, nullptr);
   if constexpr (Mir::kFixed) {
     if (a.stage_cap > 0) {  // halos of the staged passes, from the new rows
-      __shared__ HaloLds L;
       if (!grid_barrier(bar, &passed, a.flags)) return;
       static_assert(kRebuildBlock == kHaloBlock, "halos are built by whole workgroups");
-      build_halos(a, (N + kHaloBlock - 1) / kHaloBlock, L);
+      build_halos(a, (N + kHaloBlock - 1) / kHaloBlock, lds.halo);
     }
   }
   // every thread read the flag at entry, before the first barrier

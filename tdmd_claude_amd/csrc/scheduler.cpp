@@ -79,11 +79,9 @@ int sched_alloc(tdmd_sched* S) {
   if (static_cast<uint64_t>(N) * msz >= (uint64_t{1} << 32))
     return fail(TDMD_E_INVALID, "scheduler: at most " + std::to_string((uint64_t{1} << 32) / msz - 1) +
                                     " atoms in one scheduler at this precision");
-  // kRecPad spare records past the last atom: the list search reads its
-  // candidates in whole groups of eight from the first of a cell's atoms
   char *M, *M2;
-  if ((rc = dalloc(S, &M, (static_cast<size_t>(N) + sched::kRecPad) * msz))) return rc;
-  if ((rc = dalloc(S, &M2, (static_cast<size_t>(N) + sched::kRecPad) * msz))) return rc;
+  if ((rc = dalloc(S, &M, N * msz))) return rc;
+  if ((rc = dalloc(S, &M2, N * msz))) return rc;
   a.M = M;
   a.M2 = M2;
   if ((rc = dalloc(S, &a.flags, 8))) return rc;

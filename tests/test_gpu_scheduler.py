@@ -616,3 +616,73 @@ def test_list_counts_match_oracle_at_the_cutoffs(mirror_fp64, lz):
         assert round(obs["mean_neighbors"] * s.natoms) == n_full
         assert round(obs["mean_near_neighbors"] * s.natoms) == 2 * int(np.sum(near))
     sched.close()
+
+
+def _brute_counts(pos, L, periodic, radii):
+    out = [np.zeros(len(pos), dtype=np.int64) for _ in radii]
+    for i in range(0, len(pos), 256):
+        r2 = 0.0
+        for d in range(3):
+            x = pos[None, :, d] - pos[i:i + 256, None, d]
+            if periodic[d]:
+                x = np.where(x > 0.5 * L[d], x - L[d], np.where(x < -0.5 * L[d], x + L[d], x))
+            r2 = r2 + x * x
+        for o, r in zip(out, radii):
+            o[i:i + 256] = (r2 < r * r).sum(1) - 1
+    return out
+
+
+# name: atoms, box edges, periodic axes
+LIST_CASES = {
+    "narrow cells": (200, (16.0, 17.0, 18.0), (1, 1, 1)),  # three under r_list on each axis
+    "r_list cells": (300, (21.0 + 1e-6,) * 3, (1, 1, 1)),  # three, r_list wide
+    "wide cells": (900, (27.5, 24.0, 23.0), (1, 1, 1)),  # three, up to 1.3 r_list
+    "full rows": (2000, (22.0, 22.0, 22.0), (1, 1, 1)),
+    "full cells": (5000, (24.0, 24.0, 24.0), (1, 1, 1)),  # over the staged candidates
+    "two teams": (9000, (60.0, 57.0, 43.0), (1, 1, 1)),  # 384 cells
+    "four teams": (9000, (80.0, 72.0, 80.0), (1, 1, 1)),  # 1210 cells
+    "open axes": (1500, (30.0, 40.0, 50.0), (0, 1, 0)),
+    "sparse": (40, (90.0, 90.0, 90.0), (1, 1, 1)),
+}
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+@pytest.mark.parametrize("name", LIST_CASES)
+def test_list_counts_by_kind_of_cell(name, prec):
+    # Counts of the lists at the first build and after a fused rebuild against
+    # all pairs in FP64, with pairs planted around both radii (inside and outside
+    # the error of the FP32 sum) and, on open axes, atoms outside the box. The
+    # rows of an atom are exact: no tolerance.
+    rng = np.random.Generator(np.random.PCG64(23))
+    n, L, periodic = LIST_CASES[name]
+    L = np.array(L)
+    rc, skin = 6.0, 1.0
+    pos = rng.uniform(0.0, L, size=(n, 3))
+    for d in range(3):
+        if not periodic[d]:
+            pos[: n // 8, d] += rng.uniform(-0.3, 0.3, size=n // 8) * L[d]
+    extra = []
+    for r in (rc, rc + skin):
+        for e in (1e-9, 1e-7, 1e-6, 1e-5):
+            for sgn in (-1, 1):
+                p = rng.uniform(0.0, L, size=3)
+                u = rng.normal(size=3)
+                q = p + r * (1 + sgn * e) * u / np.linalg.norm(u)
+                extra += [p, np.where(periodic, np.mod(q, L), q)]
+    pos = np.concatenate([pos, np.array(extra)])
+    n = len(pos)
+    say("list counts,", name, prec, n)
+    s = I.System(lo=np.zeros(3), hi=L.copy(), pos=pos, vel=np.zeros_like(pos),
+                 types=np.ones(n, dtype=np.int32), ids=np.arange(1, n + 1, dtype=np.int32),
+                 masses=np.array([1.0, 63.546]), periodic=periodic)
+    sched = FastPipelineScheduler.for_system(
+        s, (1e-9, 1.0, 2.8, rc), FastPipelineConfig(precision=prec, rebuild_every=1, r_skin=skin,
+                                                    dt=1e-9))
+    for step in (0, 1):
+        sched.run_until(step)
+        full, near = _brute_counts(sched.download()[0], L, periodic, (rc + skin, rc))
+        obs = sched.observables()
+        assert round(obs["mean_neighbors"] * n) == full.sum()
+        assert round(obs["mean_near_neighbors"] * n) == near.sum()
+        assert round(sched.thermo()["max_nbr"]) == full.max()
+    sched.close()
