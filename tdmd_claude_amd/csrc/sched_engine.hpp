@@ -8,8 +8,11 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <numeric>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include <hip/hip_ext.h>
@@ -107,6 +110,9 @@ struct tdmd_sched {
   int32_t* d_maxcnt = nullptr;
   int64_t* d_rebuilds = nullptr;
   double* d_scalars = nullptr;
+  mutable double* h_stage = nullptr;  // pinned, from the first download on
+  mutable hipEvent_t ev_stage[4] = {};
+  mutable std::mutex download_mu;  // the staging buffer's and the scratch block's
   std::vector<int32_t> h_types, h_ids;
   std::vector<double> h_masses;
   bool uploaded = false, initial_forces = false;

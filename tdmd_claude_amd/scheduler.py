@@ -139,11 +139,11 @@ class FastPipelineScheduler:
 
     def download(self):
         n = self.natoms
-        pos = np.zeros((n, 3))
-        vel = np.zeros((n, 3))
-        f = np.zeros((n, 3))
-        types = np.zeros(n, dtype=np.int32)
-        ids = np.zeros(n, dtype=np.int32)
+        pos = np.empty((n, 3))
+        vel = np.empty((n, 3))
+        f = np.empty((n, 3))
+        types = np.empty(n, dtype=np.int32)
+        ids = np.empty(n, dtype=np.int32)
         capi.call("tdmd_sched_download", self._h, _pd(pos), _pd(vel), _pd(f), _pi(types),
                   _pi(ids), n)
         return pos, vel, f, types, ids

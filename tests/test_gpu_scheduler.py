@@ -6,6 +6,8 @@ the GPU runs the scheduler with its fused cross-step kick. In FP64 the two
 agree to rounding over short runs; in mixed precision forces agree to 1e-5
 of the RMS force.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -685,4 +687,37 @@ def test_list_counts_by_kind_of_cell(name, prec):
         assert round(obs["mean_neighbors"] * n) == full.sum()
         assert round(obs["mean_near_neighbors"] * n) == near.sum()
         assert round(sched.thermo()["max_nbr"]) == full.max()
+    sched.close()
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+@pytest.mark.parametrize("n", [1, 7281, 7282, 116508, 116509, 262150])
+def test_download_by_size_and_wanted_arrays(n, prec):
+    # The ways a download takes by its size (one staged transfer, straight into
+    # the caller's arrays, staged by several threads), whole and for every choice
+    # of arrays: after the sort positions and velocities come back bit for bit in
+    # upload order, forces the same from each.
+    m = max(3, int(np.ceil(n ** (1 / 3))))
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    rng = np.random.Generator(np.random.PCG64(5))
+    pos = 4.0 * rng.permutation(g)[:n] + rng.uniform(0.5, 1.0, size=(n, 3))
+    L = np.full(3, max(4.0 * m, 20.0))
+    s = I.System(lo=np.zeros(3), hi=L, pos=pos, vel=rng.normal(size=(n, 3)),
+                 types=np.ones(n, dtype=np.int32), ids=np.arange(n, 0, -1).astype(np.int32),
+                 masses=np.array([1.0, 63.546]))
+    say("download", n, prec)
+    sched = FastPipelineScheduler.for_system(s, MORSE_CU[:3] + (5.0,),
+                                             FastPipelineConfig(precision=prec))
+    sched.run_until(0)
+    p, v, f, t, ids = sched.download()
+    assert np.array_equal(p, s.pos) and np.array_equal(v, s.vel)
+    assert np.array_equal(ids, s.ids) and np.isfinite(f).all()
+    assert n < 2 or np.abs(f).max() > 0
+    for want in range(8):
+        out = [np.full((n, 3), np.nan) for _ in range(3)]
+        args = [out[k].ctypes.data_as(C.POINTER(C.c_double)) if want >> k & 1 else None
+                for k in range(3)]
+        capi.call("tdmd_sched_download", sched._h, *args, None, None, n)
+        for k, ref in enumerate((p, v, f)):
+            assert np.array_equal(out[k], ref) if want >> k & 1 else np.isnan(out[k]).all()
     sched.close()
