@@ -312,8 +312,8 @@ typedef struct {
   int32_t disable_halo;   /* 1: no LDS halo staging in the single-element */
                           /* EAM passes (0: staged where records are 16 B)*/
   int32_t pair_lanes;     /* lanes per neighbour row in the force passes:  */
-                          /* 0 = by size (8 up to 131072 atoms for Morse, */
-                          /* 65536 for EAM, else 1),                      */
+                          /* 0 = by size (8 up to 40960 atoms, 4 up to    */
+                          /* about 100,000, else 1),                      */
                           /* 1, 4 or 8; EAM with more than one lane runs  */
                           /* the global-table passes (no LDS tables/halo) */
   int32_t cell_pct;       /* binning cells at least this percentage of     */

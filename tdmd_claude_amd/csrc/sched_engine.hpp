@@ -24,17 +24,33 @@ namespace tdmd_hip {
 
 using namespace sched;
 
-// Rows of small systems are split over kSplitLanes lanes in the force
-// passes (Morse, and EAM through the global-table passes): one lane per atom
-// would give 32,000 atoms 125 workgroups on 256 CUs, each lane walking ~80
-// slots in turn; the LDS EAM passes would run 32 workgroups. Thresholds from
-// the measured pass times (mixed, 8 lanes against one): Morse 32,000 atoms
-// 10.6 against 19.9 us, 108,000 26.3 against 28.9, 256,000 57.9 against
-// 51.1; EAM density + force 32,000 22.7 against 53.7 us (LDS passes),
-// 108,000 74.6 against 59.3.
-constexpr int kSplitLanes = 8;
-constexpr int kSplitMax = 131072;     // Morse
-constexpr int kEamSplitMax = 65536;   // EAM
+// Lanes per neighbour row in the force passes (Morse, and EAM through the
+// global-table passes). One lane per atom gives 32,000 atoms 125 workgroups on
+// 256 CUs, each lane walking ~80 slots in turn, and the time is flat up to a
+// wavefront per SIMD (65,536 atoms); eight lanes fill the chip at 8,000 atoms
+// and pay their shuffles and idle slots from about 40,000 on. Steps without a
+// rebuild, us with 1 / 4 / 8 lanes, mixed:
+//   EAM (1: LDS passes)        32,000: 57.6 / 30.7 / 28.2   62,500: 69.6 / 49.1 / 54.5
+//                              70,304: 59.7 / 60.1 / 62.5
+//   three elements, replicas   22,000: 59.8 / 32.4 / 28.6   80,000: 93.1 / 72.9 / 83.7
+//                              130,000: 98.7 / 117.0 / 122.8
+//   Morse                      23,328: 23.9 / 14.8 / 12.8   108,000: 39.5 / 38.4 / 40.2
+//                              131,072: 39.8 / 42.0 / 44.5
+// and in FP64:
+//   EAM                        32,000: 131.6 / 47.0 / 46.8  97,556: 139.4 / 129.8 / 132.4
+//                              131,072: 142.0 / 172.5 / 174.4
+//   three elements, replicas   80,000: 156.0 / 120.1 / 123.0  130,000: 158.0 / 174.6 / 184.0
+//   Morse                      62,500: 52.4 / 48.0 / 50.0   131,072: 67.5 / 66.1 / 72.6
+//                              186,624: 93.6 / 93.5 / 99.5
+constexpr int kSplitLanes = 8;  // the most
+constexpr int kSplit8Max = 40960;
+inline int lanes_by_size(int natoms, bool eam, int ntypes, bool fp64) {
+  if (natoms <= kSplit8Max) return kSplitLanes;
+  const int max4 = !eam         ? (fp64 ? 131072 : 114688)
+                   : ntypes > 1 ? 106496
+                                : (fp64 ? 98304 : 65536);
+  return natoms <= max4 ? 4 : 1;
+}
 // Operation codes of a step sequence (also the graph-cache key alphabet).
 enum Op : char {
   OP_BOOT = 'b',        // half kick + drift (window start, NVE)
@@ -323,11 +339,11 @@ struct Engine final : EngineBase {
   }
 
   int init() override {
-    // rows split over kSplitLanes lanes when one lane per atom would leave
-    // the chip mostly idle (partials: one per block of the larger grid)
+    // (partials: one per block of the larger grid)
     S->lanes = S->cfg.pair_lanes > 0
                    ? S->cfg.pair_lanes
-                   : (S->natoms <= (S->kind == 1 ? kEamSplitMax : kSplitMax) ? kSplitLanes : 1);
+                   : lanes_by_size(S->natoms, S->kind == 1, S->kind == 1 ? S->tables->ntypes : 0,
+                                   std::is_same_v<R, double>);
     S->nb_force = S->nblocks * S->lanes;
     S->nb_rebuild = 0;
     if (!S->cfg.split_rebuild) {

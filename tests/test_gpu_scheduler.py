@@ -721,3 +721,15 @@ def test_download_by_size_and_wanted_arrays(n, prec):
         for k, ref in enumerate((p, v, f)):
             assert np.array_equal(out[k], ref) if want >> k & 1 else np.isnan(out[k]).all()
     sched.close()
+
+
+@pytest.mark.parametrize("pot,prec,last4", [
+    ("johnson", "mixed", 65536), ("johnson", "fp64", 98304), ("alloy", "mixed", 106496),
+    ("morse", "mixed", 114688), ("morse", "fp64", 131072)])
+def test_lanes_by_size(pot, prec, last4):
+    params = I.johnson_alloy_setfl() if pot == "alloy" else potential(pot)
+    L = np.full(3, 130.0)
+    for n, lanes in ((40960, 8), (40961, 4), (last4, 4), (last4 + 1, 1)):
+        sched = FastPipelineScheduler(np.zeros(3), L, n, params, FastPipelineConfig(precision=prec))
+        assert sched.kernel_shape()["pair_lanes"] == lanes
+        sched.close()
