@@ -44,6 +44,13 @@ using namespace sched;
 //                              186,624: 93.6 / 93.5 / 99.5
 constexpr int kSplitLanes = 8;  // the most
 constexpr int kSplit8Max = 40960;
+// Up to a wavefront a SIMD at eight lanes, the passes for few wavefronts
+// (for_neighbours_few). Steps without a rebuild, us, for_neighbours_split /
+// these: EAM 256 atoms 14.0 / 12.1, 4,000 17.0 / 14.3 (FP64 21.3 / 19.0),
+// 8,788 18.8 / 17.8 (FP64 26.6 / 27.1); Morse 4,000 9.5 / 8.6 (FP64 11.8 /
+// 10.7), 8,788 10.4 / 10.6; at 32,000 their loads past a row's end and
+// registers cost 3%.
+constexpr int kFewMax = 8192;
 inline int lanes_by_size(int natoms, bool eam, int ntypes, bool fp64) {
   if (natoms <= kSplit8Max) return kSplitLanes;
   const int max4 = !eam         ? (fp64 ? 131072 : 114688)
@@ -543,11 +550,16 @@ struct Engine final : EngineBase {
     }
     density_go<kEnergy, kWin, kU, false, false>(s);
   }
+  bool few() const { return S->lanes == 8 && S->natoms <= kFewMax; }
+
   template <bool kEnergy>
   void density(hipStream_t s) {
     if (!lds) {
       const int nb = S->nblocks;
-      if (S->lanes == 8)
+      if (few() && !kEnergy)
+        go(k_eam_density<R, Mir, false, 8, true>, nb * 8, kBlock, 0, s, S->a, meta(), coeff(),
+           rc_sq());
+      else if (S->lanes == 8)
         go(k_eam_density<R, Mir, kEnergy, 8>, nb * 8, kBlock, 0, s, S->a, meta(), coeff(),
            rc_sq());
       else if (S->lanes == 4)
@@ -590,6 +602,13 @@ struct Engine final : EngineBase {
   template <int kEpi, bool kEnergy, bool kMulti>
   void eam_force_global(hipStream_t s) {
     const int nb = S->nblocks;
+    if constexpr (!kMulti && !kEnergy) {
+      if (few()) {
+        go(k_eam_force<R, Mir, kEpi, false, false, 8, true>, nb * 8, kBlock, 0, s, S->a, meta(),
+           coeff(), rc_sq());
+        return;
+      }
+    }
     if (S->lanes == 8)
       go(k_eam_force<R, Mir, kEpi, kEnergy, kMulti, 8>, nb * 8, kBlock, 0, s, S->a, meta(),
          coeff(), rc_sq());
@@ -615,7 +634,9 @@ struct Engine final : EngineBase {
       else
         eam_force_global<kEpi, kEnergy, false>(s);
     } else {
-      if (S->lanes == 8)
+      if (few() && !kEnergy)
+        go(k_morse_force<R, Mir, kEpi, false, 8, true>, nb * 8, kBlock, 0, s, S->a, mp());
+      else if (S->lanes == 8)
         go(k_morse_force<R, Mir, kEpi, kEnergy, 8>, nb * 8, kBlock, 0, s, S->a, mp());
       else if (S->lanes == 4)
         go(k_morse_force<R, Mir, kEpi, kEnergy, 4>, nb * 4, kBlock, 0, s, S->a, mp());

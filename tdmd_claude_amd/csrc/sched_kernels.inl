@@ -431,6 +431,46 @@ __device__ __forceinline__ void for_neighbours_split(const StepArgs& a, int i, i
   }
 }
 
+// for_neighbours_split for few wavefronts (kFew passes: one a SIMD, with nothing
+// to hide a load or a chain of arithmetic behind). The next quad's
+// records and the slots of the one after are loaded before a quad's pairs are
+// evaluated (past the row's end the last quad again), and pairs go side by side,
+// kB at a time: batch(records[kB], in_row[kB]) takes all distances, then all
+// table loads, then the sums in slot order. A branch around each pair would put
+// its load after the one before it.
+template <class R>
+constexpr int kFewBatch = sizeof(R) == 4 ? 4 : 2;
+
+template <class T, int kLanes, int kB, class Batch>
+__device__ __forceinline__ void for_neighbours_few(const StepArgs& a, int i, int n, int part,
+                                                   const T* __restrict__ rec, Batch&& batch) {
+  static_assert(4 % kB == 0, "batches tile a quad");
+  const int4* __restrict__ q4 = reinterpret_cast<const int4*>(a.nbr);
+  const int nq = (n + 3) >> 2;
+  if (part >= nq) return;
+  auto slots = [&](int q) { return q4[ell(i, 4 * min(q, nq - 1), a.cap) >> 2]; };
+  const int4 s = slots(part);
+  int4 s1 = slots(part + kLanes);
+  T r[4] = {gather(rec, s.x), gather(rec, s.y), gather(rec, s.z), gather(rec, s.w)};
+  for (int q = part; q < nq; q += kLanes) {
+    const T r1[4] = {gather(rec, s1.x), gather(rec, s1.y), gather(rec, s1.z), gather(rec, s1.w)};
+    s1 = slots(q + 2 * kLanes);
+#pragma unroll
+    for (int u = 0; u < 4; u += kB) {
+      T bm[kB];
+      bool br[kB];
+#pragma unroll
+      for (int v = 0; v < kB; ++v) {
+        bm[v] = r[u + v];
+        br[v] = 4 * q + u + v < n;
+      }
+      batch(bm, br);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) r[u] = r1[u];
+  }
+}
+
 // Sum over the kLanes lanes of one atom (butterfly; every lane ends with
 // the same bits, so the order is fixed).
 template <int kLanes>
@@ -446,7 +486,7 @@ __device__ __forceinline__ double lane_sum(double v) {
 // ... to lane p) and the lanes' partial sums are combined by a butterfly in
 // a fixed order, so the result is run-to-run identical; the grid is kLanes
 // times the one-lane grid and emits one energy / KE partial per 256 threads.
-template <class R, class Mir, bool kEnergy, int kLanes>
+template <class R, class Mir, bool kEnergy, int kLanes, bool kFew = false>
 __global__ void __launch_bounds__(kBlock)
 k_eam_density(StepArgs a, const SplineMeta* __restrict__ meta,
               const typename Quad<R>::type* __restrict__ coeff, double rc_sq) {
@@ -480,10 +520,44 @@ k_eam_density(StepArgs a, const SplineMeta* __restrict__ meta,
         }
       }
     };
-    if constexpr (kLanes == 1)
+    if constexpr (kFew) {
+      constexpr int kB = kFewBatch<R>;
+      for_neighbours_few<T, kLanes, kB>(
+          a, i, n, part, M, [&](const T (&mj)[kB], const bool (&in_row)[kB]) {
+            double r2[kB];
+            bool ok[kB], any = false;
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+              double dx, dy, dz;
+              r2[u] = Mir::delta(mi, mj[u], mpi, &dx, &dy, &dz);
+              ok[u] = in_row[u] && r2[u] < rc_sq;
+              r2[u] = ok[u] ? r2[u] : 0.25 * rc_sq;  // any place in the table
+              any = any || ok[u];
+            }
+            if (!any) return;
+            typename Quad<R>::type c[kB];
+            R t[kB];
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+              const SplineMeta& m = sm[a.ntypes + Mir::type_of(mj[u])];
+              int idx;
+              if constexpr (std::is_same_v<R, float>)
+                idx = locate_f32(meta_f32(m), r2[u], &t[u]);
+              else
+                idx = spline_locate<R>(m, pair_r<R>(r2[u]).r, &t[u]);
+              c[u] = coeff[m.offset + idx];
+            }
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+              const R v = c[u].x + t[u] * (c[u].y + t[u] * (c[u].z + t[u] * c[u].w));
+              rho = ok[u] ? rho + static_cast<double>(v) : rho;
+            }
+          });
+    } else if constexpr (kLanes == 1) {
       for_neighbours<T, kPairUnroll>(a, i, n, M, pair);
-    else
+    } else {
       for_neighbours_split<T, kLanes>(a, i, n, part, M, pair);
+    }
   }
   if constexpr (kLanes > 1) rho = lane_sum<kLanes>(rho);  // every lane takes part
   if (i < a.natoms && part == 0) {
@@ -500,7 +574,7 @@ k_eam_density(StepArgs a, const SplineMeta* __restrict__ meta,
   pass_clock_end(a.pclock);
 }
 
-template <class R, class Mir, int kEpi, bool kEnergy, bool kMulti, int kLanes>
+template <class R, class Mir, int kEpi, bool kEnergy, bool kMulti, int kLanes, bool kFew = false>
 __global__ void __launch_bounds__(kBlock)
 k_eam_force(StepArgs a, const SplineMeta* __restrict__ meta,
             const typename Quad<R>::type* __restrict__ coeff, double rc_sq) {
@@ -589,10 +663,62 @@ k_eam_force(StepArgs a, const SplineMeta* __restrict__ meta,
         fz = fma(fpair, dz, fz);
       }
     };
-    if constexpr (kLanes == 1)
+    if constexpr (kFew) {
+      static_assert(!kMulti && !kEnergy, "one element, forces only");
+      constexpr int kB = kFewBatch<R>;
+      for_neighbours_few<T, kLanes, kB>(
+          a, i, n, part, M2, [&](const T (&mj)[kB], const bool (&in_row)[kB]) {
+            double dx[kB], dy[kB], dz[kB], r2[kB];
+            bool ok[kB], any = false;
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+              r2[u] = Mir::delta(mi, mj[u], mpi, &dx[u], &dy[u], &dz[u]);
+              ok[u] = in_row[u] && r2[u] < rc_sq;
+              r2[u] = ok[u] ? r2[u] : 0.25 * rc_sq;
+              any = any || ok[u];
+            }
+            if (!any) return;
+            Q cphi[kB], crho[kB];
+            R t[kB], trho[kB], rinv[kB];
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+              int kphi, krho;
+              if constexpr (kF32) {
+                const PairT p = pair_t_f32(floc, r2[u]);
+                rinv[u] = p.rinv;
+                t[u] = trho[u] = p.t;
+                kphi = krho = p.idx;
+              } else {
+                const PairR<R> pr = pair_r<R>(r2[u]);
+                rinv[u] = pr.rinv;
+                kphi = spline_locate<R>(sm[2 * nt], pr.r, &t[u]);
+                krho = spline_locate<R>(sm[nt], pr.r, &trho[u]);
+              }
+              cphi[u] = coeff[sm[2 * nt].offset + kphi];
+              crho[u] = coeff[sm[nt].offset + krho];
+            }
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+              auto deriv = [](const Q& c, R x) {
+                if constexpr (kF32)
+                  return cubic_deriv_f(c, x);
+                else  // the same expression as spline_deriv
+                  return c.y + x * (static_cast<R>(2) * c.z + x * static_cast<R>(3) * c.w);
+              };
+              const R drho = deriv(crho[u], trho[u]);
+              const R fpj = Mir::template w_real<R>(mj[u]);
+              const double fpair = static_cast<double>(
+                  -(deriv(cphi[u], t[u]) + fpi * drho + fpj * drho) * rinv[u]);
+              fx = ok[u] ? fma(fpair, dx[u], fx) : fx;
+              fy = ok[u] ? fma(fpair, dy[u], fy) : fy;
+              fz = ok[u] ? fma(fpair, dz[u], fz) : fz;
+            }
+          });
+    } else if constexpr (kLanes == 1) {
       for_neighbours<T, kPairUnroll>(a, i, n, M2, pair);
-    else
+    } else {
       for_neighbours_split<T, kLanes>(a, i, n, part, M2, pair);
+    }
   }
   if constexpr (kLanes > 1) {  // every lane takes part in the shuffles
     fx = lane_sum<kLanes>(fx);
@@ -618,7 +744,7 @@ k_eam_force(StepArgs a, const SplineMeta* __restrict__ meta,
 // Morse pass (morse.hpp:37-55; pair_math.hpp precision contract)
 // ---------------------------------------------------------------------------
 
-template <class R, class Mir, int kEpi, bool kEnergy, int kLanes>
+template <class R, class Mir, int kEpi, bool kEnergy, int kLanes, bool kFew = false>
 __global__ void __launch_bounds__(kBlock) k_morse_force(StepArgs a, MorseCoef p) {
   // The pass gathers from M; with the fused kick-drift the next step's
   // records go to M2 and the host swaps the two buffers after the launch.
@@ -653,10 +779,35 @@ __global__ void __launch_bounds__(kBlock) k_morse_force(StepArgs a, MorseCoef p)
         fz = fma(fpair, dz, fz);
       }
     };
-    if constexpr (kLanes == 1)
+    if constexpr (kFew) {
+      constexpr int kB = kFewBatch<R>;
+      for_neighbours_few<T, kLanes, kB>(
+          a, i, n, part, M, [&](const T (&mj)[kB], const bool (&in_row)[kB]) {
+            double dx[kB], dy[kB], dz[kB], r2[kB];
+            bool ok[kB], any = false;
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+              r2[u] = Mir::delta(mi, mj[u], mpi, &dx[u], &dy[u], &dz[u]);
+              ok[u] = in_row[u] && r2[u] < p.rc_sq;
+              r2[u] = ok[u] ? r2[u] : p.rc_sq;
+              any = any || ok[u];
+            }
+            if (!any) return;
+#pragma unroll
+            for (int u = 0; u < kB; ++u) {
+              R e;
+              const double fpair =
+                  static_cast<double>(morse_fpair<R>(p, pair_r<R>(r2[u]), &e));
+              fx = ok[u] ? fma(fpair, dx[u], fx) : fx;
+              fy = ok[u] ? fma(fpair, dy[u], fy) : fy;
+              fz = ok[u] ? fma(fpair, dz[u], fz) : fz;
+            }
+          });
+    } else if constexpr (kLanes == 1) {
       for_neighbours<T, kPairUnroll>(a, i, n, M, pair);
-    else
+    } else {
       for_neighbours_split<T, kLanes>(a, i, n, part, M, pair);
+    }
   }
   if constexpr (kLanes > 1) {  // every lane takes part in the shuffles
     fx = lane_sum<kLanes>(fx);

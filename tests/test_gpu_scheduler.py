@@ -733,3 +733,24 @@ def test_lanes_by_size(pot, prec, last4):
         sched = FastPipelineScheduler(np.zeros(3), L, n, params, FastPipelineConfig(precision=prec))
         assert sched.kernel_shape()["pair_lanes"] == lanes
         sched.close()
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+@pytest.mark.parametrize("pot", ["johnson", "morse"])
+@pytest.mark.parametrize("nz", [1, 8, 9])
+def test_split_passes_around_one_wavefront_a_simd(nz, pot, prec):
+    # 8,192 atoms are the last of the passes for few wavefronts, 9,216 the first
+    # beyond; 1,024 leaves most of the chip idle. Against one lane per atom: FP64
+    # sums in another order; mixed, the same pair values (to a rounding of the
+    # table offset) in FP64 sums, the force rounded to float.
+    s = I.fcc_lattice(16, 16, nz, 3.615) if nz > 1 else I.fcc_lattice(8, 8, 4, 3.615)
+    I.jitter_uniform(s, 0.1, 99)
+    I.init_velocities(s, 300.0, 3)
+    say("split passes", s.natoms, pot, prec)
+    out = []
+    for lanes in (0, 1):
+        _, p, v, f = gpu_run(s, pot, 3, precision=prec, pair_lanes=lanes)
+        out.append((p, v, f))
+    tol = 1e-12 if prec == "fp64" else 2e-6
+    assert force_rel_err(out[0][2], out[1][2]) < tol
+    assert np.abs(out[0][1] - out[1][1]).max() < tol * np.abs(out[1][1]).max()
