@@ -2047,10 +2047,9 @@ static __global__ void __launch_bounds__(kHaloBlock) k_halo(StepArgs a, int nblo
 // barrier costs 1.3-7 us, so work moves into a neighbouring phase where its
 // inputs allow.
 //
-// The grid is sized by the host to what the device holds resident at once
-// (occupancy x CUs), so every workgroup of the launch runs concurrently and
-// the barrier can complete. The barrier is a count + generation pair in
-// device memory; its wait is bounded: a wait longer than kBarrierSpins
+// The host keeps the grid to at most one workgroup a CU (the LDS of the list
+// search holds one), so every workgroup of the launch runs at once and the
+// barrier can complete. Its wait is bounded: a wait longer than kBarrierSpins
 // polls sets flags[3] and the kernel returns (the host reports the error)
 // instead of hanging.
 //
@@ -2112,7 +2111,6 @@ __device__ __forceinline__ bool grid_barrier(GridBarrier* b, unsigned int* passe
 
 constexpr int kRebuildBlock = 1024;  // workgroup of the fused rebuild
 
-// The grid is at most as many workgroups as the device holds at once.
 template <class R, class Mir>
 __global__ void __launch_bounds__(kRebuildBlock)
 k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double near_sq,
