@@ -336,13 +336,18 @@ struct Engine final : EngineBase {
   // Workgroups of the list search and of the fused rebuild: a cell each up to
   // 64, two each beyond (the rebuild of 864 atoms in 27 cells: 30.9 us with 27,
   // 34.6 with 14; of 10,976 in 216: 50.4 with 216, 45.7 with 108: a barrier
-  // costs more the more arrive at it); one a CU and one per 32 atoms at most, so
-  // that several small systems can be resident together. Under the displacement
-  // policy the launch is a no-op check on nearly every step: one per 512 atoms.
+  // costs more the more arrive at it); one a CU, and by the atoms so few that
+  // the rebuilds of several schedulers on streams of their own can be resident
+  // together: one per 32 atoms where every launch rebuilds; under the
+  // displacement policy one per 1024, but up to 64 one per 512 (four such fit;
+  // steps of 32,000 EAM atoms: 27.5 us with 63, 37.9 with 8).
   int list_grid(int ncu) const {
-    const int per = S->cfg.rebuild_policy == TDMD_REBUILD_DISPLACEMENT ? 512 : 32;
+    const int n = S->natoms;
+    const int by_atoms = S->cfg.rebuild_policy == TDMD_REBUILD_DISPLACEMENT
+                             ? std::max((n + 1023) / 1024, std::min(64, (n + 511) / 512))
+                             : (n + 31) / 32;
     const int cells = std::min(S->g.ncells, std::max(64, (S->g.ncells + 1) / 2));
-    return std::max(1, std::min({ncu, (S->natoms + per - 1) / per, cells}));
+    return std::max(1, std::min({ncu, by_atoms, cells}));
   }
 
   int init() override {
