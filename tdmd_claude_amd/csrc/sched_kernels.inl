@@ -993,42 +993,28 @@ __device__ __forceinline__ void scan_cells_grid(const GridArgs& g, int phase) {
   if (c1 == g.ncells && c0 < c1 && threadIdx.x == 0) g.cstart[g.ncells] = run;
 }
 
-// Deterministic order inside a cell: by upload index.
-__device__ __forceinline__ void order_cell(const GridArgs& g, int32_t* seg, int n) {
-  for (int x = 1; x < n; ++x) {
-    const int32_t v = seg[x];
-    const int32_t kv = g.orig[v];
-    int y = x - 1;
-    while (y >= 0 && g.orig[seg[y]] > kv) {
-      seg[y + 1] = seg[y];
-      --y;
-    }
-    seg[y + 1] = v;
-  }
-}
-
-// The same order by one wavefront: lane l takes the cell's l-th atom and
-// counts the atoms with a smaller upload index (indices are unique, so the
-// counts are the sorted positions); put(old index, new slot) for each atom.
-// Cells of more than 64 atoms are sorted in place by one lane first.
+// Deterministic order inside a cell, by upload index: one wavefront, 64 of the
+// cell's atoms at a time; a lane counts the atoms with a smaller index than its
+// own (indices are unique, so the counts are the sorted positions), and
+// put(old index, new slot) is called for each atom. (Cells of more than 64 atoms
+// used to be sorted by one lane: half or more of a rebuild from 74 atoms a cell.)
 template <class Put>
 __device__ __forceinline__ void order_cell_wave(const GridArgs& g, int r, Put&& put) {
   const int lane = static_cast<int>(threadIdx.x & 63);
-  const int start = g.cstart[r], n = g.cstart[r + 1] - start;
-  int32_t* seg = g.sidx + start;
-  if (n > 64) {
-    if (lane == 0) order_cell(g, seg, n);
-    // lane 0's stores are complete before the other lanes read them
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    for (int k = lane; k < n; k += 64) put(seg[k], start + k);
-    return;
+  const int start = __builtin_amdgcn_readfirstlane(g.cstart[r]);
+  const int n = __builtin_amdgcn_readfirstlane(g.cstart[r + 1]) - start;
+  const int32_t* const seg = g.sidx + start;
+  for (int b = 0; b < n; b += 64) {
+    const int32_t v = b + lane < n ? seg[b + lane] : 0;
+    const int32_t kv = b + lane < n ? g.orig[v] : 0x7fffffff;
+    int pos = 0;
+    for (int c = 0; c < n; c += 64) {
+      const int32_t kc = c == b ? kv : c + lane < n ? g.orig[seg[c + lane]] : 0x7fffffff;
+      const int e = min(64, n - c);
+      for (int m = 0; m < e; ++m) pos += __builtin_amdgcn_readlane(kc, m) < kv ? 1 : 0;
+    }
+    if (b + lane < n) put(v, start + pos);
   }
-  const int32_t v = lane < n ? seg[lane] : 0;
-  const int32_t kv = lane < n ? g.orig[v] : 0x7fffffff;
-  int pos = 0;
-  for (int m = 0; m < n; ++m) pos += __shfl(kv, m, 64) < kv ? 1 : 0;
-  if (lane < n) put(v, start + pos);
 }
 
 // Atom o (old slot) to slot s of the scratch arrays, and its gather record.
@@ -1285,7 +1271,7 @@ __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArg
 
 // The rows of all cells, dealt to teams of wavefronts: the whole 1024-thread
 // workgroup, or halves or quarters of it where there are more cells than
-// workgroups. A team stages its cell's candidates -- the atoms of the 27
+// workgroups and their stencils fit a team's share of the LDS. A team stages its cell's candidates -- the atoms of the 27
 // stencil cells, in rank order -- in LDS once: FP32 offsets from the cell's
 // centre, from the wrapping difference of the fixed-point records or from the
 // FP64 position with the stencil entry's image. Then, in three steps:
@@ -1355,7 +1341,7 @@ __device__ __forceinline__ int nlist_cells(const StepArgs& a, const GridArgs& g,
   const int lane = static_cast<int>(threadIdx.x & 63);
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   const int grid = static_cast<int>(gridDim.x);
-  const int tsh = g.ncells > 2 * grid ? 2 : g.ncells > grid ? 1 : 0;
+  const int tsh = min(g.list_teams, g.ncells > 2 * grid ? 2 : g.ncells > grid ? 1 : 0);
   const int teams = 1 << tsh;
   const int tw = kWaves >> tsh;                           // wavefronts of a team
   const int team = w >> (4 - tsh), wt = w & (tw - 1);     // this one's team and place in it

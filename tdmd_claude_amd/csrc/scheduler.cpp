@@ -280,6 +280,7 @@ int sched_alloc(tdmd_sched* S) {
   if ((rc = dalloc(S, &img, h_img.size()))) return rc;
   TDMD_HIP_TRY(hipMemcpy(img, h_img.data(), h_img.size(), hipMemcpyHostToDevice));
   g.around_img = img;
+  g.list_teams = 2;  // until the first count
   g.images = images ? 1 : 0;  // batches: decided per box (BoxGeo::images)
   if (S->multibox) {
     BoxGeo* boxes;
@@ -469,6 +470,16 @@ int check_flags(tdmd_sched* S) {
   return TDMD_OK;
 }
 
+// log2 of the teams that a list search's workgroup may form for stencils of m
+// atoms: a team has its share of the candidates (4,096) and of the mask words
+// (8,192; m / 27 rows of m / 32 words), and what does not fit is searched from
+// memory.
+int list_teams(double m) {
+  for (int t = 2; t > 0; --t)
+    if (m <= 4096 >> t && m * m / (27 * 32) <= 8192 >> t) return t;
+  return 0;
+}
+
 // First neighbour build: sort, count exactly, size the list, fill.
 int first_build(tdmd_sched* S) {
   hipStream_t s = S->stream;
@@ -504,6 +515,15 @@ int first_build(tdmd_sched* S) {
     S->a.cap = cap;
     drop_graphs(S);
   }
+  // a stencil's candidates, from the longest row: the 27 cells against its sphere
+  double cells = 27.0 * 3.0 / (4.0 * M_PI);
+  for (int d = 0; d < 3; ++d) {
+    double inv = S->multibox ? S->h_boxes[0].inv_cs[d] : S->g.inv_cs[d];
+    if (S->multibox)
+      for (const BoxGeo& b : S->h_boxes) inv = std::min(inv, b.inv_cs[d]);
+    cells /= inv * S->r_list;
+  }
+  S->g.list_teams = list_teams(cells * (maxc + 1));
   rc = S->eng->fill_pass(s);
   if (rc) return rc;
   ++S->host_rebuilds;

@@ -754,3 +754,29 @@ def test_split_passes_around_one_wavefront_a_simd(nz, pot, prec):
     tol = 1e-12 if prec == "fp64" else 2e-6
     assert force_rel_err(out[0][2], out[1][2]) < tol
     assert np.abs(out[0][1] - out[1][1]).max() < tol * np.abs(out[1][1]).max()
+
+
+@pytest.mark.parametrize("per_cell", [1, 63, 64, 65, 128, 129, 300])
+def test_order_inside_cells_by_atoms_per_cell(per_cell):
+    # 27 cells of per_cell atoms around each 64: the sort's result does not depend
+    # on the order in which the atoms reach their cells, so two runs agree bit for
+    # bit, and every atom is still there.
+    n = 27 * per_cell
+    rng = np.random.Generator(np.random.PCG64(8))
+    L = np.full(3, 21.0)
+    cell = np.stack(np.meshgrid(*[np.arange(3)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    pos = 7.0 * (np.repeat(cell, per_cell, axis=0) + rng.uniform(0.01, 0.99, size=(n, 3)))
+    pos = pos[rng.permutation(n)]
+    s = I.System(lo=np.zeros(3), hi=L, pos=pos, vel=rng.normal(size=(n, 3)),
+                 types=np.ones(n, dtype=np.int32), ids=np.arange(1, n + 1, dtype=np.int32),
+                 masses=np.array([1.0, 63.546]))
+    out = []
+    for _ in range(2):
+        sched = FastPipelineScheduler.for_system(
+            s, (1e-9, 1.0, 2.8, 6.0), FastPipelineConfig(precision="fp64", rebuild_every=1,
+                                                         r_skin=0.9, dt=1e-6))
+        sched.run_until(4)
+        out.append(sched.download())
+        sched.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+    assert np.abs(out[0][0] - pos).max() < 1e-3  # upload order, every atom
