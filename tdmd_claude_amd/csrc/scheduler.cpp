@@ -88,6 +88,27 @@ k_upload_order(StepArgs a, const int32_t* orig, double* out) {
   out[6 * n + o + 2] = static_cast<double>(static_cast<const R*>(a.fz)[s]);
 }
 
+// The stream's device as the calling thread's, for a scope: a download may be
+// called from a thread that has another device current.
+class StreamDevice {
+ public:
+  explicit StreamDevice(hipStream_t s) {
+    int dev = 0;
+    if (hipGetDevice(&before_) == hipSuccess && hipStreamGetDevice(s, &dev) == hipSuccess &&
+        dev != before_)
+      changed_ = hipSetDevice(dev) == hipSuccess;
+  }
+  ~StreamDevice() {
+    if (changed_) (void)hipSetDevice(before_);
+  }
+  StreamDevice(const StreamDevice&) = delete;
+  StreamDevice& operator=(const StreamDevice&) = delete;
+
+ private:
+  int before_ = 0;
+  bool changed_ = false;
+};
+
 // Doubles [from, to) of the scratch block to the host by way of the staging
 // buffer; the block holds dst[0..2], 3 N doubles each (null: not wanted).
 int staged_download(const tdmd_sched* S, double* const dst[3], size_t from, size_t to) {
@@ -922,6 +943,7 @@ int tdmd_sched_download(const tdmd_sched* S, double* pos, double* vel, double* f
     // the scratch block and the staging buffer are this scheduler's: one
     // download at a time
     std::lock_guard<std::mutex> lock(S->download_mu);
+    const StreamDevice device(S->stream);
     double* const out = S->t.px;
     const int nb = (S->natoms + 255) / 256;
     if (S->cfg.precision == TDMD_MIXED)
