@@ -433,6 +433,12 @@ int tdmd_sched_autotune(tdmd_sched* s, int32_t iters, int32_t out[2]);
 /* The current kernel shape (no reference counterpart): out[0] = lanes per
  * neighbour row, out[1] = pair_unroll, out[2] = lds_budget. */
 int tdmd_sched_kernel_shape(const tdmd_sched* s, int32_t out[3]);
+/* The grid barrier of the fused rebuild (no reference counterpart;
+ * diagnostics). *workgroups (may be null) gets the rebuild's grid, all of
+ * which has to run at once (0: separate kernels). polls >= 0 sets how often a
+ * workgroup polls before it gives up and run_until reports it (at creation
+ * 4,194,304, some seconds; 0: at once); polls < 0 leaves it. */
+int tdmd_sched_rebuild_barrier(tdmd_sched* s, int32_t polls, int32_t* workgroups);
 /* Halo staging (no reference counterpart; diagnostics): out[0] = blocks of
  * 1024 atoms, out[1] = blocks whose halo is staged in LDS, out[2] = largest
  * halo (atoms), out[3] = halo atoms summed over all blocks. All zero when

@@ -246,6 +246,7 @@ _PROTOS = {
     "tdmd_sched_pass_times": (C.c_int, [_VP, C.POINTER(C.c_float)]),
     "tdmd_sched_autotune": (C.c_int, [_VP, _I32, _PI32]),
     "tdmd_sched_kernel_shape": (C.c_int, [_VP, _PI32]),
+    "tdmd_sched_rebuild_barrier": (C.c_int, [_VP, C.c_int32, _PI32]),
     "tdmd_pipe_create": (C.c_int, [C.POINTER(_VP), C.POINTER(Box), _I32, C.POINTER(MorseParams),
                                    C.POINTER(PipeConfig)]),
     "tdmd_pipe_destroy": (C.c_int, [_VP]),

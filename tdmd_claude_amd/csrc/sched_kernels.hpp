@@ -307,7 +307,10 @@ struct GridArgs {
   int32_t* orig;           // [N] upload index
   int32_t* done;           // completion counter
   int32_t* wsum;           // [kMaxScanGroups] per-workgroup cell sums (fused rebuild)
+  int polls;               // of the fused rebuild's barrier before it gives up
 };
+
+constexpr int kBarrierPolls = 1 << 22;  // some seconds
 
 constexpr int kMaxScanGroups = 4096;  // workgroups of the fused rebuild, at most
 // Up to this many cells every workgroup of the fused rebuild scans them for

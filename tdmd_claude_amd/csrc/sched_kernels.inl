@@ -2035,9 +2035,13 @@ static __global__ void __launch_bounds__(kHaloBlock) k_halo(StepArgs a, int nblo
 //
 // The host keeps the grid to at most one workgroup a CU (the LDS of the list
 // search holds one), so every workgroup of the launch runs at once and the
-// barrier can complete. Its wait is bounded: a wait longer than kBarrierSpins
-// polls sets flags[3] and the kernel returns (the host reports the error)
-// instead of hanging.
+// barrier can complete. Its wait is bounded: a workgroup that has polled
+// GridArgs::polls times sets flags[3] and returns (the host reports the error)
+// instead of hanging. One that gave up arrives at no later barrier, so none is
+// passed and no later phase starts. What it leaves -- cell counters in use,
+// arrivals that `gen` does not cover -- is no state to start from: every launch
+// until the host has cleared it (check_flags, upload) returns at its first
+// barrier, whose arrivals would otherwise count as complete.
 //
 // Only thread 0 of each workgroup touches the barrier: one release fence, a
 // relaxed arrival, relaxed polls, one acquire fence, all at agent scope, and
@@ -2047,16 +2051,17 @@ static __global__ void __launch_bounds__(kHaloBlock) k_halo(StepArgs a, int nblo
 // working.) Polls back off with a growing sleep.
 // ---------------------------------------------------------------------------
 
-constexpr long kBarrierSpins = 1L << 22;
-
 // `passed`: barriers this workgroup has passed (GridBarrier::gen at the
-// launch's start, counted on here).
+// launch's start, counted on here). `gone`, thread 0's: gives up without
+// arriving. `polls`: GridArgs::polls.
 __device__ __forceinline__ bool grid_barrier(GridBarrier* b, unsigned int* passed,
-                                             int32_t* flags) {
+                                             int32_t* flags, int polls, bool gone = false) {
   __shared__ int ok;
   __syncthreads();
   const unsigned int n = ++*passed;
-  if (threadIdx.x == 0) {
+  if (threadIdx.x == 0 && gone) {
+    ok = 0;
+  } else if (threadIdx.x == 0) {
     ok = 1;
     unsigned int target = n * gridDim.x;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
@@ -2073,21 +2078,22 @@ __device__ __forceinline__ bool grid_barrier(GridBarrier* b, unsigned int* passe
         __hip_atomic_fetch_add(&b->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
-    long spins = 0;
-    while (static_cast<int>(__hip_atomic_load(&b->count, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT) -
-                            target) < 0) {
+    for (int spins = 0;; ++spins) {
+      if (spins == polls) {
+        ok = 0;
+        atomicExch(&flags[3], 1);
+        break;
+      }
+      if (static_cast<int>(__hip_atomic_load(&b->count, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT) -
+                           target) >= 0)
+        break;
       if (spins < 64)
         __builtin_amdgcn_s_sleep(1);
       else if (spins < 256)
         __builtin_amdgcn_s_sleep(16);
       else
         __builtin_amdgcn_s_sleep(64);
-      if (++spins > kBarrierSpins) {
-        ok = 0;
-        atomicExch(&flags[3], 1);
-        break;
-      }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
@@ -2112,9 +2118,12 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
     HaloLds halo;
   } lds;
   unsigned int passed = bar->gen;  // written below once every workgroup has read it
+  // (read by one thread: workgroups of this launch may be giving up already)
+  const bool gone = threadIdx.x == 0 && __hip_atomic_load(&a.flags[3], __ATOMIC_RELAXED,
+                                                          __HIP_MEMORY_SCOPE_AGENT) != 0;
   // (the cell counters are clear: the phase that last reads them clears them)
   for (int i = tid; i < N; i += nthr) bin_atom<Mir>(a, g, i);
-  if (!grid_barrier(bar, &passed, a.flags)) return;
+  if (!grid_barrier(bar, &passed, a.flags, g.polls, gone)) return;
   if (g.ncells <= kScanOwn) {
     // few cells: every workgroup scans them for itself, without a barrier
     int32_t* const cstart = lds.cstart;
@@ -2125,12 +2134,12 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
     for (int i = tid; i < N; i += nthr) scatter_atom(g, i, cstart);
   } else {
     scan_cells_grid<kRebuildBlock>(g, 1);
-    if (!grid_barrier(bar, &passed, a.flags)) return;
+    if (!grid_barrier(bar, &passed, a.flags, g.polls)) return;
     scan_cells_grid<kRebuildBlock>(g, 2);
-    if (!grid_barrier(bar, &passed, a.flags)) return;
+    if (!grid_barrier(bar, &passed, a.flags, g.polls)) return;
     for (int i = tid; i < N; i += nthr) scatter_atom(g, i, g.cstart);
   }
-  if (!grid_barrier(bar, &passed, a.flags)) return;
+  if (!grid_barrier(bar, &passed, a.flags, g.polls)) return;
   {
     // one cell per wavefront, cells dealt to the workgroups wave by wave
     const int nw = gridDim.x * (kRebuildBlock / 64);
@@ -2142,7 +2151,7 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
       g.cursor[r] = 0;
     }
   }
-  if (!grid_barrier(bar, &passed, a.flags)) return;
+  if (!grid_barrier(bar, &passed, a.flags, g.polls)) return;
   // the state's arrays back from the scratch ones, beside the list search,
   // which reads the scratch arrays and the records
   for (int s = tid; s < N; s += nthr) copyback_atom<R, Mir>(a, g, t, s);
@@ -2150,7 +2159,7 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
   report_count<false>(a, count, nullptr);
   if constexpr (Mir::kFixed) {
     if (a.stage_cap > 0) {  // halos of the staged passes, from the new rows
-      if (!grid_barrier(bar, &passed, a.flags)) return;
+      if (!grid_barrier(bar, &passed, a.flags, g.polls)) return;
       static_assert(kRebuildBlock == kHaloBlock, "halos are built by whole workgroups");
       build_halos(a, (N + kHaloBlock - 1) / kHaloBlock, lds.halo);
     }

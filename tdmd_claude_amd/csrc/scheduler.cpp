@@ -302,6 +302,7 @@ int sched_alloc(tdmd_sched* S) {
   TDMD_HIP_TRY(hipMemcpy(img, h_img.data(), h_img.size(), hipMemcpyHostToDevice));
   g.around_img = img;
   g.list_teams = 2;  // until the first count
+  g.polls = sched::kBarrierPolls;
   g.images = images ? 1 : 0;  // batches: decided per box (BoxGeo::images)
   if (S->multibox) {
     BoxGeo* boxes;
@@ -840,6 +841,18 @@ int tdmd_sched_autotune(tdmd_sched* S, int32_t iters, int32_t out[2]) {
 int tdmd_sched_kernel_shape(const tdmd_sched* S, int32_t out[3]) {
   if (!S || !out || !S->eng) return fail(TDMD_E_INVALID, "sched_kernel_shape: null");
   S->eng->shape(out);
+  return TDMD_OK;
+}
+
+int tdmd_sched_rebuild_barrier(tdmd_sched* S, int32_t polls, int32_t* workgroups) {
+  if (!S) return fail(TDMD_E_INVALID, "sched_rebuild_barrier: null");
+  if (workgroups) *workgroups = S->nb_rebuild;
+  if (polls >= 0 && polls != S->g.polls) {
+    // captured graphs hold the limit
+    TDMD_HIP_TRY(hipStreamSynchronize(S->stream));
+    drop_graphs(S);
+    S->g.polls = polls;
+  }
   return TDMD_OK;
 }
 

@@ -214,6 +214,13 @@ class FastPipelineScheduler:
         return {"pair_lanes": int(out[0]), "pair_unroll": int(out[1]),
                 "lds_budget": int(out[2])}
 
+    def rebuild_barrier(self, polls: int = -1) -> int:
+        """Workgroups of the fused rebuild, which have to run at once (0: separate
+        kernels); polls >= 0 sets how often one polls the barrier before it gives up."""
+        n = C.c_int32()
+        capi.call("tdmd_sched_rebuild_barrier", self._h, int(polls), C.byref(n))
+        return n.value
+
     def halo_info(self) -> dict:
         """LDS halo staging: 1024-atom blocks, blocks staged, largest and total halo."""
         out = (C.c_int64 * 4)()

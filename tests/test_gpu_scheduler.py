@@ -780,3 +780,33 @@ def test_order_inside_cells_by_atoms_per_cell(per_cell):
         sched.close()
     assert all(np.array_equal(a, b) for a, b in zip(*out))
     assert np.abs(out[0][0] - pos).max() < 1e-3  # upload order, every atom
+
+
+@pytest.mark.parametrize("policy,skin", [("fixed", 1.0), ("displacement", 0.02)])
+@pytest.mark.parametrize("pot,lanes", [("morse", 0), ("johnson", 1)])
+def test_rebuilds_behind_one_that_gave_up(pot, lanes, policy, skin):
+    # A rebuild whose barrier gives up (without a poll here) leaves the cell
+    # counters in use; the rebuilds behind it in the same window leave them alone,
+    # the call reports it, and after an upload the scheduler runs as a fresh one
+    # does, bit for bit.
+    s = fcc(8)
+    cfg = FastPipelineConfig(precision="mixed", pair_lanes=lanes, rebuild_policy=policy,
+                             rebuild_every=2, r_skin=skin)
+    say("rebuild that gives up", pot, policy)
+    fresh = FastPipelineScheduler.for_system(s, potential(pot), cfg)
+    fresh.run_until(24)
+    assert fresh.stats().rebuilds > 3
+    sched = FastPipelineScheduler.for_system(s, potential(pot), cfg)
+    sched.run_until(1)
+    assert sched.rebuild_barrier(0) >= 1
+    with pytest.raises(capi.TdmdError, match="barrier timed out"):
+        sched.run_until(24)
+    for call in (sched.download, lambda: sched.run_until(30)):
+        with pytest.raises(capi.TdmdError, match="upload"):
+            call()
+    sched.rebuild_barrier(1 << 22)
+    sched.upload_system(s)
+    sched.run_until(24)
+    assert all(np.array_equal(a, b) for a, b in zip(sched.download(), fresh.download()))
+    sched.close()
+    fresh.close()
