@@ -465,27 +465,34 @@ void sched_free(tdmd_sched* S) {
   if (S->stream) (void)hipStreamDestroy(S->stream);
 }
 
+// What a rebuild expects at its start, whatever the last one left: flags and
+// cell counters clear, no arrivals at the barrier.
+int clear_rebuild(tdmd_sched* S) {
+  TDMD_HIP_TRY(hipMemset(S->d_bar, 0, sizeof(GridBarrier)));
+  TDMD_HIP_TRY(hipMemset(S->g.ccount, 0, static_cast<size_t>(S->g.ncells) * 4));
+  TDMD_HIP_TRY(hipMemset(S->g.cursor, 0, static_cast<size_t>(S->g.ncells) * 4));
+  TDMD_HIP_TRY(hipMemset(S->a.flags, 0, 32));
+  return TDMD_OK;
+}
+
 int check_flags(tdmd_sched* S) {
   int32_t f[4];
   TDMD_HIP_TRY(hipMemcpy(f, S->a.flags, 16, hipMemcpyDeviceToHost));
+  if (f[3]) {
+    // The rebuild stopped between phases: the atoms may be half permuted (and,
+    // integrated on, non-finite: this flag comes first). The kernels have ended
+    // (the stream was synchronised), so the counters are cleared here; the state
+    // is unusable until the next upload.
+    S->uploaded = false;
+    S->initial_forces = false;
+    if (const int rc = clear_rebuild(S)) return rc;
+    return fail(TDMD_E_HIP, "scheduler: fused rebuild grid barrier timed out (workgroups not "
+                            "co-resident); upload again, or use split_rebuild");
+  }
   if (f[2])
     return fail(TDMD_E_NONFINITE,
                 "scheduler: non-finite position, or an atom outside the representable range "
                 "of an open axis (lo - 2W .. lo + 2W, W = max(box length, r_list))");
-  if (f[3]) {
-    // The rebuild stopped between phases: the atoms may be half permuted and
-    // the barrier's arrival counters hold the arrivals of workgroups that
-    // returned, and the cell counters may be in use. The kernel has ended (the
-    // stream was synchronised), so the counters are cleared here; the state is unusable until the next upload.
-    TDMD_HIP_TRY(hipMemset(S->d_bar, 0, sizeof(GridBarrier)));
-    TDMD_HIP_TRY(hipMemset(S->g.ccount, 0, static_cast<size_t>(S->g.ncells) * 4));
-    TDMD_HIP_TRY(hipMemset(S->g.cursor, 0, static_cast<size_t>(S->g.ncells) * 4));
-    TDMD_HIP_TRY(hipMemset(S->a.flags, 0, 32));
-    S->uploaded = false;
-    S->initial_forces = false;
-    return fail(TDMD_E_HIP, "scheduler: fused rebuild grid barrier timed out (workgroups not "
-                            "co-resident); upload again, or use split_rebuild");
-  }
   if (f[1] > S->a.cap)
     return fail(TDMD_E_OVERFLOW, "scheduler: neighbour capacity " + std::to_string(S->a.cap) +
                                      " exceeded (max count " + std::to_string(f[1]) + ")");
@@ -913,8 +920,7 @@ int tdmd_sched_upload(tdmd_sched* S, const double* pos, const double* vel, const
   std::vector<int32_t> iota(static_cast<size_t>(N));
   std::iota(iota.begin(), iota.end(), 0);
   TDMD_HIP_TRY(hipMemcpy(S->g.orig, iota.data(), N * 4, hipMemcpyHostToDevice));
-  TDMD_HIP_TRY(hipMemset(S->a.flags, 0, 32));
-  if (S->d_bar) TDMD_HIP_TRY(hipMemset(S->d_bar, 0, sizeof(GridBarrier)));
+  if (const int rc = clear_rebuild(S)) return rc;
   std::vector<double> nhc0(64, 0.0);  // fresh chain, no pending scale
   nhc0[24] = 1.0;
   TDMD_HIP_TRY(hipMemcpy(S->a.nhc, nhc0.data(), 64 * 8, hipMemcpyHostToDevice));

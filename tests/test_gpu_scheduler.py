@@ -810,3 +810,34 @@ def test_rebuilds_behind_one_that_gave_up(pot, lanes, policy, skin):
     assert all(np.array_equal(a, b) for a, b in zip(sched.download(), fresh.download()))
     sched.close()
     fresh.close()
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+@pytest.mark.parametrize("polls", [0, 2])
+def test_recovery_from_a_rebuild_that_gave_up_beside_a_lost_atom(polls, prec):
+    # An atom that leaves the finite range in the step in which the rebuild gives
+    # up raises both flags: the call reports the rebuild, refuses to go on, and an
+    # upload starts from clear cell counters.
+    s = fcc(8)
+    lost = I.System(lo=s.lo, hi=s.hi, pos=s.pos, vel=s.vel.copy(), types=s.types, ids=s.ids,
+                    masses=s.masses)
+    lost.vel[77] = np.inf
+    cfg = FastPipelineConfig(precision=prec, rebuild_every=1)
+    say("rebuild that gives up, atom lost", polls, prec)
+    fresh = FastPipelineScheduler.for_system(s, MORSE_CU, cfg)
+    fresh.run_until(12)
+    sched = FastPipelineScheduler.for_system(lost, MORSE_CU, cfg)
+    with pytest.raises(capi.TdmdError, match="non-finite"):
+        sched.run_until(4)
+    sched.upload_system(lost)
+    sched.rebuild_barrier(polls)
+    with pytest.raises(capi.TdmdError, match="barrier timed out"):
+        sched.run_until(4)
+    with pytest.raises(capi.TdmdError, match="upload"):
+        sched.download()
+    sched.rebuild_barrier(1 << 22)
+    sched.upload_system(s)
+    sched.run_until(12)
+    assert all(np.array_equal(a, b) for a, b in zip(sched.download(), fresh.download()))
+    sched.close()
+    fresh.close()
