@@ -333,19 +333,23 @@ struct Engine final : EngineBase {
     S->nb_force = lds ? nb_lds : S->nblocks * lanes;
   }
 
-  // Workgroups of the list search and of the fused rebuild: a cell each up to
-  // 64, two each beyond (the rebuild of 864 atoms in 27 cells: 30.9 us with 27,
-  // 34.6 with 14; of 10,976 in 216: 50.4 with 216, 45.7 with 108: a barrier
-  // costs more the more arrive at it); one a CU, and by the atoms so few that
-  // the rebuilds of several schedulers on streams of their own can be resident
-  // together: one per 32 atoms where every launch rebuilds; under the
-  // displacement policy one per 1024, but up to 64 one per 512 (four such fit;
-  // steps of 32,000 EAM atoms: 27.5 us with 63, 37.9 with 8).
+  // Workgroups of the fused rebuild: a cell each up to 64, two each beyond (the
+  // rebuild of 864 atoms in 27 cells: 30.9 us with 27, 34.6 with 14; of 10,976
+  // in 216: 50.4 with 216, 45.7 with 108: a barrier costs more the more arrive
+  // at it); one a CU, which the list search's LDS fills; and by the atoms one per
+  // 32 where every launch rebuilds, one per 1024 under the displacement policy
+  // and above 131,072. Rebuilds that run at the same time (schedulers on streams
+  // or in processes of their own) have to be resident together, or they wait for
+  // each other until they give up: on 256 CUs eight of 32,000 atoms under the
+  // displacement policy, but under the fixed one a single scheduler of 8,192
+  // atoms in 512 cells takes the chip. Such programs want split_rebuild.
+  // (One per 512 atoms up to 64 under the displacement policy takes 17 us less a
+  // rebuild of 32,000 Morse atoms in FP64, 63 workgroups against 32, and fits
+  // four.)
   int list_grid(int ncu) const {
     const int n = S->natoms;
-    const int by_atoms = S->cfg.rebuild_policy == TDMD_REBUILD_DISPLACEMENT
-                             ? std::max((n + 1023) / 1024, std::min(64, (n + 511) / 512))
-                             : (n + 31) / 32;
+    const bool few = S->cfg.rebuild_policy == TDMD_REBUILD_DISPLACEMENT || n > 131072;
+    const int by_atoms = few ? (n + 1023) / 1024 : (n + 31) / 32;
     const int cells = std::min(S->g.ncells, std::max(64, (S->g.ncells + 1) / 2));
     return std::max(1, std::min({ncu, by_atoms, cells}));
   }

@@ -841,3 +841,24 @@ def test_recovery_from_a_rebuild_that_gave_up_beside_a_lost_atom(polls, prec):
     assert all(np.array_equal(a, b) for a, b in zip(sched.download(), fresh.download()))
     sched.close()
     fresh.close()
+
+
+@pytest.mark.parametrize("policy", ["fixed", "displacement"])
+@pytest.mark.parametrize("n", [500, 4000, 32000, 65537, 131072, 131073, 200000])
+def test_rebuild_grids_of_several_schedulers_fit_the_chip(n, policy):
+    # Rebuilds that run at the same time have to be resident together, one
+    # workgroup a CU: at most one per 1024 atoms under the displacement policy and
+    # above 131,072 atoms (eight schedulers of 32,000 atoms fit 256 CUs), one per
+    # 32 elsewhere.
+    L = np.full(3, (n / 0.085) ** (1.0 / 3.0))
+    for pot, prec in (("morse", "mixed"), ("johnson", "fp64")):
+        sched = FastPipelineScheduler(np.zeros(3), L, n, potential(pot),
+                                      FastPipelineConfig(precision=prec, rebuild_policy=policy))
+        per = 1024 if policy == "displacement" or n > 131072 else 32
+        assert 1 <= sched.rebuild_barrier() <= min(256, -(-n // per))
+        sched.close()
+        sched = FastPipelineScheduler(np.zeros(3), L, n, potential(pot),
+                                      FastPipelineConfig(precision=prec, rebuild_policy=policy,
+                                                         split_rebuild=True))
+        assert sched.rebuild_barrier() == 0
+        sched.close()
