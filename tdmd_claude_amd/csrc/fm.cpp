@@ -207,7 +207,7 @@ __global__ void k_fm_reduce(const double* __restrict__ partials, int nblk, int n
 // FD-Hermite coefficients from knot values (build_fd_hermite on the device,
 // same operation order, no contraction): spline s = 0 F, 1 rho, 2 phi; quads:
 // F, rho, phi intervals in a row. Clears the coefficient gradients (blocks
-// [spline][4][ni]) for the adjoint.
+// [spline][4][ni]) for an adjoint that follows; null: they stay.
 template <class R>
 __global__ void k_fm_build_coeffs(const double* __restrict__ vals, int nrho, double drho, int nr,
                                   double dr, double* __restrict__ gcoef,
@@ -232,7 +232,8 @@ __global__ void k_fm_build_coeffs(const double* __restrict__ vals, int nrho, dou
   const int niF = nrho - 1, niR = nr - 1;
   const size_t base = s == 0 ? 0 : (s == 1 ? 4 * static_cast<size_t>(niF)
                                            : 4 * static_cast<size_t>(niF) + 4 * niR);
-  for (int k = 0; k < 4; ++k) gcoef[base + static_cast<size_t>(k) * ni + i] = 0.0;
+  if (gcoef)
+    for (int k = 0; k < 4; ++k) gcoef[base + static_cast<size_t>(k) * ni + i] = 0.0;
   const int qo = s == 0 ? 0 : (s == 1 ? niF : niF + niR);
   typename Quad<R>::type q;
   q.x = static_cast<R>(a);
@@ -943,8 +944,9 @@ int tdmd_fm_eam(tdmd_fm* F, int32_t nrho, double drho, int32_t nr, double dr, do
     sd.rphi.assign(static_cast<size_t>(nr), 0.0);
     int rc = eam_tables_create(&F->tables, F->precision, sd);
     if (rc) return rc;
-    if ((rc = fm_alloc(&F->d_gcoef, 4 * static_cast<size_t>(niF) + 8 * static_cast<size_t>(niR))))
-      return rc;
+    const size_t ng = 4 * static_cast<size_t>(niF) + 8 * static_cast<size_t>(niR);
+    if ((rc = fm_alloc(&F->d_gcoef, ng))) return rc;
+    if ((rc = tdmd_fill_u32(F->d_gcoef, 0u, 2 * ng, stream))) return rc;
     F->nrho = nrho;
     F->nr = nr;
     F->drho = drho;
@@ -954,11 +956,12 @@ int tdmd_fm_eam(tdmd_fm* F, int32_t nrho, double drho, int32_t nr, double dr, do
   const bool mixed = F->precision == TDMD_MIXED;
   // FD-Hermite coefficients from the knot values, and the kernels' quads
   const dim3 gc((std::max(niF, niR) + 255) / 256, 3);
+  double* const clear = d_grad ? F->d_gcoef : nullptr;
   if (mixed)
-    k_fm_build_coeffs<float><<<gc, 256, 0, s>>>(d_values, nrho, drho, nr, dr, F->d_gcoef,
+    k_fm_build_coeffs<float><<<gc, 256, 0, s>>>(d_values, nrho, drho, nr, dr, clear,
                                                 static_cast<float4*>(F->tables->d_coeff));
   else
-    k_fm_build_coeffs<double><<<gc, 256, 0, s>>>(d_values, nrho, drho, nr, dr, F->d_gcoef,
+    k_fm_build_coeffs<double><<<gc, 256, 0, s>>>(d_values, nrho, drho, nr, dr, clear,
                                                  static_cast<double4*>(F->tables->d_coeff));
   TDMD_LAUNCH_CHECK();
   // forward: density, embedding, forces (the drop-in EAM path)

@@ -203,3 +203,24 @@ def test_fm_adam_fits_reduce_the_loss():
     say(f"  EAM fit loss {losses[0]:.4e} -> {losses[-1]:.4e}")
     assert losses[-1] < 0.1 * losses[0]
     fm.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_fm_coef_grad_outlives_a_loss_only_call(prec):
+    # The coefficient gradients are the last gradient's, whatever losses were
+    # asked for since (a line search between two gradients).
+    import torch
+
+    say("fm coef grad after a loss", prec)
+    base, snaps = snapshots(n=1)
+    t, values, grid, (F, rho, phi) = eam_case(500)
+    fm = fitting.ForceMatchSet(base.lo, base.hi, snaps, grid.cutoff, prec)
+    fm.set_targets(np.zeros((1, base.natoms, 3)))
+    v = torch.tensor(values, dtype=torch.float64, device="cuda")
+    fm.eam(v, grid)
+    before = fm.eam_coef_grad(grid)
+    fm.eam(1.01 * v, grid, want_grad=False)
+    assert np.abs(before).max() > 0
+    assert np.array_equal(fm.eam_coef_grad(grid), before)
+    fm.close()
