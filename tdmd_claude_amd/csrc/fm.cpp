@@ -7,8 +7,9 @@
 //
 // Layout: the snapshots are one concatenated system of nsnap * natoms atoms
 // (AoS FP64 positions) sharing one box; each snapshot's full CSR list is
-// built once at creation with global indices, and beside it the half list
-// (neighbours j > i), so every pass is a single launch over all snapshots.
+// built once at creation with global indices, so every pass is a single launch
+// over all snapshots. The half list (neighbours j > i) beside it and the EAM
+// adjoint's records are built by the first call whose passes read them.
 // Rows are read by eight lanes side by side (csr_rows.hpp).
 //
 // Adjoint (ordered pairs i -> j, d = x_i - x_j, u = d / r, g = F - T):
@@ -50,13 +51,14 @@ struct tdmd_fm {
   int natoms = 0, nsnap = 0, ntot = 0;
   tdmd_box box{};
   double r_list = 0;
-  double r_min = 0;            // shortest listed pair
+  int64_t npairs = 0;          // listed, ordered
+  double r_min = 0;            // shortest listed pair (with the half list)
   double* d_pos = nullptr;     // [ntot][3]
   int32_t* d_cnt = nullptr;    // [ntot]
   int32_t* d_off = nullptr;    // [ntot]
-  int32_t* d_hcnt = nullptr;   // [ntot] half list: neighbours j > i
+  int32_t* d_hcnt = nullptr;   // [ntot] half list: neighbours j > i (fm_half_list)
   int32_t* d_hoff = nullptr;   // [ntot]
-  int32_t* d_hnbr = nullptr;   // [total / 2]
+  int32_t* d_hnbr = nullptr;   // [npairs / 2]
   int32_t* d_nbr = nullptr;    // [total]
   int32_t* d_types = nullptr;  // [ntot], all 1
   double* d_target = nullptr;  // [ntot][3]
@@ -552,25 +554,34 @@ __global__ void k_fm_coef_grad(const double* __restrict__ gcoef, int nrho, doubl
   out[m] = v;
 }
 
-// Rows from the snapshots' local indices to global ones, the half list's
-// counts, and *r2_min: the shortest pair's r^2 (non-negative doubles order as
-// their bits). One wavefront per row.
+// Rows from the snapshots' local indices to global ones. One wavefront per row.
 __global__ void __launch_bounds__(kBlock)
 k_fm_rows(int32_t* __restrict__ nbr, const int32_t* __restrict__ off,
-          const int32_t* __restrict__ cnt, int ntot, int natoms, const double* __restrict__ pos,
-          PairBox box, int32_t* __restrict__ hcnt, unsigned long long* r2_min) {
+          const int32_t* __restrict__ cnt, int ntot, int natoms) {
+  const int64_t row = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) >> 6;
+  if (row >= ntot) return;
+  const int i = static_cast<int>(row);
+  const int shift = i / natoms * natoms;
+  const int o = off[i], c = cnt[i];
+  for (int q = threadIdx.x & 63; q < c; q += kWave) nbr[o + q] += shift;
+}
+
+// The half list's counts, and *r2_min: the shortest pair's r^2 (non-negative
+// doubles order as their bits). One wavefront per row.
+__global__ void __launch_bounds__(kBlock)
+k_fm_half_counts(const int32_t* __restrict__ nbr, const int32_t* __restrict__ off,
+                 const int32_t* __restrict__ cnt, int ntot, const double* __restrict__ pos,
+                 PairBox box, int32_t* __restrict__ hcnt, unsigned long long* r2_min) {
   const int64_t row = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) >> 6;
   if (row >= ntot) return;
   const int lane = threadIdx.x & 63;
   const int i = static_cast<int>(row);
-  const int shift = i / natoms * natoms;
   const int o = off[i], c = cnt[i];
   const Neighbour a = neighbour_at(pos, i);
   int nh = 0;
   double r2 = __builtin_huge_val();
   for (int q = lane; q < c; q += kWave) {
-    const int j = nbr[o + q] + shift;
-    nbr[o + q] = j;
+    const int j = nbr[o + q];
     nh += j > i ? 1 : 0;
     const Neighbour b = neighbour_at(pos, j);
     const double dx = image(a.x - b.x, box.size[0], box.half[0]);
@@ -634,6 +645,48 @@ int fm_alloc(T** p, size_t n) {
   return rc;
 }
 
+// The half list and the shortest pair, for the passes over unordered pairs.
+int fm_half_list(tdmd_fm* F, hipStream_t s) {
+  if (F->d_hnbr) return TDMD_OK;
+  const int N = F->ntot;
+  int32_t *cnt = nullptr, *off = nullptr, *nbr = nullptr;
+  char* work = nullptr;
+  size_t sb = 0;
+  double r2 = __builtin_huge_val();
+  auto build = [&]() -> int {
+    int rc = tdmd_scan_workspace_bytes(N, &sb);
+    if (rc || (rc = fm_alloc(&cnt, N)) || (rc = fm_alloc(&off, N)) ||
+        (rc = fm_alloc(&nbr, static_cast<size_t>(F->npairs / 2 + 1))) ||
+        (rc = fm_alloc(&work, sb)))
+      return rc;
+    const int rows = grid_for(N, kBlock / kWave);
+    TDMD_HIP_TRY(hipMemcpyAsync(F->d_scalars, &r2, sizeof(r2), hipMemcpyHostToDevice, s));
+    k_fm_half_counts<<<rows, kBlock, 0, s>>>(F->d_nbr, F->d_off, F->d_cnt, N, F->d_pos,
+                                             make_pair_box(make_devbox(F->box)), cnt,
+                                             reinterpret_cast<unsigned long long*>(F->d_scalars));
+    TDMD_LAUNCH_CHECK();
+    if ((rc = tdmd_scan_exclusive_i32(cnt, off, N, nullptr, work, s))) return rc;
+    k_fm_half<<<rows, kBlock, 0, s>>>(F->d_nbr, F->d_off, F->d_cnt, N, off, nbr);
+    TDMD_LAUNCH_CHECK();
+    TDMD_HIP_TRY(hipMemcpyAsync(&r2, F->d_scalars, sizeof(r2), hipMemcpyDeviceToHost, s));
+    TDMD_HIP_TRY(hipStreamSynchronize(s));
+    return TDMD_OK;
+  };
+  const int rc = build();
+  if (rc) (void)hipStreamSynchronize(s);
+  if (work) (void)hipFree(work);
+  if (rc) {
+    for (int32_t* p : {cnt, off, nbr})
+      if (p) (void)hipFree(p);
+    return rc;
+  }
+  F->r_min = r2 < F->r_list * F->r_list ? std::sqrt(r2) : 0.0;
+  F->d_hcnt = cnt;
+  F->d_hoff = off;
+  F->d_hnbr = nbr;
+  return TDMD_OK;
+}
+
 // The adjoint passes: coefficient gradients in F->d_gcoef (cleared before).
 template <class R>
 int fm_eam_adjoint(tdmd_fm* F, hipStream_t s) {
@@ -669,10 +722,11 @@ int fm_eam_adjoint(tdmd_fm* F, hipStream_t s) {
       return TDMD_OK;
     }
   }
+  int rc = fm_half_list(F, s);
+  if (rc) return rc;
   k_fm_eam_lambda<R><<<row_grid(N, false), kBlock, 0, s>>>(rec, F->d_nbr, F->d_off, F->d_cnt, N,
                                                            box, t, quads);
   TDMD_LAUNCH_CHECK();
-  int rc;
   const size_t lf = 3 * niF * sizeof(double);
   if (lf <= lmax) {
     if ((rc = allow(reinterpret_cast<const void*>(&k_fm_eam_embed<R, true>), lf))) return rc;
@@ -732,9 +786,7 @@ int tdmd_fm_create(tdmd_fm** out, int32_t precision, const tdmd_box* box, int32_
   int rc = 0;
   if ((rc = fm_alloc(&F->d_pos, 3 * static_cast<size_t>(N))) ||
       (rc = fm_alloc(&F->d_cnt, N)) || (rc = fm_alloc(&F->d_off, N)) ||
-      (rc = fm_alloc(&F->d_hcnt, N)) || (rc = fm_alloc(&F->d_hoff, N)) ||
       (rc = fm_alloc(&F->d_types, N)) || (rc = fm_alloc(&F->d_target, 3 * static_cast<size_t>(N))) ||
-      (rc = fm_alloc(&F->d_rec, 8 * static_cast<size_t>(N))) ||
       (rc = fm_alloc(reinterpret_cast<char**>(&F->d_force), 3 * rsz * N)) ||
       (rc = fm_alloc(&F->d_rho, N)) ||
       (rc = fm_alloc(reinterpret_cast<char**>(&F->d_fp), rsz * N)) ||
@@ -804,9 +856,8 @@ int tdmd_fm_create(tdmd_fm** out, int32_t precision, const tdmd_box* box, int32_
     e = hipMemcpy(hm, meta, 8, hipMemcpyDeviceToHost);
     if (e != hipSuccess) rc = hip_fail(e, "hipMemcpy", __FILE__, __LINE__);
   }
-  const size_t total = static_cast<size_t>(std::max(hm[0], 1));
-  if (!rc && !(rc = fm_alloc(&F->d_nbr, total)) &&
-      !(rc = fm_alloc(&F->d_hnbr, total / 2 + 1))) {
+  F->npairs = hm[0];
+  if (!rc && !(rc = fm_alloc(&F->d_nbr, static_cast<size_t>(std::max(hm[0], 1))))) {
     (void)hipMemset(meta + 2, 0, 4);  // overflow: cannot happen, the rows were counted
     for (int s = 0; s < nsnap && !rc; ++s)
       rc = cells(s, [&](const double* ps, size_t a0, int32_t* c, int32_t* o, int32_t* a, int32_t* k) {
@@ -814,25 +865,11 @@ int tdmd_fm_create(tdmd_fm** out, int32_t precision, const tdmd_box* box, int32_
                                F->d_cnt + a0, hm[1], meta + 2, nullptr);
       });
     if (!rc) {
-      const double none = __builtin_huge_val();
-      e = hipMemcpy(F->d_scalars, &none, sizeof(none), hipMemcpyHostToDevice);
-      if (e != hipSuccess) rc = hip_fail(e, "hipMemcpy", __FILE__, __LINE__);
-      const int rows = grid_for(N, kBlock / kWave);
-      k_fm_rows<<<rows, kBlock>>>(F->d_nbr, F->d_off, F->d_cnt, N, natoms, F->d_pos,
-                                  make_pair_box(make_devbox(*box)), F->d_hcnt,
-                                  reinterpret_cast<unsigned long long*>(F->d_scalars));
-      if (!rc) rc = tdmd_scan_exclusive_i32(F->d_hcnt, F->d_hoff, N, nullptr, swork, nullptr);
-      k_fm_half<<<rows, kBlock>>>(F->d_nbr, F->d_off, F->d_cnt, N, F->d_hoff, F->d_hnbr);
-      k_fm_records<<<grid_for(N), kBlock>>>(F->d_pos, N, reinterpret_cast<FmRec*>(F->d_rec));
+      k_fm_rows<<<grid_for(N, kBlock / kWave), kBlock>>>(F->d_nbr, F->d_off, F->d_cnt, N, natoms);
       e = hipGetLastError();
+      if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
       if (e != hipSuccess) rc = hip_fail(e, "fm_create rows", __FILE__, __LINE__);
     }
-  }
-  if (!rc) {
-    double r2 = 0.0;  // (waits for the launches above)
-    e = hipMemcpy(&r2, F->d_scalars, sizeof(r2), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) rc = hip_fail(e, "hipMemcpy", __FILE__, __LINE__);
-    F->r_min = r2 < r_cut * r_cut ? std::sqrt(r2) : 0.0;
   }
   for (void* p : {static_cast<void*>(cc), static_cast<void*>(co), static_cast<void*>(ca),
                   static_cast<void*>(ac), static_cast<void*>(meta),
@@ -952,6 +989,12 @@ int tdmd_fm_eam(tdmd_fm* F, int32_t nrho, double drho, int32_t nr, double dr, do
     F->drho = drho;
     F->dr = dr;
     F->cutoff = cutoff;
+  }
+  if (!F->d_rec) {
+    const int rc = fm_alloc(&F->d_rec, 8 * static_cast<size_t>(N));
+    if (rc) return rc;
+    k_fm_records<<<grid_for(N), kBlock, 0, s>>>(F->d_pos, N, reinterpret_cast<FmRec*>(F->d_rec));
+    TDMD_LAUNCH_CHECK();
   }
   const bool mixed = F->precision == TDMD_MIXED;
   // FD-Hermite coefficients from the knot values, and the kernels' quads

@@ -224,3 +224,54 @@ def test_fm_coef_grad_outlives_a_loss_only_call(prec):
     assert np.abs(before).max() > 0
     assert np.array_equal(fm.eam_coef_grad(grid), before)
     fm.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_fm_set_holds_what_its_calls_read(prec):
+    # Device memory of a set after each kind of call: the list and 84 bytes an
+    # atom (FP64 100) at creation and for Morse, 64 more an atom for EAM, the half
+    # list only for the gradient passes over unordered pairs (FP64 here); and the
+    # gradient of a set that has been used otherwise before. Slack for the
+    # allocator's granules and the tables: a quarter of the half list's size.
+    import torch
+
+    say("fm memory", prec)
+    base, snaps = snapshots(n=2, cells=8)
+    snaps = np.concatenate([snaps] * 100)
+    t, values, grid, _ = eam_case(500)
+    v = torch.tensor(values, dtype=torch.float64, device="cuda")
+    _ = torch.empty_like(v), torch.empty_like(v)
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    small = fitting.ForceMatchSet(base.lo, base.hi, snaps[:1], RC_MORSE, prec)
+    small.set_targets(np.zeros(snaps[:1].shape))
+    small.morse(MORSE, RC_MORSE)
+    small.eam(v, grid)  # the runtime's own allocations
+    small.close()
+    start = free()
+    fm = fitting.ForceMatchSet(base.lo, base.hi, snaps, RC_MORSE, prec)
+    fm.set_targets(np.zeros(snaps.shape))
+    n, half = fm.ntot, 2 * fm.npairs()
+    own = 4 * fm.npairs() + (84 if prec == "mixed" else 100) * n
+    slack = half // 4
+    assert half > 50e6
+    fm.morse(MORSE, RC_MORSE)
+    assert start - free() < own + slack
+    fm.eam(v, grid, want_grad=False)
+    assert start - free() < own + 64 * n + slack
+    G = fm.eam(v, grid)[1].cpu().numpy()
+    used = start - free()
+    if prec == "mixed":
+        assert used < own + 64 * n + slack
+    else:
+        assert used < own + 72 * n + half + slack
+    fm.close()
+    fm = fitting.ForceMatchSet(base.lo, base.hi, snaps, RC_MORSE, prec)
+    fm.set_targets(np.zeros(snaps.shape))
+    G0 = fm.eam(v, grid)[1].cpu().numpy()
+    assert np.abs(G - G0).max() < (1e-10 if prec == "fp64" else 1e-5) * np.abs(G0).max()
+    fm.close()
