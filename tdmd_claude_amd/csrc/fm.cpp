@@ -273,18 +273,10 @@ k_fm_residual(const R* __restrict__ f, const R* __restrict__ fp, const double* _
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
-// 1 / r to FP64 rounding: as pair_r has it, or its float seed and one Newton
-// step (relative error ~1e-14).
-__device__ __forceinline__ double inverse(const PairR<double>& p) { return p.rinv; }
-__device__ __forceinline__ double inverse(const PairR<float>& p) {
-  const double y = static_cast<double>(p.rinv);
-  return fma(y, fma(-p.r, y, 1.0), y);
-}
-
 // w_ij = -2 (g_i - g_j) . d_ij / r_ij
 __device__ __forceinline__ double fm_weight(const FmRec& a, const FmRec& b, double dx, double dy,
-                                            double dz, double rinv) {
-  return -2.0 * ((a.gx - b.gx) * dx + (a.gy - b.gy) * dy + (a.gz - b.gz) * dz) * rinv;
+                                            double dz, double r) {
+  return -2.0 * ((a.gx - b.gx) * dx + (a.gy - b.gy) * dy + (a.gz - b.gz) * dz) / r;
 }
 
 // lam_i = sum_j w_ij rho'(r_ij) over full rows, left in rec[i].mu.
@@ -314,7 +306,7 @@ k_fm_eam_lambda(FmRec* rec, const int32_t* __restrict__ nbr, const int32_t* __re
         R x;
         const int k = spline_locate<R>(t.r, pr.r, &x);
         const R drho = quad_deriv<R>(quads[t.rho_at(0) + k], x);
-        lam = fma(fm_weight(a, b, dx, dy, dz, inverse(pr)), static_cast<double>(drho), lam);
+        lam = fma(fm_weight(a, b, dx, dy, dz, pr.r), static_cast<double>(drho), lam);
       }
     });
     lam = row_sum(lam);
@@ -401,7 +393,7 @@ k_fm_eam_hist(const FmRec* __restrict__ rec, const int32_t* __restrict__ nbr,
         const PairR<R> pr = pair_r<R>(r2);
         R x;
         const int k = spline_locate<R>(t.r, pr.r, &x);
-        const double w = fm_weight(a, b, dx, dy, dz, inverse(pr));
+        const double w = fm_weight(a, b, dx, dy, dz, pr.r);
         const double td = static_cast<double>(x);
         if (kPhi) {
           add(0, k, w);
@@ -471,7 +463,7 @@ k_fm_eam_adjoint_f32(const FmRec* __restrict__ rec, const int32_t* __restrict__ 
         float t;
         const int q = spline_locate<float>(tab.r, pr.r, &t);
         const float drho = quad_deriv<float>(quads[tab.rho_at(0) + q], t);
-        const double w = fm_weight(a, b, dx, dy, dz, inverse(pr));
+        const double w = fm_weight(a, b, dx, dy, dz, pr.r);
         const double hw = 0.5 * w;  // the two orderings of the pair give w
         const double P = static_cast<double>(static_cast<float>(a.fp) + static_cast<float>(b.fp));
         const double td = static_cast<double>(t);
