@@ -552,7 +552,11 @@ int first_build(tdmd_sched* S) {
       for (const BoxGeo& b : S->h_boxes) inv = std::min(inv, b.inv_cs[d]);
     cells /= inv * S->r_list;
   }
-  S->g.list_teams = list_teams(cells * (maxc + 1));
+  const int teams = list_teams(cells * (maxc + 1));
+  if (teams != S->g.list_teams) {
+    drop_graphs(S);  // captured graphs hold it
+    S->g.list_teams = teams;
+  }
   rc = S->eng->fill_pass(s);
   if (rc) return rc;
   ++S->host_rebuilds;

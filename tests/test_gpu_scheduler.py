@@ -862,3 +862,37 @@ def test_rebuild_grids_of_several_schedulers_fit_the_chip(n, policy):
                                                          split_rebuild=True))
         assert sched.rebuild_barrier() == 0
         sched.close()
+
+
+def _blob(cells, L, seed=5):
+    """A crystal of `cells` unit cells in a corner of a box of edge L."""
+    s = I.fcc_lattice(*cells, 3.615)
+    s.hi = s.lo + L
+    s.pos = s.pos + 0.5
+    I.init_velocities(s, 900.0, seed)
+    return s
+
+
+def test_reupload_of_another_density_matches_a_fresh_scheduler():
+    # Captured graphs hold how a list search's workgroup is divided, which goes by
+    # the longest row: after 4,096 atoms spread over the box, the same atoms as a
+    # crystal in its corner (rows of 86 in a capacity of 88, with a shell at the
+    # cutoff) run as in a fresh scheduler, bit for bit. (17 steps: an even number
+    # of exchanges of the record buffers, so that the graphs are found again.)
+    blob = _blob((8, 16, 8), 68.7)
+    g = np.stack(np.meshgrid(*[np.arange(16)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    spread = I.System(lo=blob.lo, hi=blob.hi, pos=(g + 0.5) * 68.7 / 16, vel=blob.vel,
+                      types=blob.types, ids=blob.ids, masses=blob.masses)
+    cfg = FastPipelineConfig(precision="fp64", rebuild_every=4, r_skin=0.785, max_neighbors=88,
+                             cell_pct=150)
+    morse = MORSE_CU[:3] + (5.715,)
+    say("re-upload of another density", blob.natoms)
+    sched = FastPipelineScheduler.for_system(spread, morse, cfg)
+    sched.run_until(17)
+    sched.upload_system(blob)
+    fresh = FastPipelineScheduler.for_system(blob, morse, cfg)
+    for x in (sched, fresh):
+        x.run_until(17)
+    assert all(np.array_equal(a, b) for a, b in zip(sched.download(), fresh.download()))
+    sched.close()
+    fresh.close()
