@@ -1131,9 +1131,10 @@ __device__ __forceinline__ float pre_r2(const int4& mj, const int4& mi, const Pr
 // stencil entry t's cell range and image, shared by shuffles; each cell's
 // candidates are then tested 32 at a time, and a hit's place in the row is
 // its rank among the hits in candidate order (ballot, then a prefix count):
-// near entries go to the front and shell entries to the back; after a
-// workgroup-scope fence (this wave's row stores complete before it reads them
-// back) the shell block is moved behind the near block and the row padded.
+// near entries go to the front and shell entries to the back, from the row's
+// end down; after a workgroup-scope fence (this wave's row stores complete
+// before it reads them back) the shell block is moved behind the near block, in
+// increasing index, and the row padded.
 // Every lane of the wave runs the loop (the ballots and shuffles need
 // them); `act` is false for a half with no atom, whose i is any valid atom.
 template <bool kCount, class Mir>
@@ -1249,15 +1250,33 @@ __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArg
     }
   }
   if constexpr (kCount) return act ? count : 0;
-  // the row stores above are complete before the shell entries are read back
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  auto stored = [] {  // this wave's stores, before its other lanes read them
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  };
+  stored();
+  const int gap = cap - nn - nf;  // [nn, cap - nf), the shell at [cap - nf, cap)
+  const bool full = act && nf > gap;  // source and destination overlap
+  if (__any(full)) {
+    // turned round in place first, then down by the gap, 32 at a time
+    if (full)
+      for (int q = l; q < nf / 2; q += 32) {
+        const size_t x = ell(i, cap - 1 - q, cap), y = ell(i, cap - nf + q, cap);
+        const int32_t v = nbr[x];
+        nbr[x] = nbr[y];
+        nbr[y] = v;
+      }
+    stored();
+    for (int q0 = 0; __any(full && q0 < nf); q0 += 32) {
+      const bool move = full && gap > 0 && q0 + l < nf;
+      const int32_t v = move ? nbr[ell(i, cap - nf + q0 + l, cap)] : 0;
+      stored();
+      if (move) nbr[ell(i, nn + q0 + l, cap)] = v;
+    }
+  }
   if (act) {
-    // Shell entries sit at [cap - nf, cap); the gap [nn, cap - nf) has room
-    // for the m that move (source and destination ranges are disjoint).
-    const int gap = cap - nn - nf;
-    const int m = nf < gap ? nf : gap;
-    for (int q = l; q < m; q += 32) nbr[ell(i, nn + q, cap)] = nbr[ell(i, cap - 1 - q, cap)];
+    if (!full)
+      for (int q = l; q < nf; q += 32) nbr[ell(i, nn + q, cap)] = nbr[ell(i, cap - 1 - q, cap)];
     const int n = nn + nf;  // == min(count, cap)
     if (l == 0) {
       cnt[i] = n;

@@ -896,3 +896,28 @@ def test_reupload_of_another_density_matches_a_fresh_scheduler():
     assert all(np.array_equal(a, b) for a, b in zip(sched.download(), fresh.download()))
     sched.close()
     fresh.close()
+
+
+@pytest.mark.parametrize("prec,cells,L,pct", [
+    ("fp64", (5, 5, 5), None, 0),  # three cells narrower than r_list
+    ("mixed", (10, 10, 10), None, 300),  # cells over the staged candidates
+    ("fp64", (10, 10, 10), None, 300),
+    ("fp64", (6, 6, 6), 150.0, 0),  # a droplet in mostly empty cells
+    ("mixed", (6, 6, 6), 150.0, 0)])
+def test_rows_do_not_depend_on_the_capacity_left(prec, cells, L, pct):
+    # Rows of 86 slots in a capacity of 88, 104 and 160, by the fused rebuild and by
+    # separate kernels: the same rows in the same order, so the same bits, with
+    # pairs of the skin shell entering the cutoff between rebuilds.
+    s = _blob(cells, L) if L else I.fcc_lattice(*cells, 3.615)
+    I.init_velocities(s, 400.0, 5)  # no atom gets an 89th
+    say("full rows", prec, s.natoms, pct)
+    out = []
+    for cap in (88, 104, 160):
+        for split in (False, True):
+            cfg = FastPipelineConfig(precision=prec, rebuild_every=8, max_neighbors=cap,
+                                     cell_pct=pct, split_rebuild=split, r_skin=0.785)
+            sched = FastPipelineScheduler.for_system(s, MORSE_CU[:3] + (5.715,), cfg)
+            sched.run_until(24)
+            out.append(sched.download())
+            sched.close()
+    assert all(np.array_equal(a, b) for o in out[1:] for a, b in zip(o, out[0]))
