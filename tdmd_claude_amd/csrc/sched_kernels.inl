@@ -1303,7 +1303,8 @@ __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArg
 //    which the whole workgroup waits for: a wider band costs time). That error,
 //    with S = 2 |a| + r_list >= |a| + |b| near a radius: the offsets' rounding,
 //    2^-22 r_list S; the squares', products' and sum's, 6.5 2^-24 S^2; and a
-//    unit of the records on each axis, 3.5 r_list units.
+//    unit of the records on each axis, 3.5 r_list units (open axes are taken in
+//    units of two, so that an atom far out keeps its side of the centre).
 // 2. Half a wavefront turns a row's masks into the list of its candidates, near
 //    ones first: a popcount prefix over the words, then each lane its own bits.
 // 3. It writes the row, one quad of slots a lane.
@@ -1413,7 +1414,7 @@ __device__ __forceinline__ int nlist_cells(const StepArgs& a, const GridArgs& g,
     const MirrorParams& mp = mp_of<Mir>(a, h0);
     bool images = false, flat = false;  // flat: offsets carry the image
     double ctr[3] = {0.0, 0.0, 0.0};
-    int ref[3] = {0, 0, 0};  // the centre as a record
+    int ref[3] = {0, 0, 0}, half[3] = {0, 0, 0};  // the centre as a record
     float u[3] = {0.0f, 0.0f, 0.0f}, unit_err = 0.0f;
     auto shift = [&](int img, int d) {
       const int s = (img >> (2 * d)) & 3;
@@ -1436,15 +1437,21 @@ __device__ __forceinline__ int nlist_cells(const StepArgs& a, const GridArgs& g,
           // half a cell and r_list stay within half the box
           flat = flat && (!mp.periodic[d] || cs * cs >= r_list_sq * 1.00001);
           u[d] = static_cast<float>(mp.unit[d]);
-          unit_err = fmaxf(unit_err, 4.0f * rl * u[d]);
-          const double o = (ctr[d] - at[d]) / mp.unit[d];
-          const int4 r0 = static_cast<const int4*>(a.M)[h0];
-          ref[d] = static_cast<int>(static_cast<unsigned>(d == 0 ? r0.x : d == 1 ? r0.y : r0.z) +
-                                    static_cast<unsigned>(static_cast<int>(
-                                        fmin(fmax(o, -2147483647.0), 2147483647.0))));
+          // (an open axis: 0 to 2^30 units, a periodic one mod 2^32)
+          ref[d] = MirrorFixed::enc1(ctr[d], mp.lo[d], mp.q[d]);
         } else {
           // FP64 itself resolves 1e-7 r_list there
           flat = flat && (fabs(ctr[d]) + mp.L[d]) * (fabs(ctr[d]) + mp.L[d]) < 1e16 * r_list_sq;
+        }
+      }
+      if constexpr (Mir::kFixed) {
+        for (int d = 0; d < 3; ++d) {
+          // an open axis in units of two: an atom far out may be more than 2^31
+          // units from the centre
+          half[d] = flat && !mp.periodic[d] ? 1 : 0;
+          ref[d] >>= half[d];
+          u[d] = half[d] ? 2.0f * u[d] : u[d];
+          unit_err = fmaxf(unit_err, 4.0f * rl * u[d]);
         }
       }
     }
@@ -1467,9 +1474,9 @@ __device__ __forceinline__ int nlist_cells(const StepArgs& a, const GridArgs& g,
         float o[3];
         if constexpr (Mir::kFixed) {
           if (flat) {
-            o[0] = static_cast<float>(MirrorFixed::wdiff(v.x, ref[0])) * u[0];
-            o[1] = static_cast<float>(MirrorFixed::wdiff(v.y, ref[1])) * u[1];
-            o[2] = static_cast<float>(MirrorFixed::wdiff(v.z, ref[2])) * u[2];
+            o[0] = static_cast<float>(MirrorFixed::wdiff(v.x >> half[0], ref[0])) * u[0];
+            o[1] = static_cast<float>(MirrorFixed::wdiff(v.y >> half[1], ref[1])) * u[1];
+            o[2] = static_cast<float>(MirrorFixed::wdiff(v.z >> half[2], ref[2])) * u[2];
           } else {
             o[0] = __int_as_float(v.x);
             o[1] = __int_as_float(v.y);

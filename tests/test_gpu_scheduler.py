@@ -7,6 +7,7 @@ agree to rounding over short runs; in mixed precision forces agree to 1e-5
 of the RMS force.
 """
 import ctypes as C
+import functools
 
 import numpy as np
 import pytest
@@ -921,3 +922,62 @@ def test_rows_do_not_depend_on_the_capacity_left(prec, cells, L, pct):
             out.append(sched.download())
             sched.close()
     assert all(np.array_equal(a, b) for o in out[1:] for a, b in zip(o, out[0]))
+
+
+FORCE_CASES = {**LIST_CASES,
+               # a slab of each open axis near the end of the range lo - 2 W
+               "far out": (800, (30.0, 40.0, 50.0), (0, 1, 0))}
+WEAK_MORSE = (0.01, 0.5, 2.8, 6.0)
+
+
+def _brute_morse(pos, L, periodic, D, alpha, r0, rc):
+    f = np.zeros_like(pos)
+    for i in range(0, len(pos), 256):
+        d = pos[i:i + 256, None, :] - pos[None, :, :]
+        for a in range(3):
+            if periodic[a]:
+                d[..., a] -= L[a] * np.round(d[..., a] / L[a])
+        r = np.sqrt((d * d).sum(-1))
+        e = np.exp(-alpha * (r - r0))
+        g = np.where((r < rc) & (r > 0), 2.0 * D * alpha * (e * e - e) / np.maximum(r, 1e-300), 0.0)
+        f[i:i + 256] = (g[..., None] * d).sum(1)
+    return f
+
+
+@functools.lru_cache(maxsize=None)
+def _force_case(name):
+    """Positions (no pair planted at a radius), box and forces of a case."""
+    rng = np.random.Generator(np.random.PCG64(29))
+    n, L, periodic = FORCE_CASES[name]
+    pos = rng.uniform(0.0, np.array(L), size=(n, 3))
+    for d in range(3):
+        if not periodic[d]:
+            pos[: n // 8, d] += rng.uniform(-0.3, 0.3, size=n // 8) * L[d]
+        if not periodic[d] and name == "far out":
+            far = slice((d + 2) * n // 8, (d + 3) * n // 8)
+            pos[far, d] = rng.uniform(-1.99, -1.7, size=n // 8) * L[d]
+    ref = _brute_morse(pos, L, periodic, *WEAK_MORSE)
+    return pos, np.array(L), periodic, ref
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+@pytest.mark.parametrize("name", FORCE_CASES)
+def test_list_forces_by_kind_of_cell(name, prec):
+    # Forces from the lists of the first build and of a fused rebuild against all
+    # pairs in FP64: a Morse bond of -1.6e-3 eV/A at its cutoff and at most 0.12, so
+    # that any wrong neighbour shows (rms forces are 0.1-0.5). FP64: the order of
+    # ~100 terms. Mixed: the coordinates' units (at most 5e-8 A) and FP32 pair
+    # functions.
+    pos, L, periodic, ref = _force_case(name)
+    n = len(pos)
+    say("list forces,", name, prec, n)
+    s = I.System(lo=np.zeros(3), hi=L.copy(), pos=pos, vel=np.zeros_like(pos),
+                 types=np.ones(n, dtype=np.int32), ids=np.arange(1, n + 1, dtype=np.int32),
+                 masses=np.array([1.0, 63.546]), periodic=periodic)
+    sched = FastPipelineScheduler.for_system(
+        s, WEAK_MORSE, FastPipelineConfig(precision=prec, rebuild_every=1, r_skin=1.0, dt=1e-9))
+    for step in (0, 2):  # steps too short to change a force
+        sched.run_until(step)
+        f = sched.download()[2]
+        assert force_rel_err(f, ref) < (1e-9 if prec == "fp64" else 1e-5)
+    sched.close()
