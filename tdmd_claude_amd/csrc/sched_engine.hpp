@@ -333,10 +333,10 @@ struct Engine final : EngineBase {
     S->nb_force = lds ? nb_lds : S->nblocks * lanes;
   }
 
-  // Workgroups of the fused rebuild: a cell each up to 64, two each beyond (the
-  // rebuild of 864 atoms in 27 cells: 30.9 us with 27, 34.6 with 14; of 10,976
-  // in 216: 50.4 with 216, 45.7 with 108: a barrier costs more the more arrive
-  // at it); one a CU, which the list search's LDS fills; and by the atoms one per
+  // Workgroups of the fused rebuild: where the list is searched by cells, a cell
+  // each up to 64, two each beyond (the rebuild of 864 atoms in 27 cells: 30.9 us
+  // with 27, 34.6 with 14; of 10,976 in 216: 50.4 with 216, 45.7 with 108: a
+  // barrier costs more the more arrive at it); one a CU, which the list search's LDS fills; and by the atoms one per
   // 32 where every launch rebuilds, one per 1024 under the displacement policy
   // and above 131,072. Rebuilds that run at the same time (schedulers on streams
   // or in processes of their own) have to be resident together, or they wait for
@@ -350,6 +350,7 @@ struct Engine final : EngineBase {
     const int n = S->natoms;
     const bool few = S->cfg.rebuild_policy == TDMD_REBUILD_DISPLACEMENT || n > 131072;
     const int by_atoms = few ? (n + 1023) / 1024 : (n + 31) / 32;
+    if (S->g.list_lanes > 0) return std::max(1, std::min(ncu, by_atoms));
     const int cells = std::min(S->g.ncells, std::max(64, (S->g.ncells + 1) / 2));
     return std::max(1, std::min({ncu, by_atoms, cells}));
   }
@@ -681,8 +682,8 @@ struct Engine final : EngineBase {
     k_bin<Mir><<<gb, kBlock, 0, s>>>(S->a, S->g);
     k_cell_scan<<<1, 1024, 0, s>>>(S->a.flags, S->g);
     k_scatter<<<gb, kBlock, 0, s>>>(S->a, S->g);
-    k_order_permute<R, Mir><<<grid_for(S->g.ncells, kBlock / 64), kBlock, 0, s>>>(S->a, S->g,
-                                                                                  S->t);
+    k_order_permute<R, Mir><<<S->g.list_lanes > 0 ? gb : grid_for(S->g.ncells, kBlock / 64),
+                              kBlock, 0, s>>>(S->a, S->g, S->t);
     k_copyback<R, Mir><<<gb, kBlock, 0, s>>>(S->a, S->g, S->t);
     k_zero_cells<<<gc, kBlock, 0, s>>>(S->a.flags, S->g);
     S->launches += 6;
@@ -692,10 +693,18 @@ struct Engine final : EngineBase {
   // Counts (into *d_max) or rows of the sorted atoms.
   template <bool kCount>
   void nlist(hipStream_t s, int32_t* d_max) {
-    k_nlist_ell<kCount, Mir><<<std::min(256, (S->g.ncells + 1) / 2), kListBlock, 0, s>>>(
-        S->a, S->g, S->t, S->r_list * S->r_list, S->cutoff * S->cutoff,
-        kCount ? nullptr : const_cast<int32_t*>(S->a.nbr),
-        kCount ? nullptr : const_cast<int32_t*>(S->a.cnt), d_max);
+    auto go = [&](auto kernel, int grid, int block) {
+      kernel<<<grid, block, 0, s>>>(S->a, S->g, S->t, S->r_list * S->r_list,
+                                    S->cutoff * S->cutoff,
+                                    kCount ? nullptr : const_cast<int32_t*>(S->a.nbr),
+                                    kCount ? nullptr : const_cast<int32_t*>(S->a.cnt), d_max);
+    };
+    if (S->g.list_lanes == 0)
+      go(&k_nlist_ell<kCount, Mir>, std::min(256, (S->g.ncells + 1) / 2), kListBlock);
+    else if (S->g.list_lanes == 1)
+      go(&k_nlist_atoms<kCount, 1, Mir>, grid_for(S->natoms), kBlock);
+    else
+      go(&k_nlist_atoms<kCount, 32, Mir>, grid_for(32 * static_cast<int64_t>(S->natoms)), kBlock);
   }
   int fill_pass(hipStream_t s) override {
     const int gb = grid_for(S->natoms);

@@ -298,6 +298,7 @@ struct GridArgs {
   int images;  // 1: every periodic axis has >= 3 cells no smaller than r_list,
                // so a stencil entry's image is the minimum image of any pair
                // within r_list that it holds (batches: per box, BoxGeo)
+  int list_lanes;  // 0: the list search by cells; 1 or 32: by so many lanes an atom
   int list_teams;  // log2 of the list search's teams a workgroup, at most
   int32_t* ccount;         // [ncells] by rank; zero between rebuilds
   int32_t* cstart;         // [ncells + 1] by rank: cell r's slots [cstart[r], cstart[r + 1])

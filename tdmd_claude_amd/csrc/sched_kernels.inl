@@ -1017,6 +1017,18 @@ __device__ __forceinline__ void order_cell_wave(const GridArgs& g, int r, Put&& 
   }
 }
 
+// The same by a lane per atom of the scatter's order: for cells of few atoms,
+// where a wavefront per cell leaves most lanes idle.
+template <class Put>
+__device__ __forceinline__ void order_slot(const GridArgs& g, int s, Put&& put) {
+  const int v = g.sidx[s];
+  const int kv = g.orig[v], r = g.key[v];
+  const int start = g.cstart[r], end = g.cstart[r + 1];
+  int pos = start;
+  for (int c = start; c < end; ++c) pos += g.orig[g.sidx[c]] < kv ? 1 : 0;
+  put(v, pos);
+}
+
 // Atom o (old slot) to slot s of the scratch arrays, and its gather record.
 template <class R, class Mir>
 __device__ __forceinline__ void permute_atom(const StepArgs& a, const GridArgs& g,
@@ -1127,16 +1139,16 @@ __device__ __forceinline__ float pre_r2(const int4& mj, const int4& mi, const Pr
 // `cap` hits, and its true count is reported.
 //
 // nlist_atom_group: 32 lanes per atom, two atoms per wavefront, straight from
-// memory: for what nlist_cells leaves (below). Lane t < 27 of a group loads
-// stencil entry t's cell range and image, shared by shuffles; each cell's
-// candidates are then tested 32 at a time, and a hit's place in the row is
-// its rank among the hits in candidate order (ballot, then a prefix count):
-// near entries go to the front and shell entries to the back, from the row's
-// end down; after a workgroup-scope fence (this wave's row stores complete
-// before it reads them back) the shell block is moved behind the near block, in
-// increasing index, and the row padded.
-// Every lane of the wave runs the loop (the ballots and shuffles need
-// them); `act` is false for a half with no atom, whose i is any valid atom.
+// memory: for sparse systems (GridArgs::list_lanes) and what nlist_cells leaves
+// (below). Lane t < 27 of a group loads stencil entry t's cell range and image,
+// shared by shuffles; each cell's candidates are then tested 32 at a time, and a
+// hit's place in the row is its rank among the hits in candidate order (ballot,
+// then a prefix count): near entries go to the front and shell entries to the
+// back, from the row's end down; after a workgroup-scope fence (this wave's row
+// stores complete before it reads them back) the shell block is moved behind the
+// near block, in increasing index, and the row padded. Every lane of the wave
+// runs the loop (the ballots and shuffles need them); `act` is false for a half
+// with no atom, whose i is any valid atom.
 template <bool kCount, class Mir>
 __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArgs& g,
                                                 const PermArgs& p, int i,
@@ -1286,6 +1298,166 @@ __device__ __forceinline__ int nlist_atom_group(const StepArgs& a, const GridArg
     if (k < ((n + 7) & ~7)) nbr[ell(i, k, cap)] = i;
   }
   return act ? count : 0;
+}
+
+// nlist_atom: the same rows by one lane per atom, with a group of candidates'
+// loads in flight at a time, for more atoms than there are groups of lanes.
+template <bool kCount, class Mir>
+__device__ __forceinline__ int nlist_atom(const StepArgs& a, const GridArgs& g, const PermArgs& p,
+                                          int i, double r_list_sq, double near_sq, int32_t* nbr,
+                                          int32_t* cnt) {
+  using T = typename Mir::T;
+  constexpr int kG = Mir::kFixed ? 8 : 4;
+  const int cap = a.cap;
+  const double xi = p.px[i], yi = p.py[i], zi = p.pz[i];
+  const MirrorParams& mp = mp_of<Mir>(a, i);
+  const CellGrid cg = grid_of<Mir>(a, g, i);
+  int c[3];
+  cell_coords(cg, xi, yi, zi, c);
+  const size_t row =
+      27 * static_cast<size_t>(g.rank_of[cg.off + (c[2] * cg.n[1] + c[1]) * cg.n[0] + c[0]]);
+  const T* __restrict__ const M = static_cast<const T*>(a.M);
+  int4 mi_rec = make_int4(0, 0, 0, 0);
+  PreBounds pb{};
+  if constexpr (Mir::kFixed) {
+    mi_rec = M[i];
+    pb = pre_bounds(mp, r_list_sq, near_sq);
+  }
+  int count = 0, nn = 0, nf = 0;
+  int32_t* const to = kCount ? nullptr : nbr + ell(i, 0, cap);
+  auto slot = [&](int k) -> int32_t& { return to[(k >> 2) * 256 + (k & 3)]; };
+  // one copy of the search per image mode, so that a group's loads issue together
+  auto search = [&](auto with_images, auto iso_units) {
+    constexpr bool kImg = decltype(with_images)::value;
+    constexpr bool kIsoU = decltype(iso_units)::value;
+    for (int t = 0; t < 27; ++t) {
+      const int r = g.around[row + t];
+      const int start = g.cstart[r], end = g.cstart[r + 1];
+      const int img = kImg ? g.around_img[row + t] : 0;
+      auto shift = [&](int d) {
+        const int s = (img >> (2 * d)) & 3;
+        return s == 0 ? 0.0 : s == 1 ? mp.L[d] : -mp.L[d];
+      };
+      const double sx = shift(0), sy = shift(1), sz = shift(2);
+      auto r2_of = [&](double x, double y, double z) {
+        double dx = x - xi, dy = y - yi, dz = z - zi;
+        if constexpr (kImg) {
+          dx += sx;
+          dy += sy;
+          dz += sz;
+        } else {
+          dx = min_image(dx, mp.L[0], mp.hL[0], mp.periodic[0]);
+          dy = min_image(dy, mp.L[1], mp.hL[1], mp.periodic[1]);
+          dz = min_image(dz, mp.L[2], mp.hL[2], mp.periodic[2]);
+        }
+        return r2_unfused(dx, dy, dz);
+      };
+      for (int j0 = start; j0 < end; j0 += kG) {
+        T m[kG];
+#pragma unroll
+        for (int q = 0; q < kG; ++q) m[q] = M[min(j0 + q, end - 1)];
+        bool in[kG], near[kG];
+        if constexpr (Mir::kFixed) {
+          // (bitwise: no branch splits the group)
+          bool band[kG], any = false;
+#pragma unroll
+          for (int q = 0; q < kG; ++q) {
+            const float r2f = pre_r2<kIsoU>(m[q], mi_rec, pb);
+            const bool valid = (j0 + q < end) & (j0 + q != i);
+            in[q] = valid & (r2f < pb.lo_list);
+            near[q] = valid & (r2f < pb.lo_near);
+            band[q] = valid & (((r2f <= pb.hi_list) & !(r2f < pb.lo_list)) |
+                               ((r2f <= pb.hi_near) & !(r2f < pb.lo_near)));
+            any |= band[q];
+          }
+          if (any) {
+#pragma unroll
+            for (int q = 0; q < kG; ++q)
+              if (band[q]) {
+                const int j = j0 + q;
+                const double r2 = r2_of(p.px[j], p.py[j], p.pz[j]);
+                in[q] = r2 < r_list_sq;
+                near[q] = r2 < near_sq;
+              }
+          }
+        } else {
+#pragma unroll
+          for (int q = 0; q < kG; ++q) {
+            const double r2 = r2_of(m[q].x, m[q].y, m[q].z);
+            const bool valid = (j0 + q < end) & (j0 + q != i);
+            in[q] = valid & (r2 < r_list_sq);
+            near[q] = r2 < near_sq;
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < kG; ++q)
+          if (in[q]) {
+            if (!kCount && nn + nf < cap) {
+              if (near[q])
+                slot(nn++) = j0 + q;
+              else
+                slot(cap - 1 - nf++) = j0 + q;
+            }
+            ++count;
+          }
+      }
+    }
+  };
+  bool images;
+  if constexpr (Mir::kMB)
+    images = a.boxes[a.rep[i]].images != 0;
+  else
+    images = g.images != 0;
+  if (images)
+    pb.iso ? search(std::true_type{}, std::true_type{})
+           : search(std::true_type{}, std::false_type{});
+  else
+    pb.iso ? search(std::false_type{}, std::true_type{})
+           : search(std::false_type{}, std::false_type{});
+  if constexpr (!kCount) {
+    const int gap = cap - nn - nf;
+    if (nf > gap) {  // turned round in place first, then down by the gap
+      for (int q = 0; q < nf / 2; ++q) {
+        const int32_t v = slot(cap - 1 - q);
+        slot(cap - 1 - q) = slot(cap - nf + q);
+        slot(cap - nf + q) = v;
+      }
+      if (gap > 0)
+        for (int q = 0; q < nf; ++q) slot(nn + q) = slot(cap - nf + q);
+    } else {
+      for (int q = 0; q < nf; ++q) slot(nn + q) = slot(cap - 1 - q);
+    }
+    const int n = nn + nf;  // == min(count, cap)
+    cnt[i] = n;
+    a.cntn[i] = nn;
+    for (int k = n; k < ((n + 7) & ~7); ++k) slot(k) = i;
+  }
+  return count;
+}
+
+// The rows of all atoms by kLanes lanes (1 or 32) each, by `waves` wavefronts of
+// which this is `wave`. Returns the largest count this lane's rows had.
+template <bool kCount, int kLanes, class Mir>
+__device__ __forceinline__ int nlist_atoms(const StepArgs& a, const GridArgs& g, const PermArgs& p,
+                                           double r_list_sq, double near_sq, int32_t* nbr,
+                                           int32_t* cnt, int wave, int waves) {
+  const int lane = static_cast<int>(threadIdx.x & 63);
+  int most = 0;
+  if constexpr (kLanes == 1) {
+    for (int64_t i = 64 * static_cast<int64_t>(wave) + lane; i < a.natoms;
+         i += 64 * static_cast<int64_t>(waves))
+      most = max(most, nlist_atom<kCount, Mir>(a, g, p, static_cast<int>(i), r_list_sq, near_sq,
+                                               nbr, cnt));
+    return most;
+  }
+  for (int64_t b = 2 * static_cast<int64_t>(wave); b < a.natoms;
+       b += 2 * static_cast<int64_t>(waves)) {
+    const int i = static_cast<int>(b) + (lane >> 5);
+    const bool act = i < a.natoms;
+    most = max(most, nlist_atom_group<kCount, Mir>(a, g, p, act ? i : static_cast<int>(b), act,
+                                                   r_list_sq, near_sq, nbr, cnt));
+  }
+  return most;
 }
 
 // The rows of all cells, dealt to teams of wavefronts: the whole 1024-thread
@@ -1732,10 +1904,15 @@ static __global__ void __launch_bounds__(kBlock) k_scatter(StepArgs a, GridArgs 
   scatter_atom(g, i, g.cstart);
 }
 
-// One wavefront per cell.
+// One wavefront per cell, or one lane per atom with the searches by atoms.
 template <class R, class Mir>
 __global__ void __launch_bounds__(kBlock) k_order_permute(StepArgs a, GridArgs g, PermArgs t) {
   if (!a.flags[0]) return;
+  if (g.list_lanes > 0) {
+    const int s = blockIdx.x * kBlock + threadIdx.x;
+    if (s < a.natoms) order_slot(g, s, [&](int o, int to) { permute_atom<R, Mir>(a, g, t, o, to); });
+    return;
+  }
   const int r = blockIdx.x * (kBlock / 64) + static_cast<int>(threadIdx.x >> 6);
   if (r >= g.ncells) return;
   order_cell_wave(g, r, [&](int o, int s) { permute_atom<R, Mir>(a, g, t, o, s); });
@@ -1756,6 +1933,19 @@ k_nlist_ell(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double near_sq
   if (!kCount && !a.flags[0]) return;
   __shared__ ListLds L;
   const int count = nlist_cells<kCount, Mir>(a, g, t, r_list_sq, near_sq, nbr, cnt, L);
+  report_count<kCount>(a, count, maxcnt);
+}
+
+template <bool kCount, int kLanes, class Mir>
+__global__ void __launch_bounds__(kBlock)
+k_nlist_atoms(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double near_sq, int32_t* nbr,
+              int32_t* cnt, int32_t* maxcnt) {
+  if (!kCount && !a.flags[0]) return;
+  constexpr int kWaves = kBlock / 64;
+  const int count = nlist_atoms<kCount, kLanes, Mir>(
+      a, g, t, r_list_sq, near_sq, nbr, cnt,
+      static_cast<int>(blockIdx.x) * kWaves + static_cast<int>(threadIdx.x >> 6),
+      static_cast<int>(gridDim.x) * kWaves);
   report_count<kCount>(a, count, maxcnt);
 }
 
@@ -2170,8 +2360,11 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
     // one cell per wavefront, cells dealt to the workgroups wave by wave
     const int nw = gridDim.x * (kRebuildBlock / 64);
     const int wv = (threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-    for (int r = wv; r < g.ncells; r += nw)
-      order_cell_wave(g, r, [&](int o, int s) { permute_atom<R, Mir>(a, g, t, o, s); });
+    auto put = [&](int o, int s) { permute_atom<R, Mir>(a, g, t, o, s); };
+    if (g.list_lanes > 0)
+      for (int s = tid; s < N; s += nthr) order_slot(g, s, put);
+    else
+      for (int r = wv; r < g.ncells; r += nw) order_cell_wave(g, r, put);
     for (int r = tid; r < g.ncells; r += nthr) {
       g.ccount[r] = 0;
       g.cursor[r] = 0;
@@ -2181,7 +2374,14 @@ k_rebuild_fused(StepArgs a, GridArgs g, PermArgs t, double r_list_sq, double nea
   // the state's arrays back from the scratch ones, beside the list search,
   // which reads the scratch arrays and the records
   for (int s = tid; s < N; s += nthr) copyback_atom<R, Mir>(a, g, t, s);
-  const int count = nlist_cells<false, Mir>(a, g, t, r_list_sq, near_sq, nbr, cnt, lds.list);
+  const int wave = tid >> 6, waves = nthr >> 6;
+  int count;
+  if (g.list_lanes == 0)
+    count = nlist_cells<false, Mir>(a, g, t, r_list_sq, near_sq, nbr, cnt, lds.list);
+  else if (g.list_lanes == 1)
+    count = nlist_atoms<false, 1, Mir>(a, g, t, r_list_sq, near_sq, nbr, cnt, wave, waves);
+  else
+    count = nlist_atoms<false, 32, Mir>(a, g, t, r_list_sq, near_sq, nbr, cnt, wave, waves);
   report_count<false>(a, count, nullptr);
   if constexpr (Mir::kFixed) {
     if (a.stage_cap > 0) {  // halos of the staged passes, from the new rows

@@ -161,6 +161,47 @@ int staged_download(const tdmd_sched* S, double* const dst[3], size_t from, size
   return TDMD_OK;
 }
 
+// How the lists are searched (GridArgs::list_lanes): by cells where cells hold
+// enough atoms on average, else by atoms, as many lanes each as the rebuild's grid
+// gives them. A cell costs a team of the workgroup about the same whatever it
+// holds, so the search by cells is slow where they are nearly empty: vacuum around
+// a droplet, a gas. Rebuilds in us, by cells / 32 lanes / 1 lane, mixed, by random
+// atoms a cell:
+//                              8                 4                 2
+//   fixed        4,096    44 / 53 / 173     44 / 48 / 99      53 / 49 / 97
+//                64,000  116 / 210 / 180   151 / 208 / 129   223 / 206 / 124
+//               125,000  172 / 361 / 183   234 / 363 / 134   389 / 362 / 130
+//               262,144  294 / 672 / 195   445 / 678 / 150   765 / 672 / 152
+//                        (20: 273 / 681 / 306, 12: 282 / 677 / 244)
+//   displacement  4,096  231 / 606 / 164   386 / 605 / 90    615 / 590 / 89
+//                        (20: 208 / 794 / 303)
+//   split        32,768   67 / 103 / 115    89 / 107 / 90    142 / 118 / 99
+//   4,096 atoms of a solid in the middle of a box six times as wide, fixed:
+//   124 / 63 / 257; 262,144 in a box twice as wide: 907 / 683 / 328.
+// FP64 records in boxes of under three cells of r_list on a periodic axis are
+// searched from memory in any case, and by atoms faster (fixed, FP64: 500 atoms
+// 63 / 45 / 208, films of 57,600 atoms 311 / 235 / 391, 160,000 1012 / 815 / 377,
+// 500 boxes of 108 atoms 606 / 339 / 176).
+int list_lanes(const tdmd_sched* S) {
+  const int n = S->natoms;
+  const bool split = S->cfg.split_rebuild != 0;
+  const bool few = S->cfg.rebuild_policy == TDMD_REBUILD_DISPLACEMENT && !split;
+  const int by_atoms = !few && n <= (split ? 16384 : 65536) ? 32 : 1;
+  const int per_cell = by_atoms == 32        ? 2
+                       : few || n > 131072 ? 15
+                       : n > 32768         ? 7
+                                           : 4;
+  if (n < static_cast<int64_t>(per_cell) * S->g.ncells) return by_atoms;
+  if (S->cfg.precision == TDMD_MIXED && !S->cfg.mirror_fp64) return 0;
+  int64_t narrow = S->g.images ? 0 : n;
+  if (S->multibox) {
+    narrow = 0;
+    for (size_t b = 0; b < S->h_boxes.size(); ++b)
+      if (!S->h_boxes[b].images) narrow += S->rep_off[b + 1] - S->rep_off[b];
+  }
+  return 4 * narrow > n ? by_atoms : 0;
+}
+
 int sched_alloc(tdmd_sched* S) {
   const int N = S->natoms;
   const size_t fsz = S->cfg.precision == TDMD_MIXED ? sizeof(float) : sizeof(double);
@@ -304,6 +345,7 @@ int sched_alloc(tdmd_sched* S) {
   g.list_teams = 2;  // until the first count
   g.polls = sched::kBarrierPolls;
   g.images = images ? 1 : 0;  // batches: decided per box (BoxGeo::images)
+  g.list_lanes = list_lanes(S);
   if (S->multibox) {
     BoxGeo* boxes;
     int32_t* rep;

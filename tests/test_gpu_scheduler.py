@@ -981,3 +981,63 @@ def test_list_forces_by_kind_of_cell(name, prec):
         f = sched.download()[2]
         assert force_rel_err(f, ref) < (1e-9 if prec == "fp64" else 1e-5)
     sched.close()
+
+
+ONE_LANE = ["narrow cells", "full rows", "open axes", "sparse", "far out"]
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+@pytest.mark.parametrize("name", ONE_LANE)
+def test_list_forces_under_the_displacement_policy(name, prec):
+    # Forces against all pairs in FP64 (as above) where rebuilds have a lane per
+    # atom, with a step's displacement beyond half the skin so that each step
+    # rebuilds.
+    pos, L, periodic, _ = _force_case(name)
+    n = len(pos)
+    say("list forces, displacement policy,", name, prec, n)
+    vel = np.random.Generator(np.random.PCG64(31)).normal(size=(n, 3))
+    s = I.System(lo=np.zeros(3), hi=L.copy(), pos=pos, vel=vel, types=np.ones(n, dtype=np.int32),
+                 ids=np.arange(1, n + 1, dtype=np.int32), masses=np.array([1.0, 63.546]),
+                 periodic=periodic)
+    sched = FastPipelineScheduler.for_system(
+        s, WEAK_MORSE, FastPipelineConfig(precision=prec, rebuild_policy="displacement",
+                                          r_skin=1e-5, dt=1e-4))
+    sched.run_until(3)
+    assert sched.stats().rebuilds == 4
+    p, _, f, _, _ = sched.download()
+    ref = _brute_morse(p, L, periodic, *WEAK_MORSE)
+    assert force_rel_err(f, ref) < (1e-9 if prec == "fp64" else 1e-5)
+    sched.close()
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+@pytest.mark.parametrize("kind,edge,periodic", [
+    ("4 a cell", (84.0, 84.0, 210.0), (1, 1, 1)),  # by cells / by one lane
+    ("4 a cell, open", (84.0, 84.0, 210.0), (1, 0, 1)),
+    ("1 a cell", (133.0, 133.0, 336.0), (1, 1, 1)),  # by 32 lanes / by one
+    ("1 a cell, open", (133.0, 133.0, 336.0), (0, 1, 1)),
+    ("film", (210.0, 210.0, 16.0), (1, 1, 1))])  # FP64: by 32 lanes / by one
+def test_list_searches_give_the_same_rows(kind, edge, periodic, prec):
+    # 18,000 atoms: the fused rebuild and the separate kernels search their lists
+    # in different ways, with and without room in the rows: the same bits.
+    n, L = 18000, np.array(edge)
+    rng = np.random.Generator(np.random.PCG64(37))
+    pos = rng.uniform(0.0, L, size=(n, 3))
+    s = I.System(lo=np.zeros(3), hi=L, pos=pos, vel=rng.normal(size=(n, 3)),
+                 types=np.ones(n, dtype=np.int32), ids=np.arange(1, n + 1, dtype=np.int32),
+                 masses=np.array([1.0, 63.546]), periodic=periodic)
+    say("list searches,", kind, prec)
+    # the longest row, as nothing moves by more than 1e-3 A below
+    probe = FastPipelineScheduler.for_system(s, WEAK_MORSE, FastPipelineConfig(precision=prec))
+    longest = int(round(probe.thermo()["max_nbr"]))
+    probe.close()
+    out = []
+    for cap in (0, -(-(longest + 2) // 8) * 8):
+        for split in (False, True):
+            cfg = FastPipelineConfig(precision=prec, rebuild_every=2, split_rebuild=split,
+                                     max_neighbors=cap, dt=1e-4)
+            sched = FastPipelineScheduler.for_system(s, WEAK_MORSE, cfg)
+            sched.run_until(8)
+            out.append(sched.download())
+            sched.close()
+    assert all(np.array_equal(a, b) for o in out[1:] for a, b in zip(o, out[0]))
