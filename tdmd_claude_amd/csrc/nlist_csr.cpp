@@ -73,7 +73,8 @@ nlist_csr_kernel(const double* __restrict__ pos, int natoms, DevBox box, double 
 }
 
 
-// One workgroup per cell, for cells that hold a few atoms or more.
+// One workgroup per cell (or, for crowded cells among sparse ones, several, each
+// with its share of the cell's atoms), for cells that hold a few atoms or more.
 //
 // The candidates of a cell -- the atoms of its 27 stencil cells, in stencil
 // order (z, y, x outer to inner, then cell order), the order of the rows --
@@ -137,7 +138,8 @@ nlist_csr_cell_kernel(const double* __restrict__ pos, int ncells, DevBox box, do
     const int c = (static_cast<int>(blockIdx.x) & 7) * per + b;
     if (c >= ncells) return;
     const int n_home = cell_counts[c];
-    if (n_home == 0) continue;
+    // (a cell's atoms go to gridDim.y workgroups, kHomeMax at a time)
+    if (n_home <= kHomeMax * static_cast<int>(blockIdx.y)) continue;
     const int home = cell_offsets[c];
     const int iz = c / (ncx * ncy);
     const int iy = (c - iz * ncx * ncy) / ncx;
@@ -195,9 +197,10 @@ nlist_csr_cell_kernel(const double* __restrict__ pos, int ncells, DevBox box, do
         }
         cand[q] = v;
       }
-      for (int h0 = 0; h0 < n_home; h0 += kHomeMax) {
+      const int first = kHomeMax * static_cast<int>(blockIdx.y);
+      for (int h0 = first; h0 < n_home; h0 += kHomeMax * static_cast<int>(gridDim.y)) {
         const int nh = min(kHomeMax, n_home - h0);
-        if (h0 > 0) __syncthreads();  // the previous atoms are done with
+        if (h0 > first) __syncthreads();  // the previous atoms are done with
         if (static_cast<int>(threadIdx.x) < nh) {
           const int i = cell_atoms[home + h0 + static_cast<int>(threadIdx.x)];
           const double* p = pos + 3 * static_cast<int64_t>(i);
@@ -291,14 +294,15 @@ nlist_csr_cell_kernel(const double* __restrict__ pos, int ncells, DevBox box, do
 }
 
 template <bool kFill>
-int launch_cells(int threads, const double* pos, int64_t ncells, const DevBox& box, double r_list,
-                 const int32_t* cc, const int32_t* co, const int32_t* ca, const int32_t n[3],
-                 const int32_t* offsets, int32_t* nbrs, int32_t* counts, int32_t max_nb,
+int launch_cells(int threads, int parts, const double* pos, int64_t ncells, const DevBox& box,
+                 double r_list, const int32_t* cc, const int32_t* co, const int32_t* ca,
+                 const int32_t n[3], const int32_t* offsets, int32_t* nbrs, int32_t* counts, int32_t max_nb,
                  int32_t* overflow, hipStream_t stream) {
   const int grid = static_cast<int>(std::min<int64_t>((ncells + 7) / 8 * 8, 1 << 20));
   auto go = [&](auto kernel) {
-    kernel<<<grid, threads, 0, stream>>>(pos, static_cast<int>(ncells), box, r_list, cc, co, ca,
-                                         n[0], n[1], n[2], offsets, nbrs, counts, max_nb, overflow);
+    kernel<<<dim3(grid, parts), threads, 0, stream>>>(
+        pos, static_cast<int>(ncells), box, r_list, cc, co, ca, n[0], n[1], n[2], offsets, nbrs,
+        counts, max_nb, overflow);
   };
   switch (threads) {
     case 64: go(&nlist_csr_cell_kernel<kFill, 64>); break;
@@ -335,15 +339,23 @@ int nlist_csr(bool fill, const double* d_pos, int64_t natoms, const tdmd_box& bo
   //   65,536    64,000 (1)     74 / 83    37 / 43  125 / 136
   //   65,536   125,000 (0.5)   56 / 60    56 / 62  196 / 210
   //   1M          1M (1)      433 / 468  483 / 557
+  // Where a cell's workgroup is a wavefront, up to four share a cell of more than
+  // 64 atoms, for droplets with long cutoffs; the idle ones of other cells cost
+  // ~1 us per 4,000 cells each. Parts 1, 2, 4 against a lane per atom:
+  //   10,976 atoms, r_list 20 A, 8,000 cells    11151 / 17784  5673 / 9047
+  //                                  3034 / 4837; lane 8936 / 11347
+  //   32,768 atoms in as many cells  21 / 24  26 / 30  41 / 47; lane 75 / 84
+  //   64,000 atoms in as many cells  36 / 41  48 / 55  78 / 88; lane 75 / 83
   const int64_t ncells = static_cast<int64_t>(n[0]) * n[1] * n[2];
   if (natoms >= 2 * ncells || (ncells <= 65536 && 2 * natoms >= ncells)) {
     const bool dense = natoms >= 8 * ncells;
     const int threads = dense ? (ncells >= 2048 ? 256 : ncells >= 216 ? 512 : 1024)
                               : (ncells >= 1024 ? 64 : 256);
-    return fill ? launch_cells<true>(threads, d_pos, ncells, db, r_list, cc, co, ca, n, offsets,
-                                     nbrs, counts, max_nb, overflow, stream)
-                : launch_cells<false>(threads, d_pos, ncells, db, r_list, cc, co, ca, n, nullptr,
-                                      nullptr, counts, 0, nullptr, stream);
+    const int parts = threads > 64 ? 1 : ncells <= 32768 ? 4 : ncells <= 65536 ? 2 : 1;
+    return fill ? launch_cells<true>(threads, parts, d_pos, ncells, db, r_list, cc, co, ca, n,
+                                     offsets, nbrs, counts, max_nb, overflow, stream)
+                : launch_cells<false>(threads, parts, d_pos, ncells, db, r_list, cc, co, ca, n,
+                                      nullptr, nullptr, counts, 0, nullptr, stream);
   }
   if (fill) {
     nlist_csr_kernel<true><<<grid_for(natoms), kBlock, 0, stream>>>(

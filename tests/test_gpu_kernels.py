@@ -471,3 +471,21 @@ def test_invalid_arguments_return_status():
     st = capi.lib().tdmd_morse_force(7, None, None, None, None, None, 5, C.byref(box),
                                      C.byref(capi.MorseParams.make(*MORSE_CU)), None, None, None)
     assert st == 1
+
+
+def test_list_of_a_droplet_with_a_long_cutoff():
+    # 2,048 atoms in a box of 1,331 cells: up to ~120 atoms in few cells, whose
+    # workgroups are single wavefronts, several to a cell. Rows against the oracle.
+    s = I.fcc_lattice(8, 8, 8, 3.615)
+    I.jitter_uniform(s, 0.1, 5)
+    lo, hi = s.lo, s.lo + 11 * 11.0 + 0.5
+    pos = s.pos + 40.0
+    say("csr droplet", len(pos))
+    g = csr_build(pos, lo, hi, 10.0, 1.0)
+    assert g["cells"]["ncells"] == 1331 and g["cells"]["cc"].download().max() > 64
+    rcnt, roff, rnb = O.HalfList(pos, lo, hi, 10.0, 1.0).full()
+    cnt, off, nb = g["counts"].download(), g["offsets"].download(), g["nbrs"].download()
+    assert g["overflow"] == 0
+    assert np.array_equal(cnt, rcnt) and np.array_equal(g["counts_pass1"].download(), rcnt)
+    for i in range(len(pos)):
+        assert np.array_equal(np.sort(nb[off[i]:off[i] + cnt[i]]), rnb[roff[i]:roff[i] + rcnt[i]])
