@@ -135,7 +135,9 @@ struct tdmd_sched {
   double* d_scalars = nullptr;
   mutable double* h_stage = nullptr;  // pinned, from the first download on
   mutable hipEvent_t ev_stage[4] = {};
-  mutable std::mutex download_mu;  // the staging buffer's and the scratch block's
+  // the staging buffer's and the scratch block's: a download gathers into the
+  // latter, which a rebuild by separate kernels uses from one to the next
+  mutable std::mutex scratch_mu;
   std::vector<int32_t> h_types, h_ids;
   std::vector<double> h_masses;
   bool uploaded = false, initial_forces = false;

@@ -553,6 +553,7 @@ int list_teams(double m) {
 
 // First neighbour build: sort, count exactly, size the list, fill.
 int first_build(tdmd_sched* S) {
+  std::lock_guard<std::mutex> lock(S->scratch_mu);
   hipStream_t s = S->stream;
   k_set_flag<<<1, 64, 0, s>>>(S->a.flags);
   TDMD_LAUNCH_CHECK();
@@ -616,6 +617,7 @@ int launch_ops(tdmd_sched* S, const std::string& ops, hipStream_t s) {
 // Enqueue a sequence of ops, as one cached graph when enabled.
 int run_ops(tdmd_sched* S, const std::string& ops) {
   if (ops.empty()) return TDMD_OK;
+  std::lock_guard<std::mutex> lock(S->scratch_mu);
   hipStream_t s = S->stream;
   if (!S->cfg.use_graph) return launch_ops(S, ops, s);
   // a graph holds the record buffers of the state it was captured in (and
@@ -1005,9 +1007,9 @@ int tdmd_sched_download(const tdmd_sched* S, double* pos, double* vel, double* f
   while (first < 3 && !dst[first]) ++first;
   while (last > first && !dst[last - 1]) --last;
   if (first < last) {
-    // the scratch block and the staging buffer are this scheduler's: one
-    // download at a time
-    std::lock_guard<std::mutex> lock(S->download_mu);
+    // one download at a time, and none between the kernels of a rebuild that
+    // another thread is enqueuing
+    std::lock_guard<std::mutex> lock(S->scratch_mu);
     const StreamDevice device(S->stream);
     double* const out = S->t.px;
     const int nb = (S->natoms + 255) / 256;

@@ -8,6 +8,7 @@ of the RMS force.
 """
 import ctypes as C
 import functools
+import threading
 
 import numpy as np
 import pytest
@@ -1041,3 +1042,38 @@ def test_list_searches_give_the_same_rows(kind, edge, periodic, prec):
             out.append(sched.download())
             sched.close()
     assert all(np.array_equal(a, b) for o in out[1:] for a, b in zip(o, out[0]))
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+def test_downloads_beside_a_run_leave_it_alone(prec):
+    # A thread that downloads again and again while another runs steps with a
+    # rebuild each, by separate kernels without graphs: the run ends as one that
+    # nobody watched, bit for bit, and each download holds every atom of some step.
+    s = fcc(10)
+    cfg = FastPipelineConfig(precision=prec, rebuild_every=1, split_rebuild=True, use_graph=False)
+    say("downloads beside a run", prec)
+    quiet = FastPipelineScheduler.for_system(s, MORSE_CU, cfg)
+    for step in range(10, 301, 10):
+        quiet.run_until(step)
+    sched = FastPipelineScheduler.for_system(s, MORSE_CU, cfg)
+    sched.run_until(0)
+    seen, done = [], threading.Event()
+
+    def watch():
+        while not done.is_set():
+            seen.append(sched.download()[0])
+
+    t = threading.Thread(target=watch)
+    t.start()
+    for step in range(10, 301, 10):
+        sched.run_until(step)
+    done.set()
+    t.join()
+    assert len(seen) > 1
+    for p in seen[:: max(1, len(seen) // 20)]:
+        d = p - s.pos
+        d -= np.round(d / s.hi[0]) * s.hi[0]
+        assert np.abs(d).max() < 2.0  # 0.3 ps at 300 K
+    assert all(np.array_equal(a, b) for a, b in zip(sched.download(), quiet.download()))
+    sched.close()
+    quiet.close()
