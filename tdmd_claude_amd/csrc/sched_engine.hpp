@@ -11,7 +11,6 @@
 #include <mutex>
 #include <numeric>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 

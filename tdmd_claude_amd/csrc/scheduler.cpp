@@ -149,7 +149,7 @@ int staged_download(const tdmd_sched* S, double* const dst[3], size_t from, size
     };
     try {
       th[t] = std::thread(work);
-    } catch (const std::system_error&) {  // no thread to be had
+    } catch (...) {  // no thread, or no memory for one, to be had
       rc[t] = copy(t);
     }
   }
