@@ -473,12 +473,14 @@ int tdmd_fm_morse(tdmd_fm* fm, const double params[3], double rc,
 /* Single-element EAM from knot values on the device, d_values =
  * [F(nrho) | rho(nr) | phi(nr)] (phi = (r phi)/r, EamAlloy's form).
  * Device outputs, any may be NULL: d_loss[1], d_grad (same layout as
- * d_values), d_forces[3 ntot]. Synchronises `stream` before returning. */
+ * d_values), d_forces[3 ntot]. Synchronises `stream` before returning.
+ * Allocates on the first call, and the half list on the first gradient that
+ * goes over unordered pairs (FP64, and mixed tables beyond the LDS). */
 int tdmd_fm_eam(tdmd_fm* fm, int32_t nrho, double drho, int32_t nr,
                 double dr, double cutoff, const double* d_values,
                 double* d_loss, double* d_grad, double* d_forces,
                 void* stream);
-/* Coefficient gradient of the last tdmd_fm_eam call (host copy):
+/* Coefficient gradient of the last tdmd_fm_eam call with d_grad (host copy):
  * F{a,b,c,d}[nrho-1], rho{a,b,c,d}[nr-1], phi{a,b,c,d}[nr-1]. */
 int tdmd_fm_eam_coef_grad(const tdmd_fm* fm, double* gcoef);
 

@@ -1,14 +1,13 @@
 """The step path at the benchmark shapes, against the FP64 oracle.
 
-* 1,048,576-atom Johnson Cu EAM (64^3 FCC cells, 300 K, seed 7): above
-  131,072 atoms the fused rebuild searches each atom's cells with one lane,
-  its grid is the whole chip (two 1024-thread workgroups per CU), and the
-  LDS passes serve four 1024-atom blocks per persistent workgroup with the
-  next block's halo gathered while the current one is evaluated. Forced
-  rebuilds (fixed interval) make every run here go through the fused
-  rebuild at least twice.
+* 1,048,576-atom Johnson Cu EAM (64^3 FCC cells, 300 K, seed 7): the
+  fused rebuild's grid is the whole chip (one 1024-thread workgroup per CU),
+  each working through many cells, and the LDS passes serve four 1024-atom
+  blocks per persistent workgroup with the next block's halo gathered while
+  the current one is evaluated. Forced rebuilds (fixed interval) make every
+  run here go through the fused rebuild at least twice.
 * 143,748-atom Morse Cu (33^3 cells): above the sizes where the Morse rows
-  are split over 8 lanes and the list search takes 32 lanes per atom.
+  are split over 4 or 8 lanes.
 * 64 Ni/Co/Cr replicas (571,384 atoms, 5000-point three-element tables):
   the batched multi-element passes.
 
