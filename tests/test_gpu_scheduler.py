@@ -1015,15 +1015,19 @@ def test_list_forces_under_the_displacement_policy(name, prec):
 @pytest.mark.parametrize("kind,edge,periodic", [
     ("4 a cell", (84.0, 84.0, 210.0), (1, 1, 1)),  # by cells / by one lane
     ("4 a cell, open", (84.0, 84.0, 210.0), (1, 0, 1)),
+    ("4 a cell, crowded", (84.0, 84.0, 210.0), (1, 1, 1)),
     ("1 a cell", (133.0, 133.0, 336.0), (1, 1, 1)),  # by 32 lanes / by one
     ("1 a cell, open", (133.0, 133.0, 336.0), (0, 1, 1)),
     ("film", (210.0, 210.0, 16.0), (1, 1, 1))])  # FP64: by 32 lanes / by one
 def test_list_searches_give_the_same_rows(kind, edge, periodic, prec):
     # 18,000 atoms: the fused rebuild and the separate kernels search their lists
-    # in different ways, with and without room in the rows: the same bits.
+    # and order their cells in different ways (crowded: also 12 cells of ~130),
+    # with and without room in the rows: the same bits.
     n, L = 18000, np.array(edge)
     rng = np.random.Generator(np.random.PCG64(37))
     pos = rng.uniform(0.0, L, size=(n, 3))
+    if "crowded" in kind:
+        pos[rng.permutation(n)[:1500]] = rng.uniform(0.0, (14.0, 14.0, 21.0), size=(1500, 3))
     s = I.System(lo=np.zeros(3), hi=L, pos=pos, vel=rng.normal(size=(n, 3)),
                  types=np.ones(n, dtype=np.int32), ids=np.arange(1, n + 1, dtype=np.int32),
                  masses=np.array([1.0, 63.546]), periodic=periodic)
